@@ -1,0 +1,48 @@
+/*
+ * tfgfa_gpt2.h - C ABI of the GPT-2 block kernels around the attention (MI355X, gfx950).
+ *
+ * The reference's block runs its norms, GELU and residual adds as chains of PyTorch operators
+ * (src/py/model_inference.py:96-164).  These entry points compute the same functions in one pass
+ * each.  Values are float32 with float32 arithmetic; a result marked bf16 is rounded once, to
+ * nearest even.
+ *
+ * Conventions as in tfgfa.h: device pointers, the caller owns every buffer, launches are
+ * asynchronous on `hip_stream`, arguments are checked before any HIP call; 0 on success, > 0
+ * an invalid argument (TFGFA_ERR_*), < 0 a negated hipError_t.  Tensors are contiguous and 16-byte
+ * aligned.  Row counts of 0 launch nothing.
+ */
+#ifndef TFGFA_GPT2_H
+#define TFGFA_GPT2_H
+
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* Largest row width of the norm: a row lives in one wave's registers. */
+#define TFGPT2_MAX_NORM_DIM 2048
+
+/*
+ * LayerNorm over rows of width d (a multiple of 4, at most TFGPT2_MAX_NORM_DIM), biased variance:
+ *   s = x            (delta == NULL)
+ *   s = x + delta    (delta: (rows, d) bf16; s is also written to sum, (rows, d) float32)
+ *   y = (s - mean) / sqrt(var + eps) * scale + shift
+ * y is (rows, d), float32 (y_bf16 = 0) or bf16 (y_bf16 = 1).  sum may be x itself.
+ * src/py/model_inference.py:96-107 (LayerNorm), :157-160 (the residual add before norm2).
+ */
+int tfgpt2_layernorm(const float* x, const void* delta, float* sum, const float* scale,
+                     const float* shift, void* y, int y_bf16, int64_t rows, int d, float eps,
+                     void* hip_stream);
+
+/*
+ * GELU, tanh form, elementwise over n float32 values:
+ *   y = 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))      (model_inference.py:109-117)
+ */
+int tfgpt2_gelu(const float* x, float* y, int64_t n, void* hip_stream);
+
+#ifdef __cplusplus
+}
+#endif
+
+#endif /* TFGFA_GPT2_H */

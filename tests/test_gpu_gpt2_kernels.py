@@ -1,0 +1,143 @@
+"""The GPT-2 block kernels (include/tfgfa_gpt2.h) against float64 references of the same
+functions, and the modules that use them against their torch operators (GPU box only, except the
+argument checks).
+
+Tolerances.  Values are float32 with float32 sums: a result carries a few roundings of 2^-24
+relative to the terms it is made of, so the relative 2-norm error is held to 1e-6 (8 roundings of
+2^-23).  bf16 results are rounded once more, 2^-9 at most: 2-norm error 2^-9.
+"""
+import math
+
+import pytest
+import torch
+
+import custom_flash_attn  # noqa: F401
+import model_inference as mi
+from custom_flash_attn import _C
+
+DEV = "cuda:0"
+F32, BF16 = 1e-6, 2.0 ** -9
+
+
+def _rel(x, ref):
+    x, ref = x.double(), ref.double()
+    return ((x - ref).norm() / ref.norm()).item()
+
+
+def _randn(g, *shape):
+    return torch.randn(shape, device=DEV, generator=g)
+
+
+def _norm64(x, scale, shift, eps=1e-5):
+    x = x.double()
+    y = (x - x.mean(-1, keepdim=True)) / torch.sqrt(x.var(-1, keepdim=True, unbiased=False) + eps)
+    return y * scale.double() + shift.double()
+
+
+def _gelu64(x):
+    x = x.double()
+    return 0.5 * x * (1 + torch.tanh(math.sqrt(2 / math.pi) * (x + 0.044715 * x ** 3)))
+
+
+def test_kernel_arguments_are_checked_before_any_hip_call():
+    P = 0x10000
+    with pytest.raises(RuntimeError, match="negative batch|shape|size"):
+        _C.gpt2_layernorm(P, 0, 0, P, P, P, False, 1, 6, 1e-5, 0)          # width not a multiple of 4
+    with pytest.raises(RuntimeError):
+        _C.gpt2_layernorm(P, 0, 0, P, P, P, False, 1, 2052, 1e-5, 0)       # too wide
+    with pytest.raises(RuntimeError, match="null"):
+        _C.gpt2_layernorm(P, P, 0, P, P, P, False, 1, 64, 1e-5, 0)         # delta without sum
+    with pytest.raises(RuntimeError, match="misaligned"):
+        _C.gpt2_layernorm(P + 4, 0, 0, P, P, P, False, 1, 64, 1e-5, 0)
+    _C.gpt2_layernorm(0, 0, 0, 0, 0, 0, False, 0, 64, 1e-5, 0)             # no rows: nothing to do
+    with pytest.raises(RuntimeError, match="misaligned"):
+        _C.gpt2_gelu(P + 8, P, 4, 0)
+    _C.gpt2_gelu(0, 0, 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,d", [(1, 4), (3, 252), (4, 256), (5, 260), (7, 768), (2, 1024), (3, 1028),
+                                    (9, 1600), (1, 2048)])
+def test_layernorm_matches_float64(rows, d):
+    """Widths at the edges of a lane's four values, of a wave's 256 and of the two register sizes;
+    rows that fill and do not fill a workgroup; an offset mean, so the variance must be centred."""
+    from custom_flash_attn import gpt2
+
+    g = torch.Generator(device=DEV).manual_seed(rows * 10007 + d)
+    x, scale, shift = _randn(g, rows, d) * 3 + 100, 1 + _randn(g, d), _randn(g, d)
+    delta = (_randn(g, rows, d) * 2).to(torch.bfloat16)
+    # The centred values lose log2(100 / 3) bits of x's 24.
+    y = gpt2.layernorm(x, scale, shift, 1e-5)
+    assert _rel(y, _norm64(x, scale, shift)) <= 40 * F32
+    s, y = gpt2.layernorm(x, scale, shift, 1e-5, delta=delta)
+    assert torch.equal(s, x + delta)
+    assert _rel(y, _norm64(s, scale, shift)) <= 40 * F32
+    y = gpt2.layernorm(x, scale, shift, 1e-5, torch.bfloat16)
+    assert y.dtype == torch.bfloat16 and _rel(y, _norm64(x, scale, shift)) <= BF16
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1024, 1025, 40000])
+def test_gelu_matches_float64(n):
+    from custom_flash_attn import gpt2
+
+    x = _randn(torch.Generator(device=DEV).manual_seed(n), n) * 3
+    assert _rel(gpt2.gelu(x), _gelu64(x)) <= F32
+    special = torch.tensor([math.inf, -math.inf, math.nan, 0.0, -0.0, 3e38, -3e38, 1e-40, 50.0, -50.0], device=DEV)
+    want = 0.5 * special * (1 + torch.tanh(math.sqrt(2.0 / math.pi) * (special + 0.044715 * torch.pow(special, 3))))
+    assert torch.equal(gpt2.gelu(special).nan_to_num(nan=7.0), want.nan_to_num(nan=7.0))
+
+
+def _block(emb, heads, **kw):
+    cfg = dict(mi.GPT_CONFIG_124M)
+    cfg.update({"emb_dim": emb, "n_heads": heads, "context_length": 128, "drop_rate": 0.0, "qkv_bias": True,
+                "impl_type": "hip", **kw})
+    blk = mi.TransformerBlock(cfg).to(DEV).eval()
+    g = torch.Generator(device=DEV).manual_seed(emb)
+    with torch.no_grad():
+        for p in blk.parameters():
+            p.add_(_randn(g, *p.shape) * 0.05)
+    return blk, g
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("emb,heads,bias", [(256, 4, True), (512, 8, False)])
+def test_block_matches_its_torch_operators(emb, heads, bias):
+    """The fused block against the same block on its torch operators, which a gradient-requiring
+    input selects.  The attention's bf16 results are the difference: 2^-8 of its share of x."""
+    blk, g = _block(emb, heads, qkv_bias=bias)
+    x = _randn(g, 2, 37, emb)
+    with torch.no_grad():
+        fused = blk(x)
+    assert blk._fused(x) is False  # parameters need a gradient outside no_grad
+    hook = blk.norm1.register_forward_hook(lambda m, i, o: None)
+    seen = []
+    hook2 = blk.norm2.register_forward_hook(lambda m, i, o: seen.append(o.shape))
+    with torch.no_grad():
+        assert not blk._fused(x)
+        hooked = blk(x)
+    hook.remove()
+    hook2.remove()
+    assert seen == [x.shape] and _rel(hooked, fused) <= 1e-3
+
+
+@pytest.mark.gpu
+def test_modules_keep_gradients_and_transforms():
+    """Where a gradient, a function transform, forward-mode or another type is in play the modules
+    run their torch operators."""
+    norm, act = mi.LayerNorm({"emb_dim": 64}).to(DEV), mi.GELU()
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = _randn(g, 5, 64)
+    y = act(norm(x))
+    y.sum().backward()
+    assert norm.scale.grad is not None and torch.isfinite(norm.scale.grad).all()
+    with torch.no_grad():
+        ref = act(norm(x))
+        torch.testing.assert_close(torch.func.vmap(lambda r: act(norm(r)))(x), ref, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(act(norm(x.double())), ref.double(), rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(act(norm(x.t().contiguous().t())), ref, rtol=1e-5, atol=1e-5)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+            out = act(dual)
+            assert torch.autograd.forward_ad.unpack_dual(out).tangent is not None
+    assert norm(torch.empty(0, 64, device=DEV)).shape == (0, 64)

@@ -15,6 +15,7 @@
 #include <string>
 
 #include "tfgfa.h"
+#include "tfgfa_gpt2.h"
 
 namespace py = pybind11;
 
@@ -123,6 +124,37 @@ void decode_general(std::uintptr_t q, const Strides3& qs, std::uintptr_t kc, con
   }
 }
 
+void check(int st, const char* what) {
+  if (st != TFGFA_OK) {
+    throw std::runtime_error(std::string(what) + " failed (status " + std::to_string(st) +
+                             "): " + tfgfa_strerror(st));
+  }
+}
+
+void gpt2_layernorm(std::uintptr_t x, std::uintptr_t delta, std::uintptr_t sum,
+                    std::uintptr_t scale, std::uintptr_t shift, std::uintptr_t y, bool y_bf16,
+                    std::int64_t rows, int d, float eps, std::uintptr_t stream) {
+  int st;
+  {
+    py::gil_scoped_release nogil;
+    st = tfgpt2_layernorm(reinterpret_cast<const float*>(x), reinterpret_cast<const void*>(delta),
+                          reinterpret_cast<float*>(sum), reinterpret_cast<const float*>(scale),
+                          reinterpret_cast<const float*>(shift), reinterpret_cast<void*>(y),
+                          y_bf16 ? 1 : 0, rows, d, eps, reinterpret_cast<void*>(stream));
+  }
+  check(st, "tfgpt2_layernorm");
+}
+
+void gpt2_gelu(std::uintptr_t x, std::uintptr_t y, std::int64_t n, std::uintptr_t stream) {
+  int st;
+  {
+    py::gil_scoped_release nogil;
+    st = tfgpt2_gelu(reinterpret_cast<const float*>(x), reinterpret_cast<float*>(y), n,
+                     reinterpret_cast<void*>(stream));
+  }
+  check(st, "tfgpt2_gelu");
+}
+
 py::dict device_info() {
   int cu = 0, mhz = 0;
   char arch[128] = {0};
@@ -188,6 +220,13 @@ PYBIND11_MODULE(_C, m) {
   m.def("decode_workspace_size", [](int B, int H, int N_max, int D) {
     return tfgfa_decode_workspace_size(B, H, N_max, D);
   });
+  m.def("gpt2_layernorm", &gpt2_layernorm, "LayerNorm, with an optional residual add before it",
+        py::arg("x"), py::arg("delta"), py::arg("sum"), py::arg("scale"), py::arg("shift"),
+        py::arg("y"), py::arg("y_bf16"), py::arg("rows"), py::arg("d"), py::arg("eps"),
+        py::arg("stream"));
+  m.def("gpt2_gelu", &gpt2_gelu, "GELU (tanh form), elementwise", py::arg("x"), py::arg("y"),
+        py::arg("n"), py::arg("stream"));
+  m.attr("GPT2_MAX_NORM_DIM") = TFGPT2_MAX_NORM_DIM;
   m.def("device_info", &device_info, "CU count, shader clock (MHz) and arch of the current device");
   m.def("strerror", [](int st) { return std::string(tfgfa_strerror(st)); });
   m.def("abi_version", []() { return tfgfa_abi_version(); });

@@ -38,6 +38,40 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 # --------------------------------------------------------------------------------------
+# The block kernels (custom_flash_attn.gpt2) in place of chains of torch operators.
+
+_gpt2_module = None
+
+
+def _gpt2():
+    """custom_flash_attn.gpt2, or None where the native extension is not built (the modules then
+    run their torch operators; the attention branches that need the extension raise)."""
+    global _gpt2_module
+    if _gpt2_module is None:
+        try:
+            from custom_flash_attn import gpt2 as _gpt2_module
+        except ImportError:
+            _gpt2_module = False
+    return _gpt2_module or None
+
+
+def _plain(module, cls) -> bool:
+    """``module`` is a ``cls`` as this file or torch defines it, with no hook that a call of it
+    would run: a caller may then take its parameters and leave the call out."""
+    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
+            and "forward" not in module.__dict__)
+
+
+def _no_global_hooks() -> bool:
+    m = torch.nn.modules.module
+    return not (m._global_forward_hooks or m._global_forward_pre_hooks)
+
+
+def _inactive(dropout) -> bool:
+    return _plain(dropout, nn.Dropout) and (not dropout.training or dropout.p == 0)
+
+
+# --------------------------------------------------------------------------------------
 # Attention implementations: (queries, keys, values, mask_bool, dropout) -> (B, N, H, d).
 # queries/keys/values arrive as (B, H, N, d) views (model_inference.py:64-66).
 
@@ -115,6 +149,10 @@ class MultiHeadAttention(nn.Module):
         self.register_buffer(
             "mask", torch.triu(torch.ones(context_length, context_length), diagonal=1)
         )
+
+    def _plain_linears(self) -> bool:
+        return (_plain(self, MultiHeadAttention)
+                and all(_plain(m, nn.Linear) for m in (self.W_query, self.W_key, self.W_value, self.out_proj)))
 
     def forward(self, x, kv_cache=None, layer: int = 0):
         if kv_cache is not None:
@@ -252,7 +290,15 @@ class LayerNorm(nn.Module):
         self.scale = nn.Parameter(torch.ones(config["emb_dim"]))
         self.shift = nn.Parameter(torch.zeros(config["emb_dim"]))
 
+    def _native(self, x) -> bool:
+        d = x.shape[-1] if x.dim() else 0
+        return (d % 4 == 0 and 4 <= d <= _gpt2().MAX_NORM_DIM and self.scale.shape == (d,)
+                and self.shift.shape == (d,))
+
     def forward(self, x):
+        g = _gpt2() if x.is_cuda else None
+        if g is not None and g.eager() and g.takes(x, self.scale, self.shift) and self._native(x):
+            return g.layernorm(x, self.scale, self.shift, self.eps)
         mean = torch.mean(x, dim=-1, keepdim=True)
         variance = torch.var(x, dim=-1, keepdim=True, unbiased=False)
         norm_x = (x - mean) / torch.sqrt(variance + self.eps)
@@ -263,6 +309,9 @@ class GELU(nn.Module):
     """tanh-approximation GELU (model_inference.py:109-117)."""
 
     def forward(self, x):
+        g = _gpt2() if x.is_cuda else None
+        if g is not None and g.eager() and g.takes(x):
+            return g.gelu(x)
         return 0.5 * x * (1 + torch.tanh(math.sqrt(2.0 / math.pi) * (x + 0.044715 * torch.pow(x, 3))))
 
 
@@ -296,7 +345,39 @@ class TransformerBlock(nn.Module):
         self.norm2 = LayerNorm(cfg)
         self.drop_shortcut = nn.Dropout(cfg["drop_rate"])
 
+    def _fused(self, x) -> bool:
+        """Whether the block may run as fused kernels: float32 GPU tensors, nothing that needs a
+        gradient, a hook or an active dropout, no autocast around the block (the norms and the MLP
+        are then float32, only the attention is under bf16 autocast)."""
+        g = _gpt2() if x.is_cuda else None
+        if g is None or not g.eager() or torch.is_autocast_enabled("cuda") or not _no_global_hooks():
+            return False
+        att, norm1, norm2 = self.att, self.norm1, self.norm2
+        if not (isinstance(att, MultiHeadAttention) and _plain(norm1, LayerNorm)
+                and _plain(norm2, LayerNorm) and _inactive(self.drop_shortcut)):
+            return False
+        return (x.dim() == 3 and g.takes(x, norm1.scale, norm1.shift, norm2.scale, norm2.shift)
+                and norm1._native(x) and norm2._native(x))
+
+    def _forward_fused(self, x, kv_cache, layer):
+        """The block with each norm one kernel: norm1 writes the bf16 that autocast would round its
+        result to (once, not for each projection), the residual add runs inside norm2's kernel."""
+        g = _gpt2()
+        norm1, norm2 = self.norm1, self.norm2
+        dtype = torch.bfloat16 if self.att._plain_linears() else torch.float32
+        h = g.layernorm(x, norm1.scale, norm1.shift, norm1.eps, dtype)
+        with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+            y = self.att(h, kv_cache, layer)
+        if g.takes(y, dtypes=(torch.bfloat16,)) and y.shape == x.shape:
+            x, h = g.layernorm(x, norm2.scale, norm2.shift, norm2.eps, delta=y)
+        else:
+            x = y + x
+            h = norm2(x)
+        return self.ff(h) + x
+
     def forward(self, x, kv_cache=None, layer: int = 0):
+        if self._fused(x):
+            return self._forward_fused(x, kv_cache, layer)
         shortcut = x
         x = self.norm1(x)
         # model_inference.py:153 - autocast only has an effect for CUDA(HIP) tensors, so it
