@@ -1,10 +1,10 @@
 /*
  * tfgfa_gpt2.h - C ABI of the GPT-2 block kernels around the attention (MI355X, gfx950).
  *
- * The reference's block runs its norms, GELU and residual adds as chains of PyTorch operators
- * (src/py/model_inference.py:96-164).  These entry points compute the same functions in one pass
- * each.  Values are float32 with float32 arithmetic; a result marked bf16 is rounded once, to
- * nearest even.
+ * The reference's block runs its norms, GELU, residual adds and the one-token projections as
+ * separate PyTorch operators (src/py/model_inference.py:39-164).  These entry points compute
+ * the same functions in one pass each.  Values are float32 with float32 arithmetic; a result
+ * marked bf16 is rounded once, to nearest even.
  *
  * Conventions as in tfgfa.h: device pointers, the caller owns every buffer, launches are
  * asynchronous on `hip_stream`, arguments are checked before any HIP call; 0 on success, > 0
@@ -20,8 +20,10 @@
 extern "C" {
 #endif
 
-/* Largest row width of the norm: a row lives in one wave's registers. */
+/* Largest row width of the norm (a row lives in one wave's registers) and the most rows of the
+ * few-row projections. */
 #define TFGPT2_MAX_NORM_DIM 2048
+#define TFGPT2_MAX_ROWS     8
 
 /*
  * LayerNorm over rows of width d (a multiple of 4, at most TFGPT2_MAX_NORM_DIM), biased variance:
@@ -40,6 +42,25 @@ int tfgpt2_layernorm(const float* x, const void* delta, float* sum, const float*
  *   y = 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))      (model_inference.py:109-117)
  */
 int tfgpt2_gelu(const float* x, float* y, int64_t n, void* hip_stream);
+
+/*
+ * A linear layer on few rows (1 <= M <= TFGPT2_MAX_ROWS), the projections of one decode step:
+ *   y[m, n] = f( sum_k xhat[m, k] w[n, k] + bias[n] ) + residual[m, n]
+ * with up to three weight matrices sharing x (query, key and value): parts in 1..3, part p uses
+ * w[p] (N, K) float32, bias[p] (N) float32 or NULL, y[p] (M, N).
+ *   x        (M, K), float32 (x_bf16 = 0) or bf16 (x_bf16 = 1)
+ *   ln_scale, ln_shift   both NULL, or (K): xhat = LayerNorm(x) with eps, as above (x float32,
+ *                        K <= TFGPT2_MAX_NORM_DIM, M * (K + 4) <= 15360); otherwise xhat = x
+ *   gelu     1: f is the GELU above (with a norm, float32 y), 0: identity
+ *   residual (M, N) float32 or NULL (parts == 1); y[0] may be residual itself
+ *   y_bf16   element type of every y: float32 (0), or bf16 (1) with a norm and no GELU
+ * K a multiple of 4.  Products and sums are float32; the result does not depend on the device or
+ * the launch.
+ */
+int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_scale, const float* ln_shift,
+                       float eps, int parts, const float* const* w, const float* const* bias,
+                       int gelu, const float* residual, void* const* y, int y_bf16, int M, int N,
+                       int K, void* hip_stream);
 
 #ifdef __cplusplus
 }

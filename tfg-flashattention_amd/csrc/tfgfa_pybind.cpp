@@ -13,6 +13,8 @@
 #include <cstdint>
 #include <stdexcept>
 #include <string>
+#include <tuple>
+#include <vector>
 
 #include "tfgfa.h"
 #include "tfgfa_gpt2.h"
@@ -155,6 +157,33 @@ void gpt2_gelu(std::uintptr_t x, std::uintptr_t y, std::int64_t n, std::uintptr_
   check(st, "tfgpt2_gelu");
 }
 
+// parts: (weight, bias or 0, output) of each weight matrix.
+void gpt2_linear_rows(
+    std::uintptr_t x, bool x_bf16, std::uintptr_t ln_scale, std::uintptr_t ln_shift, float eps,
+    const std::vector<std::tuple<std::uintptr_t, std::uintptr_t, std::uintptr_t>>& parts,
+    bool gelu, std::uintptr_t residual, bool y_bf16, int M, int N, int K, std::uintptr_t stream) {
+  constexpr std::size_t kMax = 3;
+  if (parts.size() > kMax) check(TFGFA_ERR_BAD_SHAPE, "tfgpt2_linear_rows");
+  const float* w[kMax] = {};
+  const float* bias[kMax] = {};
+  void* y[kMax] = {};
+  for (std::size_t i = 0; i < parts.size(); ++i) {
+    w[i] = reinterpret_cast<const float*>(std::get<0>(parts[i]));
+    bias[i] = reinterpret_cast<const float*>(std::get<1>(parts[i]));
+    y[i] = reinterpret_cast<void*>(std::get<2>(parts[i]));
+  }
+  int st;
+  {
+    py::gil_scoped_release nogil;
+    st = tfgpt2_linear_rows(reinterpret_cast<const void*>(x), x_bf16 ? 1 : 0,
+                            reinterpret_cast<const float*>(ln_scale),
+                            reinterpret_cast<const float*>(ln_shift), eps, (int)parts.size(), w,
+                            bias, gelu ? 1 : 0, reinterpret_cast<const float*>(residual), y,
+                            y_bf16 ? 1 : 0, M, N, K, reinterpret_cast<void*>(stream));
+  }
+  check(st, "tfgpt2_linear_rows");
+}
+
 py::dict device_info() {
   int cu = 0, mhz = 0;
   char arch[128] = {0};
@@ -226,7 +255,13 @@ PYBIND11_MODULE(_C, m) {
         py::arg("stream"));
   m.def("gpt2_gelu", &gpt2_gelu, "GELU (tanh form), elementwise", py::arg("x"), py::arg("y"),
         py::arg("n"), py::arg("stream"));
+  m.def("gpt2_linear_rows", &gpt2_linear_rows,
+        "A linear layer on few rows, with LayerNorm, bias, GELU and residual", py::arg("x"),
+        py::arg("x_bf16"), py::arg("ln_scale"), py::arg("ln_shift"), py::arg("eps"),
+        py::arg("parts"), py::arg("gelu"), py::arg("residual"), py::arg("y_bf16"), py::arg("M"),
+        py::arg("N"), py::arg("K"), py::arg("stream"));
   m.attr("GPT2_MAX_NORM_DIM") = TFGPT2_MAX_NORM_DIM;
+  m.attr("GPT2_MAX_ROWS") = TFGPT2_MAX_ROWS;
   m.def("device_info", &device_info, "CU count, shader clock (MHz) and arch of the current device");
   m.def("strerror", [](int st) { return std::string(tfgfa_strerror(st)); });
   m.def("abi_version", []() { return tfgfa_abi_version(); });

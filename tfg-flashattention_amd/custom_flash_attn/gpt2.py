@@ -11,6 +11,8 @@ from torch.autograd import forward_ad
 from . import _C
 
 MAX_NORM_DIM = _C.GPT2_MAX_NORM_DIM
+MAX_ROWS = _C.GPT2_MAX_ROWS
+_NORM_LDS_FLOATS = 15360  # rows * (width + 4) of a projection with a norm before it
 _TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -68,3 +70,25 @@ def gelu(x):
     with torch.cuda.device(x.device):
         _C.gpt2_gelu(x.data_ptr(), y.data_ptr(), x.numel(), _stream(x.device))
     return y
+
+
+def rows_fit(rows: int, width: int, norm: bool) -> bool:
+    """Whether :func:`linear_rows` takes ``rows`` rows of ``width`` values."""
+    return (1 <= rows <= MAX_ROWS and width % 4 == 0 and width >= 4
+            and (not norm or (width <= MAX_NORM_DIM and rows * (width + 4) <= _NORM_LDS_FLOATS)))
+
+
+def linear_rows(x, parts, dtype, norm=None, gelu=False, residual=None):
+    """y = f(xhat w^T + bias) (+ residual) for each (w, bias) of ``parts`` (at most 3, equal shapes),
+    as a list of tensors of ``dtype``.  ``x``: (..., K) float32 or bf16, few rows (:func:`rows_fit`);
+    ``norm`` = (scale, shift, eps): xhat is x's LayerNorm (x float32); with a norm ``gelu`` makes f the
+    GELU, or ``dtype`` may be bf16."""
+    N, K = parts[0][0].shape
+    ys = [torch.empty(x.shape[:-1] + (N,), dtype=dtype, device=x.device) for _ in parts]
+    scale, shift, eps = norm if norm is not None else (None, None, 0.0)
+    with torch.cuda.device(x.device):
+        _C.gpt2_linear_rows(x.data_ptr(), x.dtype == torch.bfloat16, _ptr(scale), _ptr(shift), eps,
+                            [(w.data_ptr(), _ptr(b), y.data_ptr()) for (w, b), y in zip(parts, ys)],
+                            gelu, _ptr(residual), dtype == torch.bfloat16, x.numel() // K, N, K,
+                            _stream(x.device))
+    return ys

@@ -359,9 +359,46 @@ class TransformerBlock(nn.Module):
         return (x.dim() == 3 and g.takes(x, norm1.scale, norm1.shift, norm2.scale, norm2.shift)
                 and norm1._native(x) and norm2._native(x))
 
+    def _rows_fused(self, x, cache) -> bool:
+        """Whether a decode step may run its projections on the few-row kernel: as for _fused, with
+        plain linears, float32 weights, a bf16 cache that holds tokens and few enough rows."""
+        g, att, ff = _gpt2(), self.att, self.ff
+        if not (cache is not None and cache.length > 0 and x.shape[1] == 1 and att.impl_type in ("hip", "cuda")
+                and att._plain_linears() and _plain(ff, FeedForward) and _plain(ff.layers, nn.Sequential)
+                and len(ff.layers) == 3 and _plain(ff.layers[0], nn.Linear) and _plain(ff.layers[1], GELU)
+                and _plain(ff.layers[2], nn.Linear) and cache.k[0].dtype == torch.bfloat16):
+            return False
+        rows, d = x.shape[0], x.shape[2]
+        qkv, up, down = (att.W_query, att.W_key, att.W_value), ff.layers[0], ff.layers[2]
+        hidden = up.weight.shape[0]
+        return (all(m.weight.shape == (d, d) for m in (*qkv, att.out_proj)) and up.weight.shape == (hidden, d)
+                and down.weight.shape == (d, hidden) and g.rows_fit(rows, d, True) and g.rows_fit(rows, hidden, False)
+                and g.takes(x, *(t for m in (*qkv, att.out_proj, up, down) for t in (m.weight, m.bias))))
+
+    def _forward_rows(self, x, cache, layer):
+        """One decode step as five kernels: norm1 + query/key/value, attention, output projection
+        + residual, norm2 + MLP up + GELU, MLP down + residual.  The weights are read in place, so
+        the bf16 roundings autocast makes of the attention's weights, input and output fall away."""
+        import custom_flash_attn
+
+        g, att, norm1, norm2 = _gpt2(), self.att, self.norm1, self.norm2
+        b, _, d = x.shape
+        H, hd = att.num_heads, att.head_dim
+        q, k, v = (t.view(b, H, hd) for t in g.linear_rows(
+            x, [(m.weight, m.bias) for m in (att.W_query, att.W_key, att.W_value)], torch.bfloat16,
+            norm=(norm1.scale, norm1.shift, norm1.eps)))
+        ctx = custom_flash_attn.decode(q, cache.k[layer], cache.v[layer], cache.seqlens, k, v,
+                                       workspace=cache.workspace)
+        x, = g.linear_rows(ctx.view(b, 1, d), [(att.out_proj.weight, att.out_proj.bias)], torch.float32, residual=x)
+        up, down = self.ff.layers[0], self.ff.layers[2]
+        h, = g.linear_rows(x, [(up.weight, up.bias)], torch.float32, norm=(norm2.scale, norm2.shift, norm2.eps), gelu=True)
+        return g.linear_rows(h, [(down.weight, down.bias)], torch.float32, residual=x)[0]
+
     def _forward_fused(self, x, kv_cache, layer):
         """The block with each norm one kernel: norm1 writes the bf16 that autocast would round its
         result to (once, not for each projection), the residual add runs inside norm2's kernel."""
+        if self._rows_fused(x, kv_cache):
+            return self._forward_rows(x, kv_cache, layer)
         g = _gpt2()
         norm1, norm2 = self.norm1, self.norm2
         dtype = torch.bfloat16 if self.att._plain_linears() else torch.float32
