@@ -20,10 +20,11 @@
 extern "C" {
 #endif
 
-/* Largest row width of the norm (a row lives in one wave's registers) and the most rows of the
- * few-row projections. */
+/* Largest row width of the norm (a row lives in one wave's registers), the most rows of the
+ * few-row projections and the most arrays of one cast. */
 #define TFGPT2_MAX_NORM_DIM 2048
 #define TFGPT2_MAX_ROWS     8
+#define TFGPT2_MAX_CASTS    10
 
 /*
  * LayerNorm over rows of width d (a multiple of 4, at most TFGPT2_MAX_NORM_DIM), biased variance:
@@ -42,6 +43,13 @@ int tfgpt2_layernorm(const float* x, const void* delta, float* sum, const float*
  *   y = 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))      (model_inference.py:109-117)
  */
 int tfgpt2_gelu(const float* x, float* y, int64_t n, void* hip_stream);
+
+/*
+ * float32 -> bf16 copies of up to TFGPT2_MAX_CASTS arrays in one launch: dst[i][0 .. n[i]) = src[i][0 .. n[i]).
+ * n[i] a multiple of 4.
+ */
+int tfgpt2_cast_bf16(int count, const float* const* src, void* const* dst, const int64_t* n,
+                     void* hip_stream);
 
 /*
  * A linear layer on few rows (1 <= M <= TFGPT2_MAX_ROWS), the projections of one decode step:

@@ -53,6 +53,13 @@ def test_kernel_arguments_are_checked_before_any_hip_call():
     with pytest.raises(RuntimeError, match="misaligned"):
         _C.gpt2_gelu(P + 8, P, 4, 0)
     _C.gpt2_gelu(0, 0, 0, 0)
+    with pytest.raises(RuntimeError, match="shape|size"):
+        _C.gpt2_cast_bf16([(P, P, 6)], 0)
+    with pytest.raises(RuntimeError, match="shape|size"):
+        _C.gpt2_cast_bf16([(P, P, 4)] * 11, 0)
+    with pytest.raises(RuntimeError, match="misaligned"):
+        _C.gpt2_cast_bf16([(P, P + 8, 4)], 0)
+    _C.gpt2_cast_bf16([], 0)
     part = (P, 0, P)
     with pytest.raises(RuntimeError, match="shape|size"):
         _C.gpt2_linear_rows(P, False, 0, 0, 0.0, [part], False, 0, False, 9, 4, 64, 0)       # too many rows
@@ -140,6 +147,43 @@ def test_linear_rows_matches_float64(M, N, K):
     xi[0, 0, 0] = math.inf
     got, = gpt2.linear_rows(xi, parts[1:2], torch.float32)
     assert torch.isinf(got[0]).all() and torch.isfinite(got[1:]).all()
+
+
+@pytest.mark.gpu
+def test_cast_rounds_as_torch_does():
+    """Arrays from one value group up to several workgroups, in one launch, bit for bit."""
+    from custom_flash_attn import gpt2
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    src = [_randn(g, n) for n in (4, 1020, 1024, 1028, 40000, 8, 4, 12, 16, 4)]
+    src[1][:6] = torch.tensor([math.inf, -math.inf, math.nan, 3.4e38, 1e-40, -0.0], device=DEV)
+    dst = [torch.full((t.numel() + 8,), 7.0, dtype=torch.bfloat16, device=DEV) for t in src]
+    gpt2.cast_bf16([(s, d[:s.numel()]) for s, d in zip(src, dst)])
+    for s, d in zip(src, dst):
+        want = torch.cat((s.to(torch.bfloat16), torch.full((8,), 7.0, dtype=torch.bfloat16, device=DEV)))
+        assert torch.equal(d.nan_to_num(nan=9.0), want.nan_to_num(nan=9.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("impl", ["hip", "cuda", "triton"])
+@pytest.mark.parametrize("emb,heads,bias,dtype", [(256, 4, True, torch.float32), (320, 5, False, torch.bfloat16)])
+def test_attention_layer_casts_together(impl, emb, heads, bias, dtype):
+    """The layer with its casts in one launch and one GEMM for queries, keys and values against the
+    layer with a hook on one linear (autocast's casts, four GEMMs).  The bf16 inputs are the same; a
+    different summation order flips bf16 roundings, half a unit (2^-8) at most in each result."""
+    torch.manual_seed(emb)
+    m = mi.MultiHeadAttention(emb, emb, 128, 0.0, heads, impl, qkv_bias=bias).to(DEV).eval()
+    x = _randn(torch.Generator(device=DEV).manual_seed(3), 2, 75, emb).to(dtype)
+    with torch.no_grad(), torch.autocast("cuda", torch.bfloat16):
+        assert m._cast_together(x)
+        got = m(x)
+        hook = m.W_key.register_forward_hook(lambda *a: None)
+        assert not m._cast_together(x)
+        want = m(x)
+        hook.remove()
+    assert got.dtype == want.dtype == torch.bfloat16 and _rel(got, want) <= BF16
+    with torch.no_grad(), torch.autocast("cuda", torch.float16):
+        assert not m._cast_together(x)
 
 
 def _block(emb, heads, **kw):

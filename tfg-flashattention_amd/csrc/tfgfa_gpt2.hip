@@ -6,6 +6,7 @@
 //   layernorm_kernel    LayerNorm of a row held in one wave's registers, with the residual add
 //                       before it and the rounding to bf16 after it where the caller has them;
 //   gelu_kernel         the tanh GELU in one pass;
+//   cast_kernel         float32 -> bf16 copies of several weights in one launch;
 //   linear_rows_kernel  a projection of at most 8 rows read straight from the float32 weights,
 //                       with the LayerNorm before it and the bias, GELU and residual after it.
 //
@@ -141,6 +142,28 @@ __global__ __launch_bounds__(kGeluThreads) void gelu_kernel(const float* __restr
     store4(y + i, f32x4{gelu(v[0]), gelu(v[1]), gelu(v[2]), gelu(v[3])});
   } else {
     for (long long j = i; j < n; ++j) y[j] = gelu(x[j]);
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// float32 -> bf16.  Bound: memory.  The arrays are laid end to end in units of 4 values.
+constexpr int kMaxCasts = TFGPT2_MAX_CASTS;
+constexpr int kCastThreads = 256;
+struct Casts {
+  const float* src[kMaxCasts];
+  __bf16* dst[kMaxCasts];
+  long long end[kMaxCasts];  // units of 4 values up to and including array i
+  int count;
+};
+__global__ __launch_bounds__(kCastThreads) void cast_kernel(Casts a) {
+  const long long u = (long long)blockIdx.x * kCastThreads + threadIdx.x;
+  long long begin = 0;
+#pragma unroll
+  for (int i = 0; i < kMaxCasts; ++i) {
+    if (i < a.count) {
+      if (u >= begin && u < a.end[i]) store4(a.dst[i] + 4 * (u - begin), load4(a.src[i] + 4 * (u - begin)));
+      begin = a.end[i];
+    }
   }
 }
 
@@ -411,6 +434,31 @@ extern "C" int tfgpt2_gelu(const float* x, float* y, int64_t n, void* hip_stream
   if (misaligned(x) || misaligned(y)) return TFGFA_ERR_ALIGNMENT;
   hipLaunchKernelGGL(gelu_kernel, dim3((unsigned)blocks), dim3(kGeluThreads), 0,
                      (hipStream_t)hip_stream, x, y, (long long)n);
+  return launched();
+}
+
+extern "C" int tfgpt2_cast_bf16(int count, const float* const* src, void* const* dst,
+                                const int64_t* n, void* hip_stream) {
+  using namespace tfgpt2;
+  if (count < 0 || count > kMaxCasts) return TFGFA_ERR_BAD_SHAPE;
+  if (count > 0 && (!src || !dst || !n)) return TFGFA_ERR_NULL_POINTER;
+  Casts a = {};
+  long long units = 0;
+  for (int i = 0; i < count; ++i) {
+    if (n[i] < 0 || (n[i] & 3)) return TFGFA_ERR_BAD_SHAPE;
+    if (n[i] > 0 && (!src[i] || !dst[i])) return TFGFA_ERR_NULL_POINTER;
+    if (misaligned(src[i]) || misaligned(dst[i])) return TFGFA_ERR_ALIGNMENT;
+    units += n[i] / 4;
+    a.src[i] = src[i];
+    a.dst[i] = static_cast<__bf16*>(dst[i]);
+    a.end[i] = units;
+  }
+  a.count = count;
+  const long long blocks = (units + kCastThreads - 1) / kCastThreads;
+  if (blocks > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
+  if (blocks == 0) return TFGFA_OK;
+  hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(kCastThreads), 0,
+                     (hipStream_t)hip_stream, a);
   return launched();
 }
 

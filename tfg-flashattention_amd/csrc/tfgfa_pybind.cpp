@@ -157,6 +157,27 @@ void gpt2_gelu(std::uintptr_t x, std::uintptr_t y, std::int64_t n, std::uintptr_
   check(st, "tfgpt2_gelu");
 }
 
+// casts: (source, destination, count) of each array.
+void gpt2_cast_bf16(
+    const std::vector<std::tuple<std::uintptr_t, std::uintptr_t, std::int64_t>>& casts,
+    std::uintptr_t stream) {
+  if (casts.size() > TFGPT2_MAX_CASTS) check(TFGFA_ERR_BAD_SHAPE, "tfgpt2_cast_bf16");
+  const float* src[TFGPT2_MAX_CASTS];
+  void* dst[TFGPT2_MAX_CASTS];
+  std::int64_t n[TFGPT2_MAX_CASTS];
+  for (std::size_t i = 0; i < casts.size(); ++i) {
+    src[i] = reinterpret_cast<const float*>(std::get<0>(casts[i]));
+    dst[i] = reinterpret_cast<void*>(std::get<1>(casts[i]));
+    n[i] = std::get<2>(casts[i]);
+  }
+  int st;
+  {
+    py::gil_scoped_release nogil;
+    st = tfgpt2_cast_bf16((int)casts.size(), src, dst, n, reinterpret_cast<void*>(stream));
+  }
+  check(st, "tfgpt2_cast_bf16");
+}
+
 // parts: (weight, bias or 0, output) of each weight matrix.
 void gpt2_linear_rows(
     std::uintptr_t x, bool x_bf16, std::uintptr_t ln_scale, std::uintptr_t ln_shift, float eps,
@@ -255,6 +276,8 @@ PYBIND11_MODULE(_C, m) {
         py::arg("stream"));
   m.def("gpt2_gelu", &gpt2_gelu, "GELU (tanh form), elementwise", py::arg("x"), py::arg("y"),
         py::arg("n"), py::arg("stream"));
+  m.def("gpt2_cast_bf16", &gpt2_cast_bf16, "float32 -> bf16 copies in one launch",
+        py::arg("casts"), py::arg("stream"));
   m.def("gpt2_linear_rows", &gpt2_linear_rows,
         "A linear layer on few rows, with LayerNorm, bias, GELU and residual", py::arg("x"),
         py::arg("x_bf16"), py::arg("ln_scale"), py::arg("ln_shift"), py::arg("eps"),

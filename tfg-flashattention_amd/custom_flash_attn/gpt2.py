@@ -72,6 +72,13 @@ def gelu(x):
     return y
 
 
+def cast_bf16(pairs) -> None:
+    """dst.copy_(src) for each (src float32, dst bf16) pair of equal, multiple-of-4 sizes."""
+    dev = pairs[0][0].device
+    with torch.cuda.device(dev):
+        _C.gpt2_cast_bf16([(s.data_ptr(), d.data_ptr(), s.numel()) for s, d in pairs], _stream(dev))
+
+
 def rows_fit(rows: int, width: int, norm: bool) -> bool:
     """Whether :func:`linear_rows` takes ``rows`` rows of ``width`` values."""
     return (1 <= rows <= MAX_ROWS and width % 4 == 0 and width >= 4

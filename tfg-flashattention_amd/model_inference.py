@@ -127,6 +127,10 @@ ATTENTION_IMPLS: Dict[str, Callable] = {
 }
 
 
+# The built-in implementations that never read their mask (causal by construction).
+_MASKLESS = (_attn_functional, _attn_triton, _attn_hip, _attn_cuda)
+
+
 class MultiHeadAttention(nn.Module):
     """Causal multi-head self-attention (model_inference.py:39-94)."""
 
@@ -154,21 +158,61 @@ class MultiHeadAttention(nn.Module):
         return (_plain(self, MultiHeadAttention)
                 and all(_plain(m, nn.Linear) for m in (self.W_query, self.W_key, self.W_value, self.out_proj)))
 
+    def _cast_together(self, x) -> bool:
+        """Whether autocast's bf16 copies of x and of the four linears may be made in one launch:
+        bf16 autocast, plain float32 linears of one shape, an attention on the HIP kernels (which
+        take any row stride)."""
+        g = _gpt2() if x.is_cuda else None
+        if not (g is not None and self.impl_type in ("hip", "cuda", "triton") and g.eager()
+                and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+                and self._plain_linears() and _no_global_hooks()):
+            return False
+        wq, wk, wv, wo = self.W_query, self.W_key, self.W_value, self.out_proj
+        rows, cols = wq.weight.shape
+        return (x.dim() == 3 and x.shape[2] == cols and rows % 8 == 0 and cols % 8 == 0
+                and wk.weight.shape == wv.weight.shape == (rows, cols) and wo.weight.shape == (rows, rows)
+                and (wq.bias is None) == (wk.bias is None) == (wv.bias is None)
+                and g.takes(x, *(t for m in (wq, wk, wv, wo) for t in (m.weight, m.bias)),
+                            dtypes=(torch.float32, torch.bfloat16)))
+
+    def _project(self, x):
+        """Queries, keys and values of x as (b, n, heads, head_dim), and the output projection.
+
+        Under bf16 autocast (_cast_together) the copies of the weights, biases and x that autocast
+        would make one by one, x's for each linear, are made by one kernel, the three input weights
+        end to end, so that queries, keys and values are one GEMM and views of its result."""
+        b, n, _ = x.shape
+        H, hd = self.num_heads, self.head_dim
+        linears = (self.W_query, self.W_key, self.W_value, self.out_proj)
+        if not self._cast_together(x):
+            return (*(m(x).view(b, n, H, hd) for m in linears[:3]), self.out_proj)
+        rows, cols = self.W_query.weight.shape
+        sources = [m.weight for m in linears] + [m.bias for m in linears if m.bias is not None]
+        buf = torch.empty(sum(t.numel() for t in sources), dtype=torch.bfloat16, device=x.device)
+        copies = buf.split([t.numel() for t in sources])
+        pairs = list(zip(sources, copies))
+        if x.dtype != torch.bfloat16:
+            pairs.append((x, torch.empty_like(x, dtype=torch.bfloat16)))
+            x = pairs[-1][1]
+        _gpt2().cast_bf16(pairs)
+        wqkv, wo = buf[:3 * rows * cols].view(3 * rows, cols), copies[3].view(rows, rows)
+        at = wqkv.numel() + wo.numel()
+        bqkv = buf[at:at + 3 * rows] if self.W_query.bias is not None else None
+        bo = copies[-1] if self.out_proj.bias is not None else None
+        q, k, v = F.linear(x, wqkv, bqkv).view(b, n, 3, H, hd).unbind(2)
+        return q, k, v, lambda ctx: F.linear(ctx, wo, bo)
+
     def forward(self, x, kv_cache=None, layer: int = 0):
         if kv_cache is not None:
             return self._forward_cached(x, kv_cache, layer)
         b, num_tokens, _ = x.shape
-        queries = self.W_query(x)
-        keys = self.W_key(x)
-        values = self.W_value(x)
-        keys = keys.view(b, num_tokens, self.num_heads, self.head_dim).transpose(1, 2)
-        queries = queries.view(b, num_tokens, self.num_heads, self.head_dim).transpose(1, 2)
-        values = values.view(b, num_tokens, self.num_heads, self.head_dim).transpose(1, 2)
-        mask_bool = self.mask.bool()[:num_tokens, :num_tokens]
-        context_vec = ATTENTION_IMPLS[self.impl_type](queries, keys, values, mask_bool, self.dropout)
+        queries, keys, values, out_proj = self._project(x)
+        attend = ATTENTION_IMPLS[self.impl_type]
+        mask_bool = None if attend in _MASKLESS else self.mask.bool()[:num_tokens, :num_tokens]
+        context_vec = attend(queries.transpose(1, 2), keys.transpose(1, 2), values.transpose(1, 2),
+                             mask_bool, self.dropout)
         context_vec = context_vec.contiguous().view(b, num_tokens, self.d_out)
-        return self.out_proj(context_vec)
-
+        return out_proj(context_vec)
 
     def _forward_cached(self, x, cache, layer):
         """Attention against a KV cache (no counterpart in the reference, whose generate()
@@ -186,9 +230,7 @@ class MultiHeadAttention(nn.Module):
             raise ValueError(f"cached attention runs on the HIP kernels; impl_type is {self.impl_type!r}")
         b, n, _ = x.shape
         H, hd = self.num_heads, self.head_dim
-        q = self.W_query(x).view(b, n, H, hd)
-        k = self.W_key(x).view(b, n, H, hd)
-        v = self.W_value(x).view(b, n, H, hd)
+        q, k, v, out_proj = self._project(x)
         kc, vc = cache.k[layer], cache.v[layer]
         ctx = torch.empty(b, n, H, hd, dtype=q.dtype, device=q.device)
         if cache.length == 0:
@@ -203,7 +245,7 @@ class MultiHeadAttention(nn.Module):
                                      out=ctx[:, 0], workspace=cache.workspace)
         else:
             raise NotImplementedError("a cache that already holds tokens takes one new token per step")
-        return self.out_proj(ctx.view(b, n, self.d_out))
+        return out_proj(ctx.view(b, n, self.d_out))
 
 
 class KVCache:
