@@ -1,0 +1,93 @@
+"""The forward's key-split workgroups and head-dim instances at the sizes where they can go wrong:
+ends of 32-key halves, 64-key tiles and query blocks, groups without a tile, head dims at the edges
+of the compiled ones (GPU box only).  Each shape's comment names the kernel it reaches on 256 CUs.
+
+Reference: float32 attention from the same 16-bit values.  With u the unit roundoff of the type
+(2^-8 bf16, 2^-11 fp16), the probabilities, their sum and the output are each rounded once:
+|dO| <= 3 u max|V|.  The LSE is float32 throughout: scores of magnitude up to 2^6 carry about
+sqrt(D) roundings of 2^-24, below 1e-4.
+"""
+import math
+
+import pytest
+import torch
+
+import custom_flash_attn
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+
+#        B, H, Nq, Nk, causal
+NARROW = [  # head dims up to 64
+    (1, 1, 1025, 1025, True),    # 2 row waves x 4 key groups, one row past a block
+    (1, 2, 33, 1100, False),     # the same, unmasked, a ragged last tile
+    (1, 1, 1300, 1090, True),    # the same, rows past the last key
+    (1, 130, 1, 1, True),        # 2 x 2: one key, the second group without a tile
+    (1, 130, 100, 100, True),
+    (1, 131, 65, 65, True),
+    (2, 65, 127, 127, True),
+    (1, 44, 641, 641, True),
+    (1, 130, 5, 1001, False),    # 4 x 2, unmasked
+    (1, 150, 127, 1056, False),
+    (1, 20, 2049, 2049, True),   # 4 x 2, causal
+    (1, 60, 640, 640, True),     # whole blocks
+]
+WIDE = [  # head dims past 64
+    (1, 3, 130, 130, True),      # 32-row blocks, 4 key waves
+    (1, 70, 65, 65, True),       # 2 x 2
+    (1, 70, 1, 1, True),
+    (1, 25, 600, 97, True),
+    (1, 96, 33, 289, False),
+    (1, 35, 700, 700, True),     # 4 x 2
+    (1, 200, 3, 705, False),
+    (1, 20, 2049, 2049, True),
+    (1, 130, 200, 130, False),   # whole blocks
+]
+
+
+def _reference(q, k, v, causal):
+    q, k, v = q.float(), k.float(), v.float()
+    s = torch.matmul(q, k.transpose(-1, -2).contiguous()) / math.sqrt(q.shape[-1])
+    if causal:
+        s.masked_fill_(torch.ones(s.shape[-2:], dtype=torch.bool, device=DEV).triu(1), -math.inf)
+    return torch.matmul(torch.softmax(s, -1), v), torch.logsumexp(s, -1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("D", [8, 32, 40, 64, 72, 96, 104, 128])
+def test_every_plan_and_head_dim(D, dtype):
+    for B, H, Nq, Nk, causal in (NARROW if D <= 64 else WIDE):
+        print(f"D={D} {dtype} B={B} H={H} Nq={Nq} Nk={Nk} causal={causal}", flush=True)
+        g = torch.Generator(device=DEV).manual_seed(Nq * 7 + Nk + D)
+        q, k, v = (torch.randn((B, n, H, D), device=DEV, generator=g).to(dtype).transpose(1, 2)
+                   for n in (Nq, Nk, Nk))
+        q = q * 2
+        buf = torch.full((B, Nq, H, D + 8), 1000.0, dtype=dtype, device=DEV)
+        o, lse = custom_flash_attn.attention(q, k, v, out=buf[..., :D].transpose(1, 2), causal=causal,
+                                             return_lse=True)
+        o_ref, lse_ref = _reference(q, k, v, causal)
+        assert (o.float() - o_ref).abs().max().item() <= 3 * U[dtype] * v.abs().max().item()
+        assert (lse - lse_ref).abs().max().item() <= 1e-4
+        assert torch.equal(buf[..., D:], torch.full_like(buf[..., D:], 1000.0))
+        # Without the LSE, and from contiguous copies: the same arithmetic, bit for bit.
+        assert torch.equal(custom_flash_attn.attention(q, k, v, causal=causal), o)
+        c = custom_flash_attn.attention(q.contiguous(), k.contiguous(), v.contiguous(), causal=causal)
+        assert torch.equal(c, o)
+
+
+@pytest.mark.parametrize("B,H,N", [(1, 4, 1500), (2, 16, 777), (1, 25, 2048)])
+def test_key_groups_merge_extreme_rows(B, H, N):
+    """Rows whose keys differ by hundreds between groups (one group's weight is 0), rows of equal
+    scores, and values at the type's largest: every merge weight stays finite."""
+    g = torch.Generator(device=DEV).manual_seed(N)
+    q, k, v = (torch.randn((B, H, N, 64), device=DEV, generator=g).to(torch.bfloat16) for _ in range(3))
+    q[:, :, ::3] = 0
+    k[:, :, 64:96] *= 40
+    v[:, 0] = 3.0e38
+    o, lse = custom_flash_attn.forward_lse(q, k, v)
+    o_ref, lse_ref = _reference(q[:, 1:], k[:, 1:], v[:, 1:], True)
+    assert (o[:, 1:].float() - o_ref).abs().max().item() <= 3 * U[torch.bfloat16] * v[:, 1:].abs().max().item()
+    assert ((lse[:, 1:] - lse_ref).abs() <= 1e-4 + 1e-5 * lse_ref.abs()).all()
+    assert torch.isfinite(lse).all()

@@ -15,6 +15,10 @@
 //   diagonal (never computed) or the single diagonal block (element mask).  Tiles wholly above
 //   the diagonal of the whole block are never loaded.  Workgroups are issued heaviest query
 //   block first.
+//   Where that leaves CUs idle (small batches), the same kernel runs with kS key groups of kR row
+//   waves: group g takes tiles g, g + kS, .. through a K/V ring of its own, and the groups' softmax
+//   states merge through LDS at the end; the grids too small even for that run fwd_split_kernel.
+//   choose_plan holds the lines between them and the times they rest on.
 //
 // Per-wave software pipeline (32-key halves u = 0, 1, ...)
 //   half-step u:  O += V_{u-1} P_{u-1}   interleaved with   P_u = exp2(S_u - m)
@@ -77,6 +81,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -93,10 +98,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kDHalf = 64;                  // head dims per LDS tile layout ("dim half")
-constexpr int kWaves = 4;                   // waves per workgroup
-constexpr int kThreads = kWaves * 64;       // 256
 constexpr int kWaveRows = 32;               // query rows per wave (one MFMA column block)
-constexpr int kBlockRows = kWaves * kWaveRows;  // 128 query rows per workgroup
+constexpr int kBlockRows = 4 * kWaveRows;   // 128 query rows: the largest workgroup's block
 constexpr int kTileKeys = 64;               // keys per K/V tile
 constexpr int kKRowBytes = kDHalf * 2;      // 128 B per key row of one dim half in LDS
 constexpr int kHalfTileBytes = kTileKeys * kKRowBytes;  // 8 KiB (K or V, one dim half)
@@ -240,25 +243,36 @@ __device__ __forceinline__ uint32_t lds_addr(const unsigned char* p) {
   return (uint32_t)(uintptr_t)(const lds_void*)p;
 }
 
-// Compile-time shape of one kernel instance: head dims kD (64 or 128, = kDH dim halves of 64),
-// element type T, and kMaskD: the actual head dim D may be below kD (a multiple of 8); 16-B
+// Compile-time shape of one kernel instance: head dims kD (32, 64, 96 or 128, held in kDH dim
+// halves of 64 and computed as kQC contraction chunks of 16 and kOT output tiles of 32), element
+// type T, and kMaskD: the actual head dim D may be below 64 * kDH (a multiple of 8); 16-B
 // chunks of dims >= D load zeros and are not stored.  kLse: the LSE is written, so the fp32
-// sum l_run is kept (without it only l_p, which normalises O, is summed).
-template <int kD_, typename T_, bool kMaskD_, bool kLse_ = true>
+// sum l_run is kept (without it only l_p, which normalises O, is summed).  kR waves of 32 query
+// rows share each K/V tile; kS such groups of a workgroup take the tiles in turn (group g: tiles
+// g, g + kS, ..) and merge their softmax states at the end.
+template <int kD_, typename T_, bool kMaskD_, bool kLse_ = true, int kR_ = 4, int kS_ = 1>
 struct Shape {
   static constexpr int kD = kD_;
   static constexpr bool kLse = kLse_;
-  static constexpr int kDH = kD_ / kDHalf;
+  static constexpr int kDH = (kD_ + kDHalf - 1) / kDHalf;
+  static constexpr int kQC = kD_ / 16;
+  static constexpr int kOT = kD_ / 32;
   static constexpr bool kMaskD = kMaskD_;
+  static constexpr int kR = kR_;
+  static constexpr int kS = kS_;
+  static constexpr int kWaves = kR_ * kS_;
+  static constexpr int kBlockRows = kR_ * kWaveRows;  // query rows per workgroup
   typedef T_ T;
-  static constexpr int kLoadsPerWave = 4 * kDH;  // transfers per tile step per wave (K and V)
+  static constexpr int kRowBlocks = 8 / kR_;  // 8-row blocks of a K (or V) tile each wave loads
+  static constexpr int kLoadsPerWave = 2 * kRowBlocks * kDH;  // transfers per tile step per wave (K and V)
   // K ring slots.  2: K_{j+2} is issued after tile step j's barrier, into the slot of K_j (last
   // read by half-step 2j, before the barrier), and has two half-steps to land.  3: K_{j+2} is
   // issued at the start of step j, into the slot of K_{j-1}, and has three.  Head dim 64 uses 2
   // (as fast, measured, and it leaves LDS for the Q stage); head dim 128 uses 3: 2 slots (a third
   // of the code, 64 KiB of LDS) measured 0.3-2.4% slower at d = 128, 120, 112, 72 and 96 (B1 H16
   // N8192), faster only at B8 H25 N1024 d = 96 (2.7%).
-  static constexpr int kKSlots = kD_ == 128 ? 3 : 2;
+  // Several groups: 2, so that two groups' rings fit at head dim 128.
+  static constexpr int kKSlots = kDH == 2 && kS_ == 1 ? 3 : 2;
   // V ring: 2 slots; V_{j+1} is issued after step j's barrier, into the slot of V_{j-1} (read by
   // half-step 2j, before the barrier).
   static constexpr int kVSlots = 2;
@@ -268,25 +282,36 @@ struct Shape {
   // that the compiler does not track, so the prologue waits for Q and K_0 only.  Head dim 64
   // (48 KiB of LDS per workgroup with the rings, three workgroups per CU); head dim 128 loads Q
   // into registers and waits for the whole prologue (its rings take 80 KiB).
-  static constexpr bool kQStage = kD_ == 64;
-  static_assert(kD_ == 64 || kD_ == 128, "compiled head dims");
+  static constexpr bool kQStage = kDH == 1;
+  // Waves per SIMD that the LDS leaves room for: three or two (head dims past 64) one-group
+  // workgroups a CU; two 4-wave workgroups of two groups, or one (past 64); one of 8 waves.
+  static constexpr int kSimdWaves = kS_ == 1 ? (kDH == 1 ? 3 : 2) : kWaves == 4 && kDH == 2 ? 1 : 2;
+  static_assert(kD_ % 32 == 0 && kD_ >= 32 && kD_ <= 128, "compiled head dims");
+  static_assert(kMaskD_ || kD_ % kDHalf == 0, "a dim half partly used is masked");
+  static_assert(4 % kR_ == 0 && 4 % kS_ == 0, "rows of a tile and of Q divide among the waves");
+
+  // MFMA i of a half's P.V: output tile and 16-key chunk.  Tiles go in pairs (the halves of a dim
+  // half), each pair's two tiles side by side for one chunk, then the odd last tile.
+  static constexpr int pv_tile(int i) { return i < 4 * (kOT / 2) ? 2 * (i >> 2) + (i & 1) : kOT - 1; }
+  static constexpr int pv_chunk(int i) { return i < 4 * (kOT / 2) ? (i >> 1) & 1 : i - 4 * (kOT / 2); }
 };
 
-// This wave's share of one K (or V) tile: rows [8*(2w), 8*(2w+2)) of each dim half as two
-// 1-KiB LDS blocks per dim half (dim half dh at byte dh * 8 KiB of the slot).  Lane i of a block
+// This wave's share of one K (or V) tile: kRowBlocks blocks of 8 rows of each dim half, 1 KiB of
+// LDS each (dim half dh at byte dh * 8 KiB of the slot); `wave` counts the group's kR waves.  Lane i of a block
 // fills physical chunk i%8 of row i/8, so it fetches the logical chunk that the swizzle maps
 // there: head dims 64*dh + 8*chunk .. +7, i.e. row bytes 128*dh + 16*chunk.
 // The lane's byte offset within a tile (from the tile's first row) is the same for every tile,
 // so it is computed once (tile_offsets); per tile only the descriptor moves (tile_desc), in
 // scalar registers, and the transfers take no VALU work.
 template <class Sh>
-__device__ __forceinline__ void tile_offsets(int (*koff)[2], int (*voff)[2], int k_row_bytes,
-                                             int v_row_bytes, int wave, int lane, int d_chunks) {
+__device__ __forceinline__ void tile_offsets(int (*koff)[Sh::kRowBlocks], int (*voff)[Sh::kRowBlocks],
+                                             int k_row_bytes, int v_row_bytes, int wave, int lane,
+                                             int d_chunks) {
 #pragma unroll
   for (int dh = 0; dh < Sh::kDH; ++dh)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = (2 * wave + i) * 8 + (lane >> 3);
+    for (int i = 0; i < Sh::kRowBlocks; ++i) {
+      const int row = (Sh::kRowBlocks * wave + i) * 8 + (lane >> 3);
       const int kc = 8 * dh + ((lane & 7) ^ swz_k(row));  // 16-B chunk of the row in memory
       const int vc = 8 * dh + ((lane & 7) ^ swz_v(row));
       int ko = row * k_row_bytes + (kc << 4);
@@ -315,35 +340,37 @@ __device__ __forceinline__ i32x4 tile_desc(i32x4 desc, int k0, int row_bytes) {
 
 template <class Sh>
 __device__ __forceinline__ void issue_tile(i32x4 desc, int row_bytes, unsigned char* dst, int k0,
-                                           int wave, const int (*off)[2]) {
+                                           int wave, const int (*off)[Sh::kRowBlocks]) {
   const i32x4 d = tile_desc(desc, k0, row_bytes);
 #pragma unroll
   for (int dh = 0; dh < Sh::kDH; ++dh)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      lds_transfer(d, lds_addr(dst + dh * kHalfTileBytes + (2 * wave + i) * 1024), off[dh][i]);
+    for (int i = 0; i < Sh::kRowBlocks; ++i)
+      lds_transfer(d, lds_addr(dst + dh * kHalfTileBytes + (Sh::kRowBlocks * wave + i) * 1024), off[dh][i]);
 }
 
-// The workgroup's Q stage (head dim 64): 4 KiB of LDS per wave, allocated only by the instances
-// that call this.
+// The workgroup's Q stage (head dims up to 64): 4 KiB of LDS per 32 rows, allocated only by the
+// instances that call this.
 template <class Sh>
 __device__ __forceinline__ unsigned char* q_stage() {
-  __shared__ __attribute__((aligned(1024))) unsigned char qst[kBlockRows * kKRowBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char qst[Sh::kBlockRows * kKRowBytes];
   return qst;
 }
 
-// This wave's 32 query rows, from the descriptor's first row, into its 4-KiB LDS stage (head
-// dim 64): row r at byte 128 r, logical 16-B chunk c (head dims 8c .. 8c+7) at physical chunk
+// 32 query rows, from the descriptor's first row, into their 4-KiB LDS stage (head dims up to
+// 64): row r at byte 128 r, logical 16-B chunk c (head dims 8c .. 8c+7) at physical chunk
 // c ^ swz_k(r), so the 8 (or 16) consecutive rows of one ds_read_b128 hit distinct banks.  Four
-// 1-KiB transfers; rows past the sequence end read zero.
+// 1-KiB transfers, divided among the kS waves that use the rows; rows past the sequence end read
+// zero.
 template <class Sh>
 __device__ __forceinline__ void issue_q_stage(i32x4 qdesc, int row_bytes, unsigned char* dst,
-                                              int d_chunks) {
+                                              int d_chunks, int grp) {
   static_assert(Sh::kDH == 1, "the Q stage holds 128-B rows");
   int lane;
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
+  for (int i = 0; i < 4 / Sh::kS; ++i) {
+    const int t = 4 / Sh::kS * grp + i;
     const int row = 8 * t + (lane >> 3);
     const int lc = (lane & 7) ^ swz_k(row);
     int off = row * row_bytes + (lc << 4);
@@ -383,8 +410,8 @@ struct Lds {
 template <class Sh>
 struct WaveState {
   typedef typename Elem<typename Sh::T>::v8 v8;
-  v8 qop[4 * Sh::kDH];   // Q^T operand: Q[qrow][16c + 8h .. +7]
-  f32x16 o[2 * Sh::kDH]; // O^T accumulators: o[t] holds d = 32t .. 32t+31
+  v8 qop[Sh::kQC];       // Q^T operand: Q[qrow][16c + 8h .. +7]
+  f32x16 o[Sh::kOT];     // O^T accumulators: o[t] holds d = 32t .. 32t+31
   f32x16 s;              // S^T of the half being softmaxed: register t = key 8(t/4) + 4h + t%4
   v8 pb[2];              // P^T of the previous half, waiting for its P.V
   float m_run;           // exp2 offset (a running max of scale*log2e*s, moved lazily)
@@ -395,8 +422,8 @@ struct WaveState {
   int voff[2][2];        // V^T transposing-read LDS offsets (within a V dim half, keys 0..15)
 };
 
-// S^T = K Q^T for key half kHalf of the tile in K slot kSlot (4 MFMAs per dim half; dim half dh
-// at byte dh * kDhBytes of the slot).
+// S^T = K Q^T for key half kHalf of the tile in K slot kSlot (one MFMA per 16 head dims; dim half
+// dh at byte dh * kDhBytes of the slot).
 template <class Sh, int kSlot, int kHalf, int kDhBytes = kHalfTileBytes>
 __device__ __forceinline__ f32x16 qk_half(const WaveState<Sh>& w, const Lds& lds) {
   typedef typename Elem<typename Sh::T>::v8 v8;
@@ -404,38 +431,31 @@ __device__ __forceinline__ f32x16 qk_half(const WaveState<Sh>& w, const Lds& lds
 #pragma unroll
   for (int t = 0; t < 16; ++t) acc[t] = 0.f;
 #pragma unroll
-  for (int dh = 0; dh < Sh::kDH; ++dh) {
-    const unsigned char* kt = lds.k[kSlot] + dh * kDhBytes + kHalf * 32 * kKRowBytes;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const v8 a = *reinterpret_cast<const v8*>(kt + w.koff[c]);
-      acc = Elem<typename Sh::T>::mfma(a, w.qop[4 * dh + c], acc);
-    }
+  for (int i = 0; i < Sh::kQC; ++i) {
+    const unsigned char* kt = lds.k[kSlot] + (i >> 2) * kDhBytes + kHalf * 32 * kKRowBytes;
+    const v8 a = *reinterpret_cast<const v8*>(kt + w.koff[i & 3]);
+    acc = Elem<typename Sh::T>::mfma(a, w.qop[i], acc);
   }
   return acc;
 }
 
-// O^T += V^T P^T for key half kHalf of the tile in V slot kSlot, with P^T = w.pb (4 MFMAs per
-// dim half).  Element e of chunk cc in lane half h is key 16*cc + 8*(e/4) + 4*h + e%4 of the
+// O^T += V^T P^T for key half kHalf of the tile in V slot kSlot, with P^T = w.pb (2 MFMAs per 32
+// head dims).  Element e of chunk cc in lane half h is key 16*cc + 8*(e/4) + 4*h + e%4 of the
 // key half: two transposing reads of 4 keys each.  Dim half dh at byte dh * kDhBytes of the slot.
 template <class Sh, int kSlot, int kHalf, int kDhBytes = kHalfTileBytes>
 __device__ __forceinline__ void pv_half(WaveState<Sh>& w, const Lds& lds) {
   typedef typename Elem<typename Sh::T>::v8 v8;
 #pragma unroll
-  for (int dh = 0; dh < Sh::kDH; ++dh) {
-    const unsigned char* vt = lds.v[kSlot] + dh * kDhBytes + kHalf * 32 * kKRowBytes;
-#pragma unroll
-    for (int cc = 0; cc < 2; ++cc) {
-#pragma unroll
-      for (int dt = 0; dt < 2; ++dt) {
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(vt + w.voff[dt][0] + cc * 16 * kKRowBytes));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(vt + w.voff[dt][1] + cc * 16 * kKRowBytes));
-        const v8 va = __builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        w.o[2 * dh + dt] = Elem<typename Sh::T>::mfma(va, w.pb[cc], w.o[2 * dh + dt]);
-      }
-    }
+  for (int i = 0; i < 2 * Sh::kOT; ++i) {
+    const int t = Sh::pv_tile(i), cc = Sh::pv_chunk(i);
+    const unsigned char* vt =
+        lds.v[kSlot] + (t >> 1) * kDhBytes + (kHalf * 32 + cc * 16) * kKRowBytes;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4*)(vt + w.voff[t & 1][0]));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (__attribute__((address_space(3))) s16x4*)(vt + w.voff[t & 1][1]));
+    const v8 va = __builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    w.o[t] = Elem<typename Sh::T>::mfma(va, w.pb[cc], w.o[t]);
   }
 }
 
@@ -475,7 +495,7 @@ __device__ __forceinline__ void move_offset(WaveState<Sh>& w, float mx, float sc
     if constexpr (Sh::kLse) w.l_run *= alpha;
     w.l_p *= alpha;
 #pragma unroll
-    for (int i = 0; i < 2 * Sh::kDH; ++i)
+    for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
       for (int t = 0; t < 16; ++t) w.o[i][t] *= alpha;
   }
@@ -517,13 +537,13 @@ template <class Sh, int kVs, int kVh>
 __device__ __forceinline__ typename Elem<typename Sh::T>::v8 v_operand(const WaveState<Sh>& w,
                                                                       const Lds& lds, int i) {
   typedef typename Elem<typename Sh::T>::v8 v8;
-  const int dh = i >> 2, cc = (i >> 1) & 1, dt = i & 1;
+  const int t = Sh::pv_tile(i), cc = Sh::pv_chunk(i);
   const unsigned char* vt =
-      lds.v[kVs] + dh * kHalfTileBytes + kVh * 32 * kKRowBytes + cc * 16 * kKRowBytes;
+      lds.v[kVs] + (t >> 1) * kHalfTileBytes + kVh * 32 * kKRowBytes + cc * 16 * kKRowBytes;
   const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) s16x4*)(vt + w.voff[dt][0]));
+      (__attribute__((address_space(3))) s16x4*)(vt + w.voff[t & 1][0]));
   const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) s16x4*)(vt + w.voff[dt][1]));
+      (__attribute__((address_space(3))) s16x4*)(vt + w.voff[t & 1][1]));
   return __builtin_bit_cast(v8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
@@ -559,8 +579,9 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
                                            float inv_scale_log2) {
   typedef typename Sh::T T;
   typedef typename Elem<T>::v8 v8;
-  constexpr int kPv = 4 * Sh::kDH;
-  constexpr int kS = 4 * Sh::kDH;
+  constexpr int kPv = 2 * Sh::kOT;
+  constexpr int kQk = Sh::kQC;
+  constexpr int kLseChunk = kQk > 2 ? 2 : 1;  // the S chunk that sums for the LSE
   constexpr float kSumBound = Elem<T>::kSumBound;
   v8 vop[2];
   if constexpr (kPV) {
@@ -573,8 +594,8 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
   v8 kop[2];
 #pragma unroll
   for (int i = 0; i < kPv; ++i) {
-    const int dh = i >> 2, cc = (i >> 1) & 1, dt = i & 1;
-    if constexpr (kPV) w.o[2 * dh + dt] = Elem<T>::mfma(vop[i & 1], w.pb[cc], w.o[2 * dh + dt]);
+    const int t = Sh::pv_tile(i);
+    if constexpr (kPV) w.o[t] = Elem<T>::mfma(vop[i & 1], w.pb[Sh::pv_chunk(i)], w.o[t]);
     if (i + 2 < kPv) {
       if constexpr (kPV) vop[i & 1] = v_operand<Sh, kVs, kVh>(w, lds, i + 2);
     } else {
@@ -603,9 +624,9 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
     }
   };
 #pragma unroll
-  for (int i = 0; i < kS; ++i) {
+  for (int i = 0; i < kQk; ++i) {
     acc = Elem<T>::mfma(kop[i & 1], w.qop[i], acc);
-    if (i + 2 < kS) kop[i & 1] = k_operand<Sh, kKs, kKh>(w, lds, i + 2);
+    if (i + 2 < kQk) kop[i & 1] = k_operand<Sh, kKs, kKh>(w, lds, i + 2);
     if (i == 0) {
       convert(p);
       asm volatile("" : "+v"(w.pb[0]), "+v"(w.pb[1]));
@@ -624,7 +645,7 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
         if constexpr (Sh::kLse) w.l_run *= alpha;
         w.l_p *= alpha;
 #pragma unroll
-        for (int j = 0; j < 2 * Sh::kDH; ++j)
+        for (int j = 0; j < Sh::kOT; ++j)
 #pragma unroll
           for (int t = 0; t < 16; ++t) w.o[j][t] *= alpha;
 #pragma unroll
@@ -635,7 +656,8 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
       }
       w.l_p = hs;
       asm volatile("" : "+v"(w.l_p));
-    } else if (i == 2 && Sh::kLse) {
+    }
+    if (i == kLseChunk && Sh::kLse) {
       float s0 = p[0], s1 = p[1];
 #pragma unroll
       for (int t = 2; t < 16; t += 2) {
@@ -650,17 +672,27 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
   w.s = acc;
 }
 
-// Loop-invariant inputs of the pipeline.
+// Loop-invariant inputs of the pipeline.  Tiles and halves are counted within the wave's group
+// (group g's tile j is tile kS j + g of the sequence).
+template <class Sh>
 struct StepArgs {
   i32x4 k_rsrc, v_rsrc;
   int k_row_bytes, v_row_bytes;  // byte distance between consecutive K (V) rows of a head
   int d_chunks;  // 16-B chunks of a row holding head dims < D
-  int k_lane[2][2], v_lane[2][2];  // this lane's byte offsets within a K / V tile (tile_offsets)
-  int nT;        // 64-key tiles loaded by the workgroup
+  // This lane's byte offsets within a K / V tile (tile_offsets).
+  int k_lane[Sh::kDH][Sh::kRowBlocks], v_lane[Sh::kDH][Sh::kRowBlocks];
+  int nT;        // tile steps of the workgroup (its groups' most 64-key tiles)
+  int nLoad;     // tiles this group loads (a prefix of the steps)
   int nAct;      // 32-key halves this wave computes (a prefix)
   int nFull;     // halves this wave computes without an element mask (a prefix of the above)
-  int wave, lane, h, last_key;
+  int wave, grp, lane, h, last_key;  // wave: within the group
   float scale_log2, inv_scale_log2;
+
+  // First key of the group's tile j, and of its half u.
+  __device__ __forceinline__ int tile_key(int j) const { return (j * Sh::kS + grp) * kTileKeys; }
+  __device__ __forceinline__ int half_key(int u) const {
+    return Sh::kS == 1 ? u * 32 : tile_key(u >> 1) + (u & 1) * 32;
+  }
 };
 
 // Half-step u: P.V of half u-1 (V slot kVs, half kVh), softmax of half u, S of half u+1 (K
@@ -672,9 +704,9 @@ struct StepArgs {
 // Otherwise (tail): u = nAct is the P.V of the last half only; u > nAct does nothing.
 template <class Sh, int kVs, int kVh, int kKs, int kKh, bool kSteady, bool kPV = true>
 __device__ __forceinline__ void half_step(WaveState<Sh>& w, const Lds& lds, int u,
-                                          const StepArgs& a) {
+                                          const StepArgs<Sh>& a) {
   if (!kSteady && u > a.nAct) return;
-  if (u >= a.nFull && u < a.nAct) mask_half(w, a.last_key - u * 32 - 4 * a.h);
+  if (u >= a.nFull && u < a.nAct) mask_half(w, a.last_key - a.half_key(u) - 4 * a.h);
   if (kSteady) {
     fused_step<Sh, kVs, kVh, kKs, kKh, kPV>(w, lds, a.scale_log2, a.inv_scale_log2);
     return;
@@ -693,15 +725,14 @@ __device__ __forceinline__ void half_step(WaveState<Sh>& w, const Lds& lds, int 
 // half-step 2j+1.
 template <class Sh, int kKs, int kVs, bool kSteady, bool kFirst = false>
 __device__ __forceinline__ void tile_step(WaveState<Sh>& w, const Lds& lds, int j,
-                                          const StepArgs& a) {
+                                          const StepArgs<Sh>& a) {
   constexpr int kKN = Sh::kKSlots;
   constexpr int kKNext = (kKs + 1) % kKN;
   constexpr int kKNext2 = (kKs + 2) % kKN;  // K_{j-1}'s slot (3 slots), K_j's (2 slots)
   constexpr int kVOther = kVs ^ 1;          // V_{j-1}, then V_{j+1}
-  const bool k2 = j + 2 < a.nT, v1 = j + 1 < a.nT;
+  const bool k2 = j + 2 < a.nLoad, v1 = j + 1 < a.nLoad;
   if (kKN == 3 && k2)
-    issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[kKNext2], (j + 2) * kTileKeys, a.wave,
-                   a.k_lane);
+    issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[kKNext2], a.tile_key(j + 2), a.wave, a.k_lane);
   // Half 2j: P.V of half 2j-1 (V_{j-1}, keys 32..63), S of half 2j+1 (K_j, keys 32..63).
   half_step<Sh, kVOther, 1, kKs, 1, kSteady, !kFirst>(w, lds, 2 * j, a);
   // K_{j+1} and V_j were issued by step j-1 (step 0: by the prologue); only K_{j+2}, issued
@@ -712,11 +743,9 @@ __device__ __forceinline__ void tile_step(WaveState<Sh>& w, const Lds& lds, int 
     wait_vmcnt<0>();
   lds_barrier();
   if (v1)
-    issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[kVOther], (j + 1) * kTileKeys, a.wave,
-                   a.v_lane);
+    issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[kVOther], a.tile_key(j + 1), a.wave, a.v_lane);
   if (kKN == 2 && k2)
-    issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[kKNext2], (j + 2) * kTileKeys, a.wave,
-                   a.k_lane);
+    issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[kKNext2], a.tile_key(j + 2), a.wave, a.k_lane);
   // Half 2j+1: P.V of half 2j (V_j, keys 0..31), S of half 2j+2 (K_{j+1}, keys 0..31).
   half_step<Sh, kVs, 0, kKNext, 0, kSteady>(w, lds, 2 * j + 1, a);
 }
@@ -724,7 +753,7 @@ __device__ __forceinline__ void tile_step(WaveState<Sh>& w, const Lds& lds, int 
 // Tile step j with its slots chosen at run time (j % kPeriod).
 template <class Sh, bool kSteady, int kP = 0>
 __device__ __forceinline__ void tile_step_at(WaveState<Sh>& w, const Lds& lds, int j,
-                                             const StepArgs& a) {
+                                             const StepArgs<Sh>& a) {
   if constexpr (kP < Sh::kPeriod) {
     if (j % Sh::kPeriod == kP)
       tile_step<Sh, kP % Sh::kKSlots, kP % Sh::kVSlots, kSteady>(w, lds, j, a);
@@ -737,7 +766,7 @@ __device__ __forceinline__ void tile_step_at(WaveState<Sh>& w, const Lds& lds, i
 // compile time.
 template <class Sh, int kJ0 = 0, int kP = 0>
 __device__ __forceinline__ void steady_period(WaveState<Sh>& w, const Lds& lds, int j0,
-                                              const StepArgs& a) {
+                                              const StepArgs<Sh>& a) {
   if constexpr (kP < Sh::kPeriod) {
     tile_step<Sh, (kJ0 + kP) % Sh::kKSlots, (kJ0 + kP) % Sh::kVSlots, true>(w, lds, j0 + kP, a);
     steady_period<Sh, kJ0, kP + 1>(w, lds, j0, a);
@@ -748,7 +777,7 @@ __device__ __forceinline__ void steady_period(WaveState<Sh>& w, const Lds& lds, 
 // kPeriod), slots at compile time.
 template <class Sh, int kJ0 = 0, int kP = 0>
 __device__ __forceinline__ void steady_rest(WaveState<Sh>& w, const Lds& lds, int j0, int n,
-                                            const StepArgs& a) {
+                                            const StepArgs<Sh>& a) {
   if constexpr (kP + 1 < Sh::kPeriod) {
     if (j0 + kP < n) {
       tile_step<Sh, (kJ0 + kP) % Sh::kKSlots, (kJ0 + kP) % Sh::kVSlots, true>(w, lds, j0 + kP, a);
@@ -774,11 +803,11 @@ __device__ __forceinline__ void store_o(const WaveState<Sh>& w, unsigned char* s
   typedef typename Sh::T T;
   typedef typename Elem<T>::v4 v4;
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-  constexpr int kChunks = Sh::kD / 8;  // 16-B chunks per row
-  constexpr int kRowB = Sh::kD * 2;
+  constexpr int kChunks = 8 * Sh::kDH;  // 16-B chunks per row of the stage
+  constexpr int kRowB = 16 * kChunks;
   const int r = lane & 31, h = lane >> 5;
 #pragma unroll
-  for (int i = 0; i < 2 * Sh::kDH; ++i)
+  for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       // Register 4g + e of tile i holds dim 32i + 8g + 4h + e: chunk 4i + g, bytes 8h .. 8h+7.
@@ -808,6 +837,99 @@ struct Strides {
   long long b, h, n;
 };
 
+// Merge of several waves' softmax states over the same 32 rows, through LDS, with the log-sum-exp
+// rule (offset m_w, rounded-probability sum lp_w, fp32 sum l_w, unnormalised O_w):
+//   M = max_w m_w,  a_w = 2^(m_w - M),  O = sum_w a_w O_w / sum_w a_w lp_w,
+//   LSE = (M + log2 sum_w a_w l_w) ln 2.
+// A wave with no half contributes m_w = -inf (a_w = 0).
+// A wave's partial: its unnormalised O rows (fp32, row-major, 64 * kDH columns, 16-B chunk c of
+// row r at physical chunk c ^ (r % (16 kDH))) and its row statistics.
+template <class Sh>
+struct Partial {
+  static constexpr int kC4 = 16 * Sh::kDH;  // 16-B fp32 chunks per row
+  static constexpr int kC8 = 8 * Sh::kDH;   // 8-dim items per row: 16 B of O
+  static constexpr int kRowB = 16 * kC4;
+  static constexpr int kBytes = kWaveRows * kRowB;
+};
+struct PartialStats {
+  float m[kWaveRows], lp[kWaveRows], l[kWaveRows];
+};
+
+template <class Sh>
+__device__ __forceinline__ void publish_partial(const WaveState<Sh>& w, unsigned char* opart,
+                                                PartialStats* st) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef Partial<Sh> P;
+  const float lp = pair_sum(w.l_p);
+  const float lr = Sh::kLse ? pair_sum(w.l_run) : 0.f;
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  const int r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < Sh::kOT; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      // Register 4g + e of tile i holds dim 32i + 8g + 4h + e: fp32 chunk 8i + 2g + h.
+      const f32x4 x = {w.o[i][4 * g], w.o[i][4 * g + 1], w.o[i][4 * g + 2], w.o[i][4 * g + 3]};
+      const int c = 8 * i + 2 * g + h;
+      *reinterpret_cast<f32x4*>(opart + r * P::kRowB + ((c ^ (r % P::kC4)) << 4)) = x;
+    }
+  if (h == 0) {
+    st->m[r] = w.m_run;
+    st->lp[r] = lp;
+    st->l[r] = lr;
+  }
+}
+
+// Row R, head dims 8 c8 .. 8 c8 + 7 of the merge of kParts partials (opart_stride bytes and
+// st_stride records apart), stored to the query row qr: each lane stores 16 B and kC8 lanes a whole
+// row (non-temporal, as in store_o).
+template <class Sh, int kParts>
+__device__ __forceinline__ void merge_item(const unsigned char* opart, int opart_stride,
+                                           const PartialStats* st, int st_stride, int R, int c8,
+                                           int qr, int Nq, int d_chunks, typename Sh::T* O,
+                                           long long o_rs, float* lse_head) {
+  typedef typename Sh::T T;
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  typedef Partial<Sh> P;
+  float M = -INFINITY;
+#pragma unroll
+  for (int v = 0; v < kParts; ++v) M = fmaxf(M, st[v * st_stride].m[R]);
+  float lsum = 0.f, lrun = 0.f;
+  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int v = 0; v < kParts; ++v) {
+    const float av = __builtin_amdgcn_exp2f(st[v * st_stride].m[R] - M);
+    lsum = fmaf(av, st[v * st_stride].lp[R], lsum);
+    if constexpr (Sh::kLse) lrun = fmaf(av, st[v * st_stride].l[R], lrun);
+    const unsigned char* src = opart + v * opart_stride + R * P::kRowB;
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(src + (((2 * c8) ^ (R % P::kC4)) << 4));
+    const f32x4 x1 = *reinterpret_cast<const f32x4*>(src + (((2 * c8 + 1) ^ (R % P::kC4)) << 4));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc0[e] = fmaf(av, x0[e], acc0[e]);
+      acc1[e] = fmaf(av, x1[e], acc1[e]);
+    }
+  }
+  const float inv = 1.0f / lsum;
+  typename Elem<T>::v8 ov;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    ov[e] = (T)(acc0[e] * inv);
+    ov[4 + e] = (T)(acc1[e] * inv);
+  }
+  if (qr < Nq && (!Sh::kMaskD || c8 < d_chunks)) {
+    u32x4* dst = reinterpret_cast<u32x4*>(O + (long long)qr * o_rs + 8 * c8);
+    if constexpr (Sh::kMaskD)
+      *dst = __builtin_bit_cast(u32x4, ov);
+    else
+      __builtin_nontemporal_store(__builtin_bit_cast(u32x4, ov), dst);
+  }
+  if (Sh::kLse && lse_head != nullptr && c8 == 0 && qr < Nq)
+    lse_head[qr] = (M + __builtin_amdgcn_logf(lrun)) * kLn2;
+}
+
 // One instance per (head dims, element type, dim masking, layout).  kDense: every operand is
 // the contiguous (B, H, N, kD) layout with N_q = N_k, so row strides are compile-time and the
 // stride arguments are not read.
@@ -819,24 +941,21 @@ struct Strides {
 // argument segment first (an L2 round trip on a CU's first workgroup: 0.3 us of a config-1
 // launch).  The LSE pointer, H, D and the strides follow; the strided instances load them.
 template <class Sh, bool kDense>
-__global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
+__global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
     const void* __restrict__ Qv, const void* __restrict__ Kv, const void* __restrict__ Vv,
     void* __restrict__ Ov, int BH, int Nq, int Nk, int nQB, int causal, float scale_log2,
     float* __restrict__ LSE, int H, int D, Strides qs, Strides ks, Strides vs, Strides os) {
   typedef typename Sh::T T;
   typedef typename Elem<T>::v8 v8;
-  typedef typename Elem<T>::v4 v4;
   constexpr int kSlotBytes = Sh::kDH * kHalfTileBytes;
+  constexpr int kRingBytes = (Sh::kVSlots + Sh::kKSlots) * kSlotBytes;  // of one group
   constexpr int kDenseRowBytes = Sh::kD * 2;
   // The V slots first, then the K slots: a ds_read reaches 64 KiB past its base register with
   // an immediate offset, and at head dim 128 (80 KiB) only the third K slot lies beyond, read by
   // 8 of a half-step's 24 reads one tile step in three (with the V ring there, half of all
   // tile steps paid an address add per V read).
-  __shared__ __attribute__((aligned(1024)))
-  unsigned char ring[(Sh::kVSlots + Sh::kKSlots) * kSlotBytes];
+  __shared__ __attribute__((aligned(1024))) unsigned char rings[Sh::kS * kRingBytes];
   constexpr int kK0 = Sh::kVSlots * kSlotBytes;
-  const Lds lds = {{ring + kK0, ring + kK0 + kSlotBytes, ring + kK0 + (Sh::kKSlots - 1) * kSlotBytes},
-                   {ring, ring + kSlotBytes}};
   const T* Q = static_cast<const T*>(Qv);
   const T* K = static_cast<const T*>(Kv);
   const T* V = static_cast<const T*>(Vv);
@@ -844,9 +963,13 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = wave_id % Sh::kR, grp = wave_id / Sh::kR;  // row block, key group
   const int r32 = lane & 31;
   const int h = lane >> 5;
+  unsigned char* const ring = rings + grp * kRingBytes;
+  const Lds lds = {{ring + kK0, ring + kK0 + kSlotBytes, ring + kK0 + (Sh::kKSlots - 1) * kSlotBytes},
+                   {ring, ring + kSlotBytes}};
 
   // Heaviest (last) query blocks first: with causal masking block qb needs qb+1 key blocks.
   // Workgroups are dealt to the 8 XCDs (one L2 each) round-robin, so when B*H is a multiple of
@@ -860,33 +983,40 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
   const T* Qh = kDense ? Q + dense_head : Q + bb * qs.b + hh * qs.h;
   const int q_row_bytes = kDense ? kDenseRowBytes : (int)qs.n * 2;
 
-  StepArgs a;
+  StepArgs<Sh> a;
   a.k_row_bytes = kDense ? kDenseRowBytes : (int)ks.n * 2;
   a.v_row_bytes = kDense ? kDenseRowBytes : (int)vs.n * 2;
   a.k_rsrc = head_desc(kDense ? K + dense_head : K + bb * ks.b + hh * ks.h, Nk, a.k_row_bytes);
   a.v_rsrc = head_desc(kDense ? V + dense_head : V + bb * vs.b + hh * vs.h, Nk, a.v_row_bytes);
   a.d_chunks = D >> 3;
-  const int q0 = qb * kBlockRows + wave * kWaveRows;  // first query row of this wave
-  const int qrow = q0 + r32;                          // this lane's query row
+  const int q0 = qb * Sh::kBlockRows + wave * kWaveRows;  // first query row of this wave
+  const int qrow = q0 + r32;                              // this lane's query row
   // Causal visibility is top-left aligned: query i sees keys j <= i (and j < Nk).
-  const int kv_end = causal ? min(Nk, (qb + 1) * kBlockRows) : Nk;
-  a.nT = (kv_end + kTileKeys - 1) / kTileKeys;
-  // 32-key halves computed by this wave: those starting at or below its first row (causal,
-  // q0 is a multiple of 32) and below Nk; unmasked: strictly below its first row (causal) and
+  const int kv_end = causal ? min(Nk, (qb + 1) * Sh::kBlockRows) : Nk;
+  const int nTiles = (kv_end + kTileKeys - 1) / kTileKeys;
+  a.nT = (nTiles + Sh::kS - 1) / Sh::kS;
+  a.nLoad = Sh::kS == 1 ? nTiles : grp < nTiles ? (nTiles - 1 - grp) / Sh::kS + 1 : 0;
+  // 32-key halves computed by this wave's rows: those starting at or below the first row (causal,
+  // q0 is a multiple of 32) and below Nk; unmasked: strictly below the first row (causal) and
   // wholly below Nk.
   const int nHalves = (kv_end + 31) / 32;
-  if (q0 >= Nq) {
-    a.nAct = 0;
-    a.nFull = 0;
-  } else if (causal) {
-    a.nAct = min(nHalves, q0 / 32 + 1);
-    a.nFull = min(q0 / 32, Nk / 32);
-  } else {
-    a.nAct = nHalves;
-    a.nFull = Nk / 32;
+  int nAct = 0, nFull = 0;
+  if (q0 < Nq) {
+    nAct = causal ? min(nHalves, q0 / 32 + 1) : nHalves;
+    nFull = causal ? min(q0 / 32, Nk / 32) : Nk / 32;
   }
-  a.nFull = min(a.nFull, a.nAct);
+  nFull = min(nFull, nAct);
+  // Both are prefixes of the sequence's halves; the group's share is a prefix of the group's: two
+  // for each of its tiles wholly inside, one for a tile half inside.
+  auto share = [grp](int n) {
+    if (Sh::kS == 1) return n;
+    const int t = n >> 1;
+    return (grp < t ? 2 * ((t - 1 - grp) / Sh::kS + 1) : 0) + ((n & 1) && t % Sh::kS == grp ? 1 : 0);
+  };
+  a.nAct = share(nAct);
+  a.nFull = share(nFull);
   a.wave = wave;
+  a.grp = grp;
   a.lane = lane;
   a.h = h;
   a.last_key = causal ? min(qrow, Nk - 1) : Nk - 1;
@@ -903,21 +1033,22 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
     // A wave past the last query row (q0 >= Nq) computes nothing; its stage reads row Nq - 1.
     const i32x4 qd = head_desc(Qh, Nq, q_row_bytes);
     issue_q_stage<Sh>(tile_desc(qd, min(q0, Nq - 1), q_row_bytes), q_row_bytes, qstage,
-                      a.d_chunks);
+                      a.d_chunks, grp);
   } else {
     const __amdgpu_buffer_rsrc_t qr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<T*>(Qh), (short)0, Nq * q_row_bytes, 0x00020000);
 #pragma unroll
-    for (int c = 0; c < 4 * Sh::kDH; ++c) {
+    for (int c = 0; c < Sh::kQC; ++c) {
       int off = qrow * q_row_bytes + 32 * c + 16 * h;  // dims 16c + 8h .. +7
       if (Sh::kMaskD) off = 2 * c + h < a.d_chunks ? off : kOutOfRange;
       w.qop[c] = __builtin_bit_cast(v8, __builtin_amdgcn_raw_buffer_load_b128(qr, off, 0, 0));
     }
   }
   tile_offsets<Sh>(a.k_lane, a.v_lane, a.k_row_bytes, a.v_row_bytes, wave, lane, a.d_chunks);
-  issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[0], 0, wave, a.k_lane);
-  if (a.nT > 1) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[1], kTileKeys, wave, a.k_lane);
-  issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[0], 0, wave, a.v_lane);
+  const bool any = Sh::kS == 1 || a.nLoad > 0;  // a late group of a short sequence has no tile
+  if (any) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[0], a.tile_key(0), wave, a.k_lane);
+  if (a.nLoad > 1) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[1], a.tile_key(1), wave, a.k_lane);
+  if (any) issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[0], a.tile_key(0), wave, a.v_lane);
   // The LSE pointer is not among the preloaded arguments: load it while the tiles are in flight.
   if constexpr (Sh::kLse) asm volatile("" ::"s"(LSE));
 
@@ -940,7 +1071,7 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
       }
   }
 #pragma unroll
-  for (int i = 0; i < 2 * Sh::kDH; ++i)
+  for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
   w.m_run = -INFINITY;
@@ -954,13 +1085,15 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
   if constexpr (Sh::kQStage) {
     // Q and K_0 have landed once K_1 and V_0 (issued after them) are all that may be in flight;
     // tile step 0 waits for those.  The barrier makes every wave's share of K_0 visible.
-    if (a.nT > 1)
+    if (a.nLoad > 1)
       wait_vmcnt<Sh::kLoadsPerWave>();
-    else
+    else if (any)
       wait_vmcnt<Sh::kLoadsPerWave / 2>();
+    else
+      wait_vmcnt<0>();
     lds_barrier();
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int c = 0; c < Sh::kQC; ++c)
       w.qop[c] = *reinterpret_cast<const v8*>(qstage + r32 * kKRowBytes +
                                               (((2 * c + h) ^ swz_k(r32)) << 4));
   } else {
@@ -969,7 +1102,7 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
     // V_0 (once, in the prologue), and leaves no compiler-tracked loads whose waits could land
     // inside the loop and drain the transfers in flight there.
 #pragma unroll
-    for (int c = 0; c < 4 * Sh::kDH; ++c) asm volatile("" ::"v"(w.qop[c]));
+    for (int c = 0; c < Sh::kQC; ++c) asm volatile("" ::"v"(w.qop[c]));
     wait_vmcnt<0>();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     lds_barrier();
@@ -998,6 +1131,29 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
       pv_half<Sh, 1, 1>(w, lds);
   }
 
+  T* ohead = kDense ? O + dense_head : O + bb * os.b + hh * os.h;
+  const long long o_rs = kDense ? (long long)Sh::kD : os.n;
+  if constexpr (Sh::kS > 1) {
+    // The groups' states merge through LDS, over the rings: past this barrier every wave's K/V reads
+    // are complete and every transfer was waited for.
+    typedef Partial<Sh> P;
+    static_assert(Sh::kWaves * P::kBytes <= (int)sizeof(rings), "the O partials fit in the rings");
+    static_assert(Sh::kBlockRows * P::kC8 % (64 * Sh::kWaves) == 0, "whole passes");
+    __shared__ PartialStats stats[Sh::kWaves];
+    lds_write_barrier();
+    publish_partial(w, rings + wave_id * P::kBytes, &stats[wave_id]);
+    lds_write_barrier();
+#pragma unroll
+    for (int pass = 0; pass < Sh::kBlockRows * P::kC8 / (64 * Sh::kWaves); ++pass) {
+      const int item = 64 * Sh::kWaves * pass + threadIdx.x;
+      const int R = item / P::kC8 % kWaveRows, rw = item / (P::kC8 * kWaveRows), c8 = item % P::kC8;
+      merge_item<Sh, Sh::kS>(rings + rw * P::kBytes, Sh::kR * P::kBytes, &stats[rw], Sh::kR, R, c8,
+                             qb * Sh::kBlockRows + rw * kWaveRows + R, Nq, a.d_chunks, ohead, o_rs,
+                             LSE != nullptr ? LSE + (size_t)bh * Nq : nullptr);
+    }
+    return;
+  }
+
   // Row sums over the lane pair (both lanes of a row hold the same offset).
   const float l_o = pair_sum(w.l_p);
   const float l_all = Sh::kLse ? pair_sum(w.l_run) : 0.f;
@@ -1014,11 +1170,9 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
     ostage = qstage;
   } else {
     lds_barrier();
-    ostage = ring + wave * (kWaveRows * Sh::kD * 2);
+    ostage = ring + wave * (kWaveRows * kKRowBytes * Sh::kDH);
   }
-  T* ohead = kDense ? O + dense_head : O + bb * os.b + hh * os.h;
-  store_o<Sh>(w, ostage, 1.0f / l_o, lane_e, ohead, kDense ? (long long)Sh::kD : os.n, q0, Nq,
-              a.d_chunks);
+  store_o<Sh>(w, ostage, 1.0f / l_o, lane_e, ohead, o_rs, q0, Nq, a.d_chunks);
   if (Sh::kLse && LSE != nullptr && h_e == 0 && qrow_e < Nq)
     LSE[(size_t)bh * Nq + qrow_e] = (w.m_run + __builtin_amdgcn_logf(l_all)) * kLn2;
 }
@@ -1031,11 +1185,7 @@ __global__ __launch_bounds__(kThreads, Sh::kDH == 1 ? 3 : 2) void fwd_kernel(
 // Then each workgroup takes one 32-row query block, and its 4 waves split the block's 32-key
 // halves (wave w: halves w, w + 4, w + 8, ...): every wave runs its own online softmax over the
 // same 32 rows, with its own 2-slot ring of K and V halves in LDS, so no wave waits for another
-// until the merge.  The merge goes through LDS with the log-sum-exp rule over the 4 partial
-// states (offset m_w, rounded-probability sum lp_w, fp32 sum l_w, unnormalised O_w):
-//   M = max_w m_w,  a_w = 2^(m_w - M),  O = sum_w a_w O_w / sum_w a_w lp_w,
-//   LSE = (M + log2 sum_w a_w l_w) ln 2.
-// A wave with no half contributes m_w = -inf (a_w = 0).  The half-step is the tail path of
+// until the merge of the 4 partial states.  The half-step is the tail path of
 // fwd_kernel (qk_half, mask_half, move_offset, exp_half, pv_half), unpipelined: at this size
 // the time is latency, and each wave has at most ceil(nH / 4) halves.  A wave with exactly two
 // (both loaded by the prologue) computes them together (split_pair): at B1 H12 N256 that took
@@ -1050,9 +1200,7 @@ struct SplitLayout {
   static constexpr int kSlotBytes = 2 * Sh::kDH * kHalfBytes;  // a K half, then a V half
   static constexpr int kWaveBytes = 2 * kSlotBytes;             // the wave's 2-slot ring
   static constexpr int kRingBytes = kWaves * kWaveBytes;
-  static constexpr int kQBytes = kWaveRows * Sh::kD * 2;        // the block's 32 Q rows
-  static constexpr int kOPartBytes = kWaveRows * Sh::kD * 4;    // one wave's O partial, fp32
-  static_assert(kWaves * kOPartBytes <= kRingBytes, "the O partials fit in the rings");
+  static constexpr int kQBytes = Sh::kDH * kHalfBytes;          // the block's 32 Q rows
   static constexpr int kLoadsPerHalf = 8 * Sh::kDH;             // 1-KiB transfers, K and V
   static constexpr int kRowsPerWave = kWaveRows / kWaves;       // rows each wave merges
 };
@@ -1072,7 +1220,7 @@ __device__ __forceinline__ void issue_rows8(i32x4 desc, int row_bytes, unsigned 
 
 // Half u of K and V (32 rows each, every dim half) into ring slot `slot` of this wave.
 template <class Sh>
-__device__ __forceinline__ void issue_split_half(const StepArgs& a, unsigned char* slot, int u) {
+__device__ __forceinline__ void issue_split_half(const StepArgs<Sh>& a, unsigned char* slot, int u) {
   const i32x4 kd = tile_desc(a.k_rsrc, 32 * u, a.k_row_bytes);
   const i32x4 vd = tile_desc(a.v_rsrc, 32 * u, a.v_row_bytes);
   unsigned char* vslot = slot + Sh::kDH * kHalfBytes;
@@ -1088,7 +1236,7 @@ __device__ __forceinline__ void issue_split_half(const StepArgs& a, unsigned cha
 // One half u from ring slot kSlot: S, mask (diagonal or last partial half), offset check, P and
 // its sums, O += V P.
 template <class Sh, int kSlot>
-__device__ __forceinline__ void split_half(WaveState<Sh>& w, const Lds& lds, int u, const StepArgs& a) {
+__device__ __forceinline__ void split_half(WaveState<Sh>& w, const Lds& lds, int u, const StepArgs<Sh>& a) {
   w.s = qk_half<Sh, kSlot, 0, kHalfBytes>(w, lds);
   if (u >= a.nFull) mask_half(w, a.last_key - u * 32 - 4 * a.h);
   move_offset(w, lane_max(w), a.scale_log2, a.inv_scale_log2);
@@ -1102,7 +1250,7 @@ __device__ __forceinline__ void split_half(WaveState<Sh>& w, const Lds& lds, int
 // runs, this is a shorter dependency chain than two split_half calls.
 template <class Sh>
 __device__ __forceinline__ void split_pair(WaveState<Sh>& w, const Lds& lds, int u0, int u1,
-                                           const StepArgs& a) {
+                                           const StepArgs<Sh>& a) {
   const f32x16 s0 = qk_half<Sh, 0, 0, kHalfBytes>(w, lds);
   w.s = qk_half<Sh, 1, 0, kHalfBytes>(w, lds);
   if (u1 >= a.nFull) mask_half(w, a.last_key - u1 * 32 - 4 * a.h);
@@ -1129,11 +1277,9 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   typedef typename Sh::T T;
   typedef typename Elem<T>::v8 v8;
   typedef SplitLayout<Sh> L;
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __shared__ __attribute__((aligned(1024))) unsigned char ring[L::kRingBytes];
   __shared__ __attribute__((aligned(1024))) unsigned char qst[L::kQBytes];
-  __shared__ float stats[L::kWaves][3][kWaveRows];  // m, lp, l per wave and row
+  __shared__ PartialStats stats[L::kWaves];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1153,7 +1299,7 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   const int q0 = rb * kWaveRows;
   const int qrow = q0 + r32;
 
-  StepArgs a;
+  StepArgs<Sh> a;
   a.k_row_bytes = kDense ? Sh::kD * 2 : (int)ks.n * 2;
   a.v_row_bytes = kDense ? Sh::kD * 2 : (int)vs.n * 2;
   a.k_rsrc = head_desc(K, Nk, a.k_row_bytes);
@@ -1165,8 +1311,9 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   const int nH = (kv_end + 31) / 32;
   a.nFull = causal ? min(q0 / 32, Nk / 32) : Nk / 32;
   a.nAct = wave < nH ? (nH - 1 - wave) / L::kWaves + 1 : 0;  // this wave's halves
-  a.nT = 0;
+  a.nT = a.nLoad = 0;
   a.wave = wave;
+  a.grp = 0;
   a.lane = lane;
   a.h = h;
   a.last_key = causal ? min(qrow, Nk - 1) : Nk - 1;
@@ -1205,7 +1352,7 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
       }
   }
 #pragma unroll
-  for (int i = 0; i < 2 * Sh::kDH; ++i)
+  for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
   w.m_run = -INFINITY;
@@ -1223,11 +1370,9 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
     wait_vmcnt<0>();
   lds_barrier();
 #pragma unroll
-  for (int dh = 0; dh < Sh::kDH; ++dh)
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      w.qop[4 * dh + c] = *reinterpret_cast<const v8*>(qst + dh * kHalfBytes + r32 * kKRowBytes +
-                                                        (((2 * c + h) ^ swz_k(r32)) << 4));
+  for (int i = 0; i < Sh::kQC; ++i)
+    w.qop[i] = *reinterpret_cast<const v8*>(qst + (i >> 2) * kHalfBytes + r32 * kKRowBytes +
+                                            (((2 * (i & 3) + h) ^ swz_k(r32)) << 4));
 
   if (a.nAct == 2) {
     // Both halves were issued by the prologue.
@@ -1252,82 +1397,24 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   }
   }
 
-  // Merge.  Each wave publishes its row statistics and its unnormalised O rows (fp32, row-major,
-  // 16-B chunk c of row r at physical chunk c ^ (r % (kD/4))) over its own ring, which only it
-  // used: its transfers were all waited for, and its LDS accesses complete in order, so its K/V
-  // reads come before these writes.  One barrier then publishes every wave's rows.
-  const float lp = pair_sum(w.l_p);
-  const float lr = Sh::kLse ? pair_sum(w.l_run) : 0.f;
-  int lane_e;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
-  const int r_e = lane_e & 31, h_e = lane_e >> 5;
-  constexpr int kC4 = Sh::kD / 4;   // 16-B fp32 chunks per O row
-  constexpr int kRowB = Sh::kD * 4;
-  static_assert(L::kOPartBytes <= L::kWaveBytes, "a wave's O partial fits in its ring");
-  unsigned char* opart = wring;
-#pragma unroll
-  for (int i = 0; i < 2 * Sh::kDH; ++i)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      // Register 4g + e of tile i holds dim 32i + 8g + 4h + e: fp32 chunk 8i + 2g + h.
-      const f32x4 x = {w.o[i][4 * g], w.o[i][4 * g + 1], w.o[i][4 * g + 2], w.o[i][4 * g + 3]};
-      const int c = 8 * i + 2 * g + h_e;
-      *reinterpret_cast<f32x4*>(opart + r_e * kRowB + ((c ^ (r_e % kC4)) << 4)) = x;
-    }
-  if (h_e == 0) {
-    stats[wave][0][r_e] = w.m_run;
-    stats[wave][1][r_e] = lp;
-    stats[wave][2][r_e] = lr;
-  }
+  // Merge.  Each wave publishes its partial over its own ring, which only it used: its transfers
+  // were all waited for, and its LDS accesses complete in order, so its K/V reads come before these
+  // writes.  One barrier then publishes every wave's rows.
+  typedef Partial<Sh> P;
+  static_assert(P::kBytes <= L::kWaveBytes, "a wave's O partial fits in its ring");
+  publish_partial(w, wring, &stats[wave]);
   lds_write_barrier();
-  // Wave w combines rows w * kRowsPerWave .. +kRowsPerWave - 1: item -> (row, 8 head dims),
-  // kD/8 items per row, so each lane stores 16 B and kD/8 lanes a whole row (non-temporal, as
-  // in store_o).
-  constexpr int kC8 = Sh::kD / 8;
-  constexpr int kItems = L::kRowsPerWave * kC8;
+  // Wave w combines rows w * kRowsPerWave .. +kRowsPerWave - 1: item -> (row, 8 head dims).
+  constexpr int kItems = L::kRowsPerWave * P::kC8;
+  static_assert(kItems % 64 == 0, "whole passes");
   T* O = static_cast<T*>(Ov) + (kDense ? dense_head : bb * os.b + hh * os.h);
-  const long long o_rs = kDense ? (long long)Sh::kD : os.n;
 #pragma unroll
-  for (int pass = 0; pass < (kItems + 63) / 64; ++pass) {
-    const int item = 64 * pass + lane_e;
-    if (kItems % 64 != 0 && item >= kItems) break;
-    const int R = L::kRowsPerWave * wave + item / kC8, c8 = item % kC8;
-    float M = -INFINITY;
-#pragma unroll
-    for (int v = 0; v < L::kWaves; ++v) M = fmaxf(M, stats[v][0][R]);
-    float lsum = 0.f, lrun = 0.f;
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int v = 0; v < L::kWaves; ++v) {
-      const float av = __builtin_amdgcn_exp2f(stats[v][0][R] - M);
-      lsum = fmaf(av, stats[v][1][R], lsum);
-      if constexpr (Sh::kLse) lrun = fmaf(av, stats[v][2][R], lrun);
-      const unsigned char* src = ring + v * L::kWaveBytes + R * kRowB;
-      const f32x4 x0 = *reinterpret_cast<const f32x4*>(src + (((2 * c8) ^ (R % kC4)) << 4));
-      const f32x4 x1 = *reinterpret_cast<const f32x4*>(src + (((2 * c8 + 1) ^ (R % kC4)) << 4));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc0[e] = fmaf(av, x0[e], acc0[e]);
-        acc1[e] = fmaf(av, x1[e], acc1[e]);
-      }
-    }
-    const float inv = 1.0f / lsum;
-    typename Elem<T>::v8 ov;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      ov[e] = (T)(acc0[e] * inv);
-      ov[4 + e] = (T)(acc1[e] * inv);
-    }
-    const int qr = q0 + R;
-    if (qr < Nq && (!Sh::kMaskD || c8 < a.d_chunks)) {
-      u32x4* dst = reinterpret_cast<u32x4*>(O + (long long)qr * o_rs + 8 * c8);
-      if constexpr (Sh::kMaskD)
-        *dst = __builtin_bit_cast(u32x4, ov);
-      else
-        __builtin_nontemporal_store(__builtin_bit_cast(u32x4, ov), dst);
-    }
-    if (Sh::kLse && LSE != nullptr && c8 == 0 && qr < Nq)
-      LSE[(size_t)bh * Nq + qr] = (M + __builtin_amdgcn_logf(lrun)) * kLn2;
+  for (int pass = 0; pass < kItems / 64; ++pass) {
+    const int item = 64 * pass + (threadIdx.x & 63);
+    const int R = L::kRowsPerWave * wave + item / P::kC8, c8 = item % P::kC8;
+    merge_item<Sh, L::kWaves>(ring, L::kWaveBytes, stats, 1, R, c8, q0 + R, Nq, a.d_chunks, O,
+                              kDense ? (long long)Sh::kD : os.n,
+                              LSE != nullptr ? LSE + (size_t)bh * Nq : nullptr);
   }
 }
 
@@ -1427,19 +1514,68 @@ static int validate(const void* q, const void* k, const void* v, const void* o, 
   return TFGFA_OK;
 }
 
-// fwd_kernel's grid of 128-row query blocks is at most one workgroup per CU: the split-key
-// kernel runs the launch instead (a 4x larger grid, a longest wave chain about 4x shorter).
-// Measured crossover (bf16, head dims 64 and 128): faster at every grid up to the CU count
-// (B1 H12 N256 6.66 -> 5.07 us, B1 H16 N1024 15.9 -> 10.1 us, B1 H16 N2048 27.9 -> 24.6 us),
-// slower from twice that (B2 H32 N1024 17.5 -> 27.9 us).  The choice depends on the sizes only,
-// never on strides or outputs, so every instance of one problem takes the same arithmetic.
-static bool use_split_grid(long long blocks, int cu_count) { return blocks <= cu_count; }
+// Which kernel runs a problem.  A grid that leaves CUs idle, or fills them once, takes as long as
+// its longest wave's chain of half-steps (N/32 of them, ~0.4 us each whatever runs beside them);
+// splitting the keys over several waves shortens the chain, at the price of a merge and, where
+// fewer than 4 waves share a K/V tile, of more traffic from the L2.
+//   kWhole    fwd_kernel, 4 row waves, one group: the most work per byte, three workgroups a CU
+//   kGroups2  4 row waves x 2 key groups (128 rows, 8 waves)
+//   kPairs    2 row waves x 2 key groups (64 rows, 4 waves)
+//   kGroups4  2 row waves x 4 key groups (64 rows, 8 waves), head dims up to 64
+//   kHalves   fwd_split_kernel: one 32-row block, 4 waves
+// The lines below are where the measured times cross on 256 CUs (bf16, us, graph replays; N x N
+// causal unless marked; "blocks" are 128-row query blocks, h the longest chain):
+//   D = 64                       blocks   h   kWhole kHalves kGroups2 kPairs kGroups4
+//     B1 H12 N512                   48   16     9.1    6.0      8.6     7.0     6.7
+//     B1 H16 N1024                 128   32    14.5    9.3     12.5    10.0     9.4
+//     B1 H8 N2048                  128   64    25.3   15.7     20.4    16.1    14.1
+//     B1 H12 N2048                 192   64    25.9   19.2     20.9    17.1    16.2
+//     B2 H16 N777                  224   25    12.0   10.9     10.8     8.8    11.6
+//     B1 H16 N2048                 256   64    25.9   23.8     21.4    18.0    18.5
+//     B8 H16 N200                  256    7     6.4    7.3      6.8     6.0     9.3
+//     B2 H16 1000 x 1333 unmasked  256   42    19.2   27.8     17.2    18.2    22.2
+//     B4 H16 500 x 300 unmasked    256   10     7.7   11.9      8.2     8.2    12.2
+//     B3 H12 N1024                 288   32    16.1   17.3     13.7    13.1    17.9
+//     B4 H20 N512                  320   16    10.3   12.9     11.8    11.5    15.0
+//     B2 H25 N1024                 400   32    16.9   23.1     18.2    20.0    25.9
+//     B1 H25 N2048                 400   64    29.0   42.8     25.6    30.1    36.3
+//     B1 H16 N4096                 512  128    52.7   70.2     45.9    48.5    55.4
+//     B1 H16 N8192                1024  256   148.0  251.6    158.2   161.6   185.6
+//   D = 128 (80 where marked)
+//     B1 H16 N300                   48   10     9.6    7.8     10.8     8.8
+//     B1 H12 N1024                  96   32    21.2   16.3     20.0    16.7
+//     B2 H16 300 x 700 unmasked     96   22    15.8   22.8     16.2    13.6
+//     B1 H25 N600                  125   19    15.4   17.0     14.6    14.1
+//     B1 H12 N2048                 192   64    36.2   45.2     31.9    27.0
+//     B1 H25 N1024                 200   32    22.5   36.1     21.7    23.5
+//     B2 H16 1000 x 1333 unm., 80  256   42    23.7   59.1     22.8    33.6
+//     B4 H16 N500                  256   16    14.7   24.0     15.0    17.8
+//     B1 H12 N3000, 80             288   94    45.4   72.4     38.2    46.7
+//     B2 H25 N1024                 400   32    26.9   68.8     29.9    45.4
+//     B1 H16 N4096                 512  128    85.9  186.2     76.3   105.6
+// The choice depends on the sizes only, never on strides or outputs, so every instance of one
+// problem takes the same arithmetic.
+enum class Plan { kWhole, kHalves, kGroups2, kPairs, kGroups4 };
+static Plan choose_plan(long long blocks, int cu_count, int Nq, int Nk, int D, int causal) {
+  const int h = ((causal ? std::min(Nq, Nk) : Nk) + 31) / 32;
+  const long long cu = cu_count;
+  if (causal && blocks > cu && blocks <= 2 * cu && h >= 64) return Plan::kGroups2;
+  if (D <= kDHalf) {
+    if (2 * blocks <= cu) return h > 32 ? Plan::kGroups4 : Plan::kHalves;
+    if (!causal) return blocks <= cu && h >= 32 ? Plan::kGroups2 : Plan::kWhole;
+    if (blocks <= cu) return h >= 64 && 4 * blocks <= 3 * cu ? Plan::kGroups4 : Plan::kPairs;
+    return 4 * blocks <= 5 * cu && h >= 22 ? Plan::kPairs : Plan::kWhole;
+  }
+  if (4 * blocks <= cu || (causal && 8 * blocks <= 3 * cu && h >= 24)) return Plan::kHalves;
+  if (4 * blocks <= 3 * cu) return Plan::kPairs;
+  return blocks <= cu && h >= 22 ? Plan::kGroups2 : Plan::kWhole;
+}
 
 struct LaunchArgs {
   const void *q, *k, *v;
   void* o;
   float* lse;
-  int H, BH, Nq, Nk, D, nQB;
+  int H, BH, Nq, Nk, D;
   float scale_log2;
   int causal;
   Strides qs, ks, vs, os;
@@ -1447,8 +1583,9 @@ struct LaunchArgs {
 
 template <class Sh, bool kDense>
 static void launch_instance(const LaunchArgs& a, hipStream_t stream) {
-  hipLaunchKernelGGL((fwd_kernel<Sh, kDense>), dim3(a.BH * a.nQB), dim3(kThreads), 0, stream, a.q,
-                     a.k, a.v, a.o, a.BH, a.Nq, a.Nk, a.nQB, a.causal, a.scale_log2, a.lse, a.H,
+  const int nQB = (a.Nq + Sh::kBlockRows - 1) / Sh::kBlockRows;
+  hipLaunchKernelGGL((fwd_kernel<Sh, kDense>), dim3(a.BH * nQB), dim3(64 * Sh::kWaves), 0, stream, a.q,
+                     a.k, a.v, a.o, a.BH, a.Nq, a.Nk, nQB, a.causal, a.scale_log2, a.lse, a.H,
                      a.D, a.qs, a.ks, a.vs, a.os);
 }
 
@@ -1461,44 +1598,63 @@ static void launch_split_instance(const LaunchArgs& a, hipStream_t stream) {
                      a.os);
 }
 
-template <int kD, typename T>
-static void launch_dims(const LaunchArgs& a, bool dense, bool split, hipStream_t stream) {
-  if (split) {
-    if constexpr (kD == 64 && std::is_same<T, __bf16>::value) {
-      if (dense && a.D == kD) {  // the reference's layout: no stride arguments to load
-        if (a.lse != nullptr)
-          launch_split_instance<Shape<kD, T, false>, true>(a, stream);
-        else
-          launch_split_instance<Shape<kD, T, false, false>, true>(a, stream);
-        return;
-      }
-    }
-    if (a.D != kD)
-      launch_split_instance<Shape<kD, T, true>>(a, stream);
-    else if (a.lse != nullptr)
-      launch_split_instance<Shape<kD, T, false>>(a, stream);
-    else
-      launch_split_instance<Shape<kD, T, false, false>>(a, stream);
-    return;
+// Launches the plan's kernel for one head-dim instance, with or without the LSE.
+template <int kD, typename T, bool kMaskD, bool kLse, bool kDense>
+static void launch_plan(const LaunchArgs& a, Plan plan, hipStream_t stream) {
+  switch (plan) {
+    case Plan::kHalves:
+      launch_split_instance<Shape<kD, T, kMaskD, kLse>, kDense>(a, stream);
+      break;
+    case Plan::kGroups2:
+      launch_instance<Shape<kD, T, kMaskD, kLse, 4, 2>, kDense>(a, stream);
+      break;
+    case Plan::kPairs:
+      launch_instance<Shape<kD, T, kMaskD, kLse, 2, 2>, kDense>(a, stream);
+      break;
+    case Plan::kGroups4:
+      if constexpr (kD <= kDHalf) launch_instance<Shape<kD, T, kMaskD, kLse, 2, 4>, kDense>(a, stream);
+      break;
+    case Plan::kWhole:
+      launch_instance<Shape<kD, T, kMaskD, kLse>, kDense>(a, stream);
+      break;
   }
-  if (a.D != kD) {
-    launch_instance<Shape<kD, T, true>, false>(a, stream);
-    return;
-  }
-  if constexpr (kD == 64 && std::is_same<T, __bf16>::value) {
-    if (dense) {  // the GPT-2 layout
-      if (a.lse != nullptr)
-        launch_instance<Shape<kD, T, false>, true>(a, stream);
-      else
-        launch_instance<Shape<kD, T, false, false>, true>(a, stream);
-      return;
-    }
-  }
-  if (a.lse != nullptr)
-    launch_instance<Shape<kD, T, false>, false>(a, stream);
-  else
-    launch_instance<Shape<kD, T, false, false>, false>(a, stream);
 }
+
+template <int kD, typename T, bool kMaskD, bool kDense = false>
+static void launch_lse(const LaunchArgs& a, Plan plan, hipStream_t stream) {
+  if (a.lse != nullptr)
+    launch_plan<kD, T, kMaskD, true, kDense>(a, plan, stream);
+  else
+    launch_plan<kD, T, kMaskD, false, kDense>(a, plan, stream);
+}
+
+// The narrowest compiled head dims that hold D: the MFMAs and LDS reads of dims past them fall away
+// (D = 80 on the 96 instance: 24 MFMAs per tile half pair instead of 32).
+template <typename T>
+void launch_dims(const LaunchArgs& a, bool dense, Plan plan, hipStream_t stream) {
+  if (a.D <= 32)
+    launch_lse<32, T, true>(a, plan, stream);
+  else if (a.D < 64)
+    launch_lse<64, T, true>(a, plan, stream);
+  else if (a.D == 64 && dense && std::is_same<T, __bf16>::value)  // the GPT-2 layout: no strides to load
+    launch_lse<64, T, false, true>(a, plan, stream);
+  else if (a.D == 64)
+    launch_lse<64, T, false>(a, plan, stream);
+  else if (a.D <= 96)
+    launch_lse<96, T, true>(a, plan, stream);
+  else if (a.D < 128)
+    launch_lse<128, T, true>(a, plan, stream);
+  else
+    launch_lse<128, T, false>(a, plan, stream);
+}
+
+// The fp16 instances are compiled by tfgfa_fwd_f16.hip, which includes this file: the two element
+// types then compile in parallel.
+#ifdef TFGFA_FWD_F16_UNIT
+template void launch_dims<_Float16>(const LaunchArgs&, bool, Plan, hipStream_t);
+}  // namespace tfgfa
+#else
+extern template void launch_dims<_Float16>(const LaunchArgs&, bool, Plan, hipStream_t);
 
 static int launch(const void* q, const void* k, const void* v, void* o, float* lse, int B, int H,
                   int Nq, int Nk, int D, int dtype, float softmax_scale, int causal,
@@ -1518,7 +1674,6 @@ static int launch(const void* q, const void* k, const void* v, void* o, float* l
   a.Nq = Nq;
   a.Nk = Nk;
   a.D = D;
-  a.nQB = (Nq + kBlockRows - 1) / kBlockRows;
   a.scale_log2 = softmax_scale * kLog2e;
   a.causal = causal;
   a.qs = operand_strides(st[0], B, H, Nq, D);
@@ -1533,19 +1688,13 @@ static int launch(const void* q, const void* k, const void* v, void* o, float* l
   int cu_count = 0;
   const int ist = tfgfa_device_info(&cu_count, nullptr, nullptr, 0);
   if (ist != TFGFA_OK) return ist;
-  const bool split = use_split_grid((long long)a.BH * a.nQB, cu_count);
+  const long long blocks = (long long)a.BH * ((Nq + kBlockRows - 1) / kBlockRows);
+  const Plan plan = choose_plan(blocks, cu_count, Nq, Nk, D, causal);
   const hipStream_t stream = (hipStream_t)hip_stream;
-  if (dtype == TFGFA_DTYPE_BF16) {
-    if (D <= 64)
-      launch_dims<64, __bf16>(a, dense, split, stream);
-    else
-      launch_dims<128, __bf16>(a, dense, split, stream);
-  } else {
-    if (D <= 64)
-      launch_dims<64, _Float16>(a, dense, split, stream);
-    else
-      launch_dims<128, _Float16>(a, dense, split, stream);
-  }
+  if (dtype == TFGFA_DTYPE_BF16)
+    launch_dims<__bf16>(a, dense, plan, stream);
+  else
+    launch_dims<_Float16>(a, dense, plan, stream);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? TFGFA_OK : -(int)e;
 }
@@ -1633,3 +1782,4 @@ extern "C" int tfgfa_device_info(int* cu_count, int* sclk_mhz, char* arch, int a
 }
 
 extern "C" int tfgfa_abi_version(void) { return TFGFA_ABI_VERSION; }
+#endif  // TFGFA_FWD_F16_UNIT
