@@ -8,7 +8,7 @@ from __future__ import annotations
 import torch
 from torch.autograd import forward_ad
 
-from . import _C
+from . import _C, _launch_on
 
 MAX_NORM_DIM = _C.GPT2_MAX_NORM_DIM
 MAX_ROWS = _C.GPT2_MAX_ROWS
@@ -47,36 +47,28 @@ def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def layernorm(x, scale, shift, eps: float, dtype=torch.float32, delta=None):
     """LayerNorm over the last dimension, in ``dtype`` (float32 or bfloat16).  With ``delta`` (bf16,
     like x): the norm of x + delta, returned as (x + delta, norm)."""
     d = x.shape[-1]
     y = torch.empty(x.shape, dtype=dtype, device=x.device)
     s = None if delta is None else torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        _C.gpt2_layernorm(x.data_ptr(), _ptr(delta), _ptr(s), scale.data_ptr(), shift.data_ptr(),
-                          y.data_ptr(), dtype == torch.bfloat16, x.numel() // d, d, eps,
-                          _stream(x.device))
+    _launch_on(x.get_device(), _C.gpt2_layernorm, x.data_ptr(), _ptr(delta), _ptr(s), scale.data_ptr(),
+               shift.data_ptr(), y.data_ptr(), dtype == torch.bfloat16, x.numel() // d, d, eps)
     return y if delta is None else (s, y)
 
 
 def gelu(x):
     """0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3)))"""
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        _C.gpt2_gelu(x.data_ptr(), y.data_ptr(), x.numel(), _stream(x.device))
+    _launch_on(x.get_device(), _C.gpt2_gelu, x.data_ptr(), y.data_ptr(), x.numel())
     return y
 
 
 def cast_bf16(pairs) -> None:
     """dst.copy_(src) for each (src float32, dst bf16) pair of equal, multiple-of-4 sizes."""
-    dev = pairs[0][0].device
-    with torch.cuda.device(dev):
-        _C.gpt2_cast_bf16([(s.data_ptr(), d.data_ptr(), s.numel()) for s, d in pairs], _stream(dev))
+    _launch_on(pairs[0][0].get_device(), _C.gpt2_cast_bf16,
+               [(s.data_ptr(), d.data_ptr(), s.numel()) for s, d in pairs])
 
 
 def rows_fit(rows: int, width: int, norm: bool) -> bool:
@@ -93,9 +85,7 @@ def linear_rows(x, parts, dtype, norm=None, gelu=False, residual=None):
     N, K = parts[0][0].shape
     ys = [torch.empty(x.shape[:-1] + (N,), dtype=dtype, device=x.device) for _ in parts]
     scale, shift, eps = norm if norm is not None else (None, None, 0.0)
-    with torch.cuda.device(x.device):
-        _C.gpt2_linear_rows(x.data_ptr(), x.dtype == torch.bfloat16, _ptr(scale), _ptr(shift), eps,
-                            [(w.data_ptr(), _ptr(b), y.data_ptr()) for (w, b), y in zip(parts, ys)],
-                            gelu, _ptr(residual), dtype == torch.bfloat16, x.numel() // K, N, K,
-                            _stream(x.device))
+    _launch_on(x.get_device(), _C.gpt2_linear_rows, x.data_ptr(), x.dtype == torch.bfloat16, _ptr(scale),
+               _ptr(shift), eps, [(w.data_ptr(), _ptr(b), y.data_ptr()) for (w, b), y in zip(parts, ys)],
+               gelu, _ptr(residual), dtype == torch.bfloat16, x.numel() // K, N, K)
     return ys
