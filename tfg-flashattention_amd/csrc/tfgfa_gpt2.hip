@@ -198,30 +198,30 @@ constexpr int kNormPad = 4;                // floats between the normalised rows
 constexpr int kMaxParts = 3;
 constexpr int kNormLdsFloats = 15360;      // M * (K + kNormPad) at most (60 KiB)
 
-struct RowsArgs {
-  const void* x;
-  const float* ln_scale;
-  const float* ln_shift;
-  const float* w[kMaxParts];
+struct RowsOut {
   const float* bias[kMaxParts];
   void* y[kMaxParts];
   const float* residual;
   float eps;
-  int M, N, K, tiles;  // tiles: workgroups per part
 };
 
-// kG: groups of 4 rows of x; kV: 256-element pieces of a normalised row (0: no norm).
+// kG: groups of 4 rows of x; kV: 256-element pieces of a normalised row (0: no norm); tiles:
+// workgroups per part.  The first 14 argument dwords arrive in SGPRs (-amdgpu-kernarg-preload-count):
+// what the weight and row loads need.  The bias and the residual are loaded beside the weights, not
+// where they are added: a round trip less at the end of a kernel of a few.
 template <int kW, int kStrips, int kG, typename X, typename Y, int kV, bool kGelu>
-__global__ __launch_bounds__(64 * kW) void linear_rows_kernel(RowsArgs a) {
+__global__ __launch_bounds__(64 * kW) void linear_rows_kernel(
+    const void* __restrict__ x, const float* __restrict__ w0, const float* __restrict__ w1,
+    const float* __restrict__ w2, int M, int N, int K, int tiles, const float* __restrict__ ln_scale,
+    const float* __restrict__ ln_shift, RowsOut out) {
   extern __shared__ __attribute__((aligned(16))) float xs[];  // kV: M rows of K + kNormPad floats
   __shared__ float red[kW][kG][4][4];                         // [wave][col group][row][col]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int i = lane & 3, b = lane >> 2;
-  const int part = blockIdx.x / a.tiles;
-  const int n0 = (blockIdx.x - part * a.tiles) * kTileRows;
-  const float* w = part == 0 ? a.w[0] : part == 1 ? a.w[1] : a.w[2];
-  const int K = a.K;
+  const int part = blockIdx.x / tiles;
+  const int n0 = (blockIdx.x - part * tiles) * kTileRows;
+  const float* w = part == 0 ? w0 : part == 1 ? w1 : w2;
   const int nStrips = (K + 63) / 64;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
@@ -229,8 +229,8 @@ __global__ __launch_bounds__(64 * kW) void linear_rows_kernel(RowsArgs a) {
   // (neither's sums are stored).
   int col[kG];
 #pragma unroll
-  for (int g = 0; g < kG; ++g) col[g] = min(4 * g + i, a.M - 1);
-  const float* wrow = w + (long long)min(n0 + i, a.N - 1) * K;
+  for (int g = 0; g < kG; ++g) col[g] = min(4 * g + i, M - 1);
+  const float* wrow = w + (long long)min(n0 + i, N - 1) * K;
   f32x4 wv[kStrips], xv[kV ? 1 : kStrips][kG];
   // The batch of strips s0, s0 + kW, ..
   auto load_batch = [&](int s0) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64 * kW) void linear_rows_kernel(RowsArgs a) {
       wv[u] = load4(wrow + kk);
       if constexpr (kV == 0) {
 #pragma unroll
-        for (int g = 0; g < kG; ++g) xv[u][g] = load4(static_cast<const X*>(a.x) + (long long)col[g] * K + kk);
+        for (int g = 0; g < kG; ++g) xv[u][g] = load4(static_cast<const X*>(x) + (long long)col[g] * K + kk);
       }
     }
   };
@@ -248,33 +248,42 @@ __global__ __launch_bounds__(64 * kW) void linear_rows_kernel(RowsArgs a) {
   if constexpr (kV > 0) {
     // Row m of x by wave m % kW, normalised into LDS.
     f32x4 v[kV], g[kV], h[kV];
-    for (int m = wave; m < a.M; m += kW) {
-      const float* xr = static_cast<const float*>(a.x) + (long long)m * K;
+    for (int m = wave; m < M; m += kW) {
+      const float* xr = static_cast<const float*>(x) + (long long)m * K;
 #pragma unroll
       for (int c = 0; c < kV; ++c) {
         const int k = 4 * (64 * c + lane), kk = k < K ? k : 0;
         v[c] = load4(xr + kk);
-        g[c] = load4(a.ln_scale + kk);
-        h[c] = load4(a.ln_shift + kk);
+        g[c] = load4(ln_scale + kk);
+        h[c] = load4(ln_shift + kk);
       }
       if (m == wave) load_batch(wave);
 #pragma unroll
       for (int c = 0; c < kV; ++c)
         if (4 * (64 * c + lane) >= K) v[c] = zero;
-      normalise_row(v, K, lane, a.eps);
+      normalise_row(v, K, lane, out.eps);
 #pragma unroll
       for (int c = 0; c < kV; ++c) {
         const int k = 4 * (64 * c + lane);
         if (k < K) *reinterpret_cast<f32x4*>(xs + m * (K + kNormPad) + k) = v[c] * g[c] + h[c];
       }
     }
-    if (wave >= a.M) load_batch(wave);
+    if (wave >= M) load_batch(wave);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   } else {
     load_batch(wave);
   }
+
+  // Thread -> (row m of x, output r of the workgroup's four) of the results.
+  const int r = threadIdx.x % kTileRows, m = threadIdx.x / kTileRows, n = n0 + r;
+  const bool writes = m < M && n < N;
+  const float* bias = part == 0 ? out.bias[0] : part == 1 ? out.bias[1] : out.bias[2];
+  const long long at = (long long)m * N + n;
+  float add_bias = 0.f, add_residual = 0.f;
+  if (writes && bias != nullptr) add_bias = bias[n];
+  if (writes && out.residual != nullptr) add_residual = out.residual[at];
 
   f32x4 acc[kG];
 #pragma unroll
@@ -304,25 +313,19 @@ __global__ __launch_bounds__(64 * kW) void linear_rows_kernel(RowsArgs a) {
 #pragma unroll
   for (int g = 0; g < kG; ++g)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float v = block_sum(acc[g][r]);
-      if (lane < 4) red[wave][g][r][lane] = v;
+    for (int c = 0; c < 4; ++c) {
+      const float v = block_sum(acc[g][c]);
+      if (lane < 4) red[wave][g][c][lane] = v;
     }
   __syncthreads();
-  // Thread -> (row m of x, output r of the workgroup's four).
-  const int r = threadIdx.x % kTileRows, m = threadIdx.x / kTileRows;
-  const int n = n0 + r;
-  if (m >= a.M || n >= a.N) return;
+  if (!writes) return;
   float v = 0.f;
 #pragma unroll
   for (int ww = 0; ww < kW; ++ww) v += red[ww][m / 4][r][m % 4];
-  const float* bias = part == 0 ? a.bias[0] : part == 1 ? a.bias[1] : a.bias[2];
-  Y* y = static_cast<Y*>(part == 0 ? a.y[0] : part == 1 ? a.y[1] : a.y[2]);
-  if (bias != nullptr) v += bias[n];
+  v += add_bias;
   if (kGelu) v = gelu(v);
-  const long long at = (long long)m * a.N + n;
-  if (a.residual != nullptr) v += a.residual[at];
-  y[at] = (Y)v;
+  Y* y = static_cast<Y*>(part == 0 ? out.y[0] : part == 1 ? out.y[1] : out.y[2]);
+  y[at] = (Y)(v + add_residual);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -348,11 +351,21 @@ static void launch_norm(const float* x, const __bf16* delta, float* sum, const f
                        scale, shift, y, d, eps);
 }
 
+struct RowsArgs {
+  const void* x;
+  const float* ln_scale;
+  const float* ln_shift;
+  const float* w[kMaxParts];
+  int M, N, K, tiles;
+  RowsOut out;
+};
+
 template <int kW, int kStrips, int kG, typename X, typename Y, int kV, bool kGelu = false>
 static void launch_rows(const RowsArgs& a, int parts, hipStream_t stream) {
   const size_t lds = kV ? (size_t)a.M * (a.K + kNormPad) * sizeof(float) : 0;
   hipLaunchKernelGGL((linear_rows_kernel<kW, kStrips, kG, X, Y, kV, kGelu>),
-                     dim3((unsigned)(a.tiles * parts)), dim3(64 * kW), lds, stream, a);
+                     dim3((unsigned)(a.tiles * parts)), dim3(64 * kW), lds, stream, a.x, a.w[0],
+                     a.w[1], a.w[2], a.M, a.N, a.K, a.tiles, a.ln_scale, a.ln_shift, a.out);
 }
 
 // With the norm: 4 waves (more would idle through the norm of 4 rows), the whole width in one
@@ -487,16 +500,16 @@ extern "C" int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_sca
     if (!w[p] || !y[p]) return TFGFA_ERR_NULL_POINTER;
     if (misaligned(w[p]) || misaligned(bias[p]) || misaligned(y[p])) return TFGFA_ERR_ALIGNMENT;
     a.w[p] = w[p];
-    a.bias[p] = bias[p];
-    a.y[p] = y[p];
+    a.out.bias[p] = bias[p];
+    a.out.y[p] = y[p];
   }
   if (misaligned(x) || misaligned(ln_scale) || misaligned(ln_shift) || misaligned(residual))
     return TFGFA_ERR_ALIGNMENT;
   a.x = x;
   a.ln_scale = ln_scale;
   a.ln_shift = ln_shift;
-  a.residual = residual;
-  a.eps = eps;
+  a.out.residual = residual;
+  a.out.eps = eps;
   a.M = M;
   a.N = N;
   a.K = K;
