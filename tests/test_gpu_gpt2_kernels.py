@@ -264,3 +264,25 @@ def test_modules_keep_gradients_and_transforms():
             out = act(dual)
             assert torch.autograd.forward_ad.unpack_dual(out).tangent is not None
     assert norm(torch.empty(0, 64, device=DEV)).shape == (0, 64)
+
+
+@pytest.mark.parametrize("tokens", [16, 17])
+def test_last_logits_are_the_models_last_position(tokens):
+    """The logits a generation loop samples from, with the head on the last position only past 32
+    rows, against the whole model's (CPU, float32: the same sums in another blocking); a hook on the
+    head sees every position."""
+    cfg = dict(mi.GPT_CONFIG_124M)
+    cfg.update({"emb_dim": 64, "n_layers": 2, "n_heads": 2, "vocab_size": 50, "context_length": 32,
+                "drop_rate": 0.0, "impl_type": "manual"})
+    torch.manual_seed(0)
+    model = mi.GPTModel(cfg).eval()
+    idx = torch.randint(0, 50, (2, tokens))
+    with torch.no_grad():
+        want = model(idx)[:, -1, :]
+        got = mi._last_logits(model, idx)
+        assert got.shape == want.shape and _rel(got, want) <= F32
+        seen = []
+        hook = model.out_head.register_forward_hook(lambda m, i, o: seen.append(o.shape[1]))
+        assert torch.equal(mi._last_logits(model, idx), want)
+        hook.remove()
+    assert seen == [tokens]

@@ -312,7 +312,7 @@ class GraphedDecoder:
     def prefill(self, idx):
         """Eager prefill of the prompt; returns the last position's logits."""
         with torch.no_grad():
-            return self.model(idx, kv_cache=self.cache)[:, -1, :]
+            return _last_logits(self.model, idx, self.cache)
 
     def step(self, tok):
         """Appends ``tok`` ((B, 1) token ids) and returns the next logits (a view of the
@@ -484,8 +484,8 @@ class GPTModel(nn.Module):
         self.final_norm = LayerNorm(cfg)
         self.out_head = nn.Linear(cfg["emb_dim"], cfg["vocab_size"], bias=False)
 
-    def forward(self, in_idx, kv_cache=None):
-        """Logits for ``in_idx``.  With ``kv_cache`` the tokens continue the cached sequence:
+    def _hidden(self, in_idx, kv_cache=None):
+        """The last block's output for ``in_idx`` (forward without final norm and head).  With ``kv_cache`` the tokens continue the cached sequence:
         positions start at the cached length, read from ``kv_cache.seqlens`` on the device (so a
         captured decode step stays correct on replay), and the cache advances by the token
         count."""
@@ -502,8 +502,27 @@ class GPTModel(nn.Module):
             for layer, blk in enumerate(self.trf_blocks):
                 x = blk(x, kv_cache, layer)
             kv_cache.advance(seq_len)
-        x = self.final_norm(x)
-        return self.out_head(x)
+        return x
+
+    def forward(self, in_idx, kv_cache=None):
+        """Logits for ``in_idx``; with ``kv_cache`` the tokens continue the cached sequence
+        (:meth:`_hidden`)."""
+        return self.out_head(self.final_norm(self._hidden(in_idx, kv_cache)))
+
+
+# Up to this many rows the head costs its weights' bytes whatever the rows (50257 x 1024: 32 us at
+# 4 rows); past it, its time grows with them (849 us at 1000 rows).
+_HEAD_ROWS = 32
+
+
+def _last_logits(model, idx, kv_cache=None):
+    """``model(idx, kv_cache)[:, -1, :]``, the logits a generation loop samples from, with the final
+    norm and the head on the last position only where all positions would cost more."""
+    if (idx.numel() > _HEAD_ROWS and _plain(model, GPTModel) and _plain(model.final_norm, LayerNorm)
+            and _plain(model.out_head, nn.Linear) and _no_global_hooks()):
+        x = model._hidden(idx, kv_cache)[:, -1:].contiguous()
+        return model.out_head(model.final_norm(x))[:, -1, :]
+    return (model(idx) if kv_cache is None else model(idx, kv_cache=kv_cache))[:, -1, :]
 
 
 def _next_token(logits, temperature, top_k):
@@ -527,7 +546,7 @@ def generate(model, idx, max_new_tokens, context_size, temperature=1.0, top_k=No
     for _ in range(max_new_tokens):
         idx_cond = idx[:, -context_size:]
         with torch.no_grad():
-            logits = model(idx_cond)[:, -1, :]
+            logits = _last_logits(model, idx_cond)
         idx_next = _next_token(logits, temperature, top_k)
         if idx_next == eos_id:
             break
@@ -550,7 +569,7 @@ def generate_cached(model, idx, max_new_tokens, context_size, temperature=1.0, t
     step_in = idx
     for _ in range(max_new_tokens):
         with torch.no_grad():
-            logits = model(step_in, kv_cache=cache)[:, -1, :]
+            logits = _last_logits(model, step_in, cache)
         idx_next = _next_token(logits, temperature, top_k)
         if idx_next == eos_id:
             break
