@@ -283,6 +283,12 @@ struct Shape {
   // (48 KiB of LDS per workgroup with the rings, three workgroups per CU); head dim 128 loads Q
   // into registers and waits for the whole prologue (its rings take 80 KiB).
   static constexpr bool kQStage = kDH == 1;
+  // The V^T operands of a half-step's first two P.V MFMAs are read before it: by the half-step
+  // before it, or right after the tile's barrier, ahead of the transfers issued there; a wave alone
+  // on its SIMD otherwise waits for the LDS at every half-step.  us: B1 H16 N2048 25.6 -> 24.6
+  // (kWhole) and 17.3 -> 16.9 (kPairs), B2 H25 N1024 16.3 -> 15.9, B1 H16 N8192 146.2 -> 145.3, B8
+  // H25 N1024 unchanged.  Not where the 8 registers would spill (one group past 64 dims).
+  static constexpr bool kEarlyV = kDH == 1 || kS_ > 1;
   // Waves per SIMD that the LDS leaves room for: three or two (head dims past 64) one-group
   // workgroups a CU; two 4-wave workgroups of two groups, or one (past 64); one of 8 waves.
   static constexpr int kSimdWaves = kS_ == 1 ? (kDH == 1 ? 3 : 2) : kWaves == 4 && kDH == 2 ? 1 : 2;
@@ -414,6 +420,7 @@ struct WaveState {
   f32x16 o[Sh::kOT];     // O^T accumulators: o[t] holds d = 32t .. 32t+31
   f32x16 s;              // S^T of the half being softmaxed: register t = key 8(t/4) + 4h + t%4
   v8 pb[2];              // P^T of the previous half, waiting for its P.V
+  v8 vop[2];             // kEarlyV: V^T operands of the next half-step's first two P.V MFMAs
   float m_run;           // exp2 offset (a running max of scale*log2e*s, moved lazily)
   float thr;             // raw score above which the offset has to move: (m_run + margin) / (scale*log2e)
   float l_run;           // this lane's running sum of exp2(scale*log2e*s - m_run) (fp32, for the LSE)
@@ -574,7 +581,7 @@ __device__ __forceinline__ typename Elem<typename Sh::T>::v8 k_operand(const Wav
 // below the number of keys).  So l_p, and with it every P and |O| / max|V|, stays at most 2^64.
 // fp16: the bound is the largest finite float, exceeded exactly when a rounded P is +inf (above
 // fp16's range) or a NaN, so every P that reaches an MFMA is finite.
-template <class Sh, int kVs, int kVh, int kKs, int kKh, bool kPV = true>
+template <class Sh, int kVs, int kVh, int kKs, int kKh, bool kPV = true, bool kNextV = false>
 __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, float scale_log2,
                                            float inv_scale_log2) {
   typedef typename Sh::T T;
@@ -585,8 +592,8 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
   constexpr float kSumBound = Elem<T>::kSumBound;
   v8 vop[2];
   if constexpr (kPV) {
-    vop[0] = v_operand<Sh, kVs, kVh>(w, lds, 0);
-    vop[1] = v_operand<Sh, kVs, kVh>(w, lds, 1);
+    vop[0] = Sh::kEarlyV ? w.vop[0] : v_operand<Sh, kVs, kVh>(w, lds, 0);
+    vop[1] = Sh::kEarlyV ? w.vop[1] : v_operand<Sh, kVs, kVh>(w, lds, 1);
   }
   TFGFA_FENCE();
   const float neg_m = -w.m_run;
@@ -626,7 +633,10 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
 #pragma unroll
   for (int i = 0; i < kQk; ++i) {
     acc = Elem<T>::mfma(kop[i & 1], w.qop[i], acc);
-    if (i + 2 < kQk) kop[i & 1] = k_operand<Sh, kKs, kKh>(w, lds, i + 2);
+    if (i + 2 < kQk)
+      kop[i & 1] = k_operand<Sh, kKs, kKh>(w, lds, i + 2);
+    else if (kNextV && Sh::kEarlyV)
+      w.vop[i + 2 - kQk] = v_operand<Sh, kVs, 1>(w, lds, i + 2 - kQk);
     if (i == 0) {
       convert(p);
       asm volatile("" : "+v"(w.pb[0]), "+v"(w.pb[1]));
@@ -682,14 +692,18 @@ struct StepArgs {
   // This lane's byte offsets within a K / V tile (tile_offsets).
   int k_lane[Sh::kDH][Sh::kRowBlocks], v_lane[Sh::kDH][Sh::kRowBlocks];
   int nT;        // tile steps of the workgroup (its groups' most 64-key tiles)
-  int nLoad;     // tiles this group loads (a prefix of the steps)
+  int nLoad;     // several groups: tiles this group loads (a prefix of the steps)
   int nAct;      // 32-key halves this wave computes (a prefix)
   int nFull;     // halves this wave computes without an element mask (a prefix of the above)
   int wave, grp, lane, h, last_key;  // wave: within the group
   float scale_log2, inv_scale_log2;
 
-  // First key of the group's tile j, and of its half u.
-  __device__ __forceinline__ int tile_key(int j) const { return (j * Sh::kS + grp) * kTileKeys; }
+  // Tiles this group loads (one group: every step's); first key of the group's tile j, and of its
+  // half u.
+  __device__ __forceinline__ int loads() const { return Sh::kS == 1 ? nT : nLoad; }
+  __device__ __forceinline__ int tile_key(int j) const {
+    return Sh::kS == 1 ? j * kTileKeys : (j * Sh::kS + grp) * kTileKeys;
+  }
   __device__ __forceinline__ int half_key(int u) const {
     return Sh::kS == 1 ? u * 32 : tile_key(u >> 1) + (u & 1) * 32;
   }
@@ -708,7 +722,7 @@ __device__ __forceinline__ void half_step(WaveState<Sh>& w, const Lds& lds, int 
   if (!kSteady && u > a.nAct) return;
   if (u >= a.nFull && u < a.nAct) mask_half(w, a.last_key - a.half_key(u) - 4 * a.h);
   if (kSteady) {
-    fused_step<Sh, kVs, kVh, kKs, kKh, kPV>(w, lds, a.scale_log2, a.inv_scale_log2);
+    fused_step<Sh, kVs, kVh, kKs, kKh, kPV, kVh == 0>(w, lds, a.scale_log2, a.inv_scale_log2);
     return;
   }
   if (u > 0) pv_half<Sh, kVs, kVh>(w, lds);
@@ -730,7 +744,7 @@ __device__ __forceinline__ void tile_step(WaveState<Sh>& w, const Lds& lds, int 
   constexpr int kKNext = (kKs + 1) % kKN;
   constexpr int kKNext2 = (kKs + 2) % kKN;  // K_{j-1}'s slot (3 slots), K_j's (2 slots)
   constexpr int kVOther = kVs ^ 1;          // V_{j-1}, then V_{j+1}
-  const bool k2 = j + 2 < a.nLoad, v1 = j + 1 < a.nLoad;
+  const bool k2 = j + 2 < a.loads(), v1 = j + 1 < a.loads();
   if (kKN == 3 && k2)
     issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[kKNext2], a.tile_key(j + 2), a.wave, a.k_lane);
   // Half 2j: P.V of half 2j-1 (V_{j-1}, keys 32..63), S of half 2j+1 (K_j, keys 32..63).
@@ -742,6 +756,10 @@ __device__ __forceinline__ void tile_step(WaveState<Sh>& w, const Lds& lds, int 
   else
     wait_vmcnt<0>();
   lds_barrier();
+  if constexpr (kSteady && Sh::kEarlyV) {
+    w.vop[0] = v_operand<Sh, kVs, 0>(w, lds, 0);
+    w.vop[1] = v_operand<Sh, kVs, 0>(w, lds, 1);
+  }
   if (v1)
     issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[kVOther], a.tile_key(j + 1), a.wave, a.v_lane);
   if (kKN == 2 && k2)
@@ -964,7 +982,8 @@ __global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wave = wave_id % Sh::kR, grp = wave_id / Sh::kR;  // row block, key group
+  const int wave = Sh::kS == 1 ? wave_id : wave_id % Sh::kR;  // row block
+  const int grp = Sh::kS == 1 ? 0 : wave_id / Sh::kR;         // key group
   const int r32 = lane & 31;
   const int h = lane >> 5;
   unsigned char* const ring = rings + grp * kRingBytes;
@@ -1047,7 +1066,7 @@ __global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
   tile_offsets<Sh>(a.k_lane, a.v_lane, a.k_row_bytes, a.v_row_bytes, wave, lane, a.d_chunks);
   const bool any = Sh::kS == 1 || a.nLoad > 0;  // a late group of a short sequence has no tile
   if (any) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[0], a.tile_key(0), wave, a.k_lane);
-  if (a.nLoad > 1) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[1], a.tile_key(1), wave, a.k_lane);
+  if (a.loads() > 1) issue_tile<Sh>(a.k_rsrc, a.k_row_bytes, lds.k[1], a.tile_key(1), wave, a.k_lane);
   if (any) issue_tile<Sh>(a.v_rsrc, a.v_row_bytes, lds.v[0], a.tile_key(0), wave, a.v_lane);
   // The LSE pointer is not among the preloaded arguments: load it while the tiles are in flight.
   if constexpr (Sh::kLse) asm volatile("" ::"s"(LSE));
@@ -1085,7 +1104,7 @@ __global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
   if constexpr (Sh::kQStage) {
     // Q and K_0 have landed once K_1 and V_0 (issued after them) are all that may be in flight;
     // tile step 0 waits for those.  The barrier makes every wave's share of K_0 visible.
-    if (a.nLoad > 1)
+    if (a.loads() > 1)
       wait_vmcnt<Sh::kLoadsPerWave>();
     else if (any)
       wait_vmcnt<Sh::kLoadsPerWave / 2>();
