@@ -25,17 +25,25 @@ extern "C" {
 #define TFGPT2_MAX_NORM_DIM 2048
 #define TFGPT2_MAX_ROWS     8
 #define TFGPT2_MAX_CASTS    10
+/* Most splits of the contraction of tfgpt2_linear_planes. */
+#define TFGPT2_MAX_K_SPLITS 8
+
+/* What a result is written as.  PLANES: (3, rows, width) bf16, three arrays whose values add up to
+ * the float32 result exactly (NaN where it is infinite or NaN). */
+#define TFGPT2_F32    0
+#define TFGPT2_BF16   1
+#define TFGPT2_PLANES 2
 
 /*
  * LayerNorm over rows of width d (a multiple of 4, at most TFGPT2_MAX_NORM_DIM), biased variance:
  *   s = x            (delta == NULL)
  *   s = x + delta    (delta: (rows, d) bf16; s is also written to sum, (rows, d) float32)
  *   y = (s - mean) / sqrt(var + eps) * scale + shift
- * y is (rows, d), float32 (y_bf16 = 0) or bf16 (y_bf16 = 1).  sum may be x itself.
+ * y is (rows, d), as y_kind says.  sum may be x itself.
  * src/py/model_inference.py:96-107 (LayerNorm), :157-160 (the residual add before norm2).
  */
 int tfgpt2_layernorm(const float* x, const void* delta, float* sum, const float* scale,
-                     const float* shift, void* y, int y_bf16, int64_t rows, int d, float eps,
+                     const float* shift, void* y, int y_kind, int64_t rows, int d, float eps,
                      void* hip_stream);
 
 /*
@@ -69,6 +77,23 @@ int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_scale, const f
                        float eps, int parts, const float* const* w, const float* const* bias,
                        int gelu, const float* residual, void* const* y, int y_bf16, int M, int N,
                        int K, void* hip_stream);
+
+/*
+ * A float32 linear layer on the bf16 matrix units:
+ *   y = x w^T + bias (+ residual)          (M, N) float32          gelu_planes = 0
+ *   y = GELU(x w^T + bias) as PLANES       (3, M, N) bf16          gelu_planes = 1 (no residual)
+ *   x  (3, M, K) bf16 PLANES    w  (N, K) float32    bias  (N) or NULL    residual  (M, N) or NULL
+ * Every product is that of the float32 values to 2^-26 of itself, sums are float32: as close to the
+ * exact result as a float32 GEMM.  Where x or w is infinite, or rounds to it as bf16, the result is NaN.
+ * splits: 1..TFGPT2_MAX_K_SPLITS partial sums of the contraction, tfgpt2_linear_planes_splits' choice
+ * for a device of cu_count CUs (0: sizes not taken: N a multiple of 4, K of 32, planes and weights
+ * below 2 GiB).  part: splits * M * N floats (NULL for one split); the partial sums are
+ * added in order, so the result depends on the sizes and `splits` only.
+ */
+int tfgpt2_linear_planes_splits(int M, int N, int K, int cu_count);
+int tfgpt2_linear_planes(const void* x, const float* w, const float* bias, int gelu_planes,
+                         const float* residual, void* y, float* part, int splits, int M, int N,
+                         int K, void* hip_stream);
 
 #ifdef __cplusplus
 }

@@ -60,6 +60,14 @@ def test_kernel_arguments_are_checked_before_any_hip_call():
     with pytest.raises(RuntimeError, match="misaligned"):
         _C.gpt2_cast_bf16([(P, P + 8, 4)], 0)
     _C.gpt2_cast_bf16([], 0)
+    with pytest.raises(RuntimeError, match="shape|size"):
+        _C.gpt2_linear_planes(P, P, 0, False, 0, P, P, 1, 4, 6, 32, 0)                        # N not a multiple of 4
+    with pytest.raises(RuntimeError, match="shape|size"):
+        _C.gpt2_linear_planes(P, P, 0, False, 0, P, P, 1, 4, 8, 48, 0)                        # K not of 32
+    with pytest.raises(RuntimeError, match="shape|size"):
+        _C.gpt2_linear_planes(P, P, 0, False, 0, P, P, 3, 4, 8, 64, 0)                        # more splits than steps
+    with pytest.raises(RuntimeError, match="null"):
+        _C.gpt2_linear_planes(P, P, 0, False, 0, P, 0, 2, 4, 8, 64, 0)                        # splits without part
     part = (P, 0, P)
     with pytest.raises(RuntimeError, match="shape|size"):
         _C.gpt2_linear_rows(P, False, 0, 0, 0.0, [part], False, 0, False, 9, 4, 64, 0)       # too many rows
@@ -149,6 +157,53 @@ def test_linear_rows_matches_float64(M, N, K):
     assert torch.isinf(got[0]).all() and torch.isfinite(got[1:]).all()
 
 
+def _to_planes(x):
+    out = []
+    for _ in range(3):
+        out.append(x.to(torch.bfloat16))
+        x = x - out[-1].float()
+    return torch.stack(out)
+
+
+def _planes64(p):
+    return p.double().sum(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 4, 32), (9, 128, 64), (127, 132, 96), (128, 124, 128), (129, 260, 160),
+                                   (300, 768, 3072), (65, 3072, 768), (613, 1600, 1600)])
+def test_linear_planes_matches_float64(M, N, K):
+    """Rows and outputs at the edges of a 128 tile, contractions of one to many steps, one and several
+    splits, with GELU planes out, with a residual, without a bias; values over eight orders of
+    magnitude.  Planes hold 24 bits: a value comes back exactly.  A product is off by at most 2^-26
+    of itself (the three dropped terms), sums are float32, so F32 holds as for the other linears; it must
+    also be no further from float64 than torch's float32 linear (x 1.25 for the chance of one draw)."""
+    from custom_flash_attn import gpt2
+
+    g = torch.Generator(device=DEV).manual_seed(M * 7 + N * 3 + K)
+    scale, shift = 1 + _randn(g, K) * 0.1, _randn(g, K) * torch.exp(_randn(g, K) * 3)
+    x = _randn(g, M, K)
+    xn = _norm64(x, scale, shift).float()
+    xp = _to_planes(xn)
+    if K <= gpt2.MAX_NORM_DIM:
+        xn = gpt2.layernorm(x, scale, shift, 1e-5)
+        xp = gpt2.layernorm(x, scale, shift, 1e-5, planes=True)
+        assert torch.equal(xp, _to_planes(xn))
+    assert torch.equal(_planes64(xp), xn.double())
+    w, b, res = _randn(g, N, K) * 0.05, _randn(g, N), _randn(g, M, N)
+    y64 = xn.double() @ w.double().t().contiguous()
+    lib = _rel(torch.nn.functional.linear(xn, w, b), y64 + b.double())
+    auto = gpt2.planes_splits(M, w)
+    assert 1 <= auto <= 8
+    for splits in sorted({1, auto, min(3, K // 32), min(8, K // 32)}):
+        got = gpt2.linear_planes(xp, w, b, splits, residual=res)
+        assert _rel(got, y64 + b.double() + res.double()) <= F32
+        got = gpt2.linear_planes(xp, w, b, splits)
+        assert _rel(got, y64 + b.double()) <= min(F32, max(1.25 * lib, 2e-7))
+        got = gpt2.linear_planes(xp, w, None, splits, gelu=True)
+        assert got.shape == (3, M, N) and _rel(_planes64(got), _gelu64(y64)) <= F32
+
+
 @pytest.mark.gpu
 def test_cast_rounds_as_torch_does():
     """Arrays from one value group up to several workgroups, in one launch, bit for bit."""
@@ -217,6 +272,23 @@ def test_block_matches_its_torch_operators(emb, heads, bias):
     hook.remove()
     hook2.remove()
     assert seen == [x.shape] and _rel(hooked, fused) <= 1e-3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,split", [(1023, False), (1024, True), (1037, True)])
+def test_block_mlp_on_split_float32(rows, split):
+    """Either side of the size from which the block's MLP runs on the split-float32 kernel, against the
+    general path (a hook on the MLP): the attention is the same, the MLP float32 on both."""
+    blk, g = _block(512, 8, context_length=1100)
+    x = _randn(g, 1, rows, 512)
+    with torch.no_grad():
+        assert (blk._mlp_splits(x) is not None) is split
+        got = blk(x)
+        hook = blk.ff.register_forward_hook(lambda *a: None)
+        assert blk._mlp_splits(x) is None
+        want = blk(x)
+        hook.remove()
+    assert _rel(got, want) <= 2 * F32
 
 
 @pytest.mark.gpu

@@ -7,6 +7,8 @@
 //                       before it and the rounding to bf16 after it where the caller has them;
 //   gelu_kernel         the tanh GELU in one pass;
 //   cast_kernel         float32 -> bf16 copies of several weights in one launch;
+//   linear_planes_kernel  the MLP's float32 linears on the bf16 matrix units, from exact three-way
+//                       splits of both operands;
 //   linear_rows_kernel  a projection of at most 8 rows read straight from the float32 weights,
 //                       with the LayerNorm before it and the bias, GELU and residual after it.
 //
@@ -20,6 +22,7 @@
 #include <algorithm>
 
 #include "tfgfa.h"
+#include "tfgfa_device.h"
 #include "tfgfa_gpt2.h"
 
 namespace tfgpt2 {
@@ -60,6 +63,30 @@ __device__ __forceinline__ float gelu(float x) {
   return 0.5f * x * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * (x * x * x))));
 }
 
+// A float32 value as three bf16 ones that add up to it exactly: itself rounded to bf16 (8 significant
+// bits), the remainder (at most 2^-9 of it, 16 bits) rounded, and the rest (at most 2^-18, 8 bits).  An
+// infinity, a NaN and what rounds to infinity (the top 2^-9 of the float range) give NaN.
+// top_pair: two values rounded, packed; drop_lo, drop_hi: what the first and the second leave.
+__device__ __forceinline__ uint32_t top_pair(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+__device__ __forceinline__ float drop_lo(float a, uint32_t top) { return a - __uint_as_float(top << 16); }
+__device__ __forceinline__ float drop_hi(float b, uint32_t top) {
+  return b - __uint_as_float(top & 0xffff0000u);
+}
+// Four values into the three planes of a (3, rows, width) array, `plane` elements apart.
+__device__ __forceinline__ void store_planes(__bf16* y, long long plane, f32x4 v) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    const u32x2 top = {top_pair(v[0], v[1]), top_pair(v[2], v[3])};
+    *reinterpret_cast<u32x2*>(y + p * plane) = top;
+    v = f32x4{drop_lo(v[0], top[0]), drop_hi(v[1], top[0]), drop_lo(v[2], top[1]), drop_hi(v[3], top[1])};
+  }
+}
+
 // Normalises a row held as v[i] = elements 4 * (64 i + lane) .. +3 (those below d; the others are
 // zero) in place: two passes over registers, so the variance is that of the centred values.
 template <int kV>
@@ -93,10 +120,12 @@ __device__ __forceinline__ void normalise_row(f32x4 (&v)[kV], int d, int lane, f
 //   613 rows of 1600: 4.9 us to bf16, 5.1 us with the residual (four rows per workgroup,
 //   scale and shift loaded where used: 7.2 and 9.3); the operators they stand for: about 32 us a
 //   norm, and 86 us for the mixed bf16 + float32 add before the second.
-template <int kV, bool kDelta, typename Y>
+enum { kOutF32 = 0, kOutBf16 = 1, kOutPlanes = 2 };
+
+template <int kV, bool kDelta, int kOut>
 __global__ __launch_bounds__(64) void layernorm_kernel(
     const float* x, const __bf16* __restrict__ delta, float* sum, const float* __restrict__ scale,
-    const float* __restrict__ shift, Y* __restrict__ y, int d, float eps) {
+    const float* __restrict__ shift, void* __restrict__ y, int d, float eps) {
   const int lane = threadIdx.x;
   const long long base = (long long)blockIdx.x * d;
   // Elements past the row are read at its start and zeroed: loads with no branch between them go
@@ -126,7 +155,14 @@ __global__ __launch_bounds__(64) void layernorm_kernel(
 #pragma unroll
   for (int i = 0; i < kV; ++i) {
     const int c = 4 * (64 * i + lane);
-    if (c < d) store4(y + base + c, v[i] * g[i] + h[i]);
+    if (c >= d) continue;
+    const f32x4 o = v[i] * g[i] + h[i];
+    if (kOut == kOutF32)
+      store4(static_cast<float*>(y) + base + c, o);
+    else if (kOut == kOutBf16)
+      store4(static_cast<__bf16*>(y) + base + c, o);
+    else
+      store_planes(static_cast<__bf16*>(y) + base + c, (long long)gridDim.x * d, o);
   }
 }
 
@@ -164,6 +200,232 @@ __global__ __launch_bounds__(kCastThreads) void cast_kernel(Casts a) {
       if (u >= begin && u < a.end[i]) store4(a.dst[i] + 4 * (u - begin), load4(a.src[i] + 4 * (u - begin)));
       begin = a.end[i];
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------
+// The MLP's float32 linears: y = x w^T + bias for many rows.
+//
+// Bound: the matrix units.  The float32 MFMA peaks at 157 TFLOP/s (a library GEMM reaches 114-139 of
+// it), the bf16 one at 16 times that.  A float32 value is the exact sum of three bf16 values, so a
+// product of two is nine bf16 products; the six larger ones are computed (smallest first, float32
+// accumulation), the other three are below 2^-26 of the product, less than float32 rounds it by.
+// The largest of the six has sums of its own, rounded once per 16 of the contraction (the float32
+// GEMM: once per 4), so the result is closer to float64's than the float32 GEMM's: 613 x 1600 -> 6400
+// 2.4e-7 (7.1e-7), 613 x 6400 -> 1600 2.8e-7 (1.4e-6), 100 x 3072 -> 768 1.4e-7 (5.0e-7).
+// x arrives as three planes, written so by the kernels that produce it; the weights are split in
+// registers, 5.5 VALU instructions a value.  A workgroup of 8 waves (2 a SIMD: one wave's splits
+// overlap the other's MFMAs) computes 128 rows x 128 outputs, a wave 64 x 32: 12 MFMAs for 12 split
+// steps per 16 of the contraction.  Steps of 32 stream into a ring of three 40-KiB slots by direct
+// buffer -> LDS loads (24 KiB of planes, 64-B rows with chunk c of row r at c ^ ((r >> 2) & 3); 16 KiB
+// of weights, 128-B rows swizzled as swz_k), one barrier a step.
+// A grid that leaves CUs idle splits the contraction into S partial sums (choose_k_splits), added in
+// order by reduce_kernel.
+//   us, with bias (float32 library GEMM): 613 x 1600 -> 6400 82 (114), 613 x 6400 -> 1600 S = 3 86
+//   (104), 1000 x 1024 -> 4096 51 (68), 1000 x 4096 -> 1024 S = 4 55 (68), 4096 x 4096 -> 1024 205 (247).
+//   Both operands split in registers, 4 waves of 64 x 64 (613 x 1600 -> 6400): 97, 87 with the splits
+//   spread between the MFMAs; a single wave a SIMD does not overlap the two.
+using tfgfa::head_desc;
+using tfgfa::lds_addr;
+using tfgfa::lds_transfer;
+using tfgfa::swz_k;
+using tfgfa::wait_vmcnt;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef tfgfa::i32x4 i32x4;
+
+// The descriptor moved on by `bytes` (within its rows), the range still ending at the same address.
+__device__ __forceinline__ i32x4 advance(i32x4 desc, int bytes) {
+  const uint64_t base = ((uint64_t)(uint32_t)desc[1] << 32 | (uint32_t)desc[0]) + (uint32_t)bytes;
+  i32x4 d;
+  d[0] = (int)(uint32_t)base;
+  d[1] = (int)(uint32_t)(base >> 32);
+  d[2] = desc[2] - bytes;
+  d[3] = desc[3];
+  return d;
+}
+
+constexpr int kTile = 128;  // rows and outputs per workgroup
+constexpr int kXBytes = 24 * 1024, kStage = 40 * 1024, kStages = 3;
+// What is written: a split's sums; GELU(sums + bias) as planes; sums + bias + residual.
+enum { kPartial = 0, kGeluPlanes = 1, kFinal = 2 };
+
+template <int kMode>
+__global__ __launch_bounds__(512, 2) void linear_planes_kernel(
+    const __bf16* __restrict__ X, const float* __restrict__ W, int M, int N, int K, int tm, int tn,
+    int S, int steps, const float* __restrict__ bias, const float* __restrict__ residual,
+    void* __restrict__ Yv) {
+  __shared__ __attribute__((aligned(1024))) unsigned char ring[kStages * kStage];
+  // Workgroups are dealt to the 8 XCDs round-robin: each XCD gets a run of consecutive tiles, row
+  // tiles fastest, so the row tiles of one weight tile read it through one L2.
+  const int T = tm * tn * S, per = (T + 7) / 8;
+  const int t = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (t >= T) return;
+  const int mt = t % tm, nt = t / tm % tn, z = t / (tm * tn);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wave & 1, wc = wave >> 1;
+  const int m0 = mt * 128, n0 = nt * 128;
+  const int s0 = z * steps, ns = min(steps, K / 32 - s0);  // this split's steps (at least one)
+  // Rows past M of a plane read the next plane's or, past the last, zero; weight rows past N read
+  // zero.  None of their sums are stored.
+  const i32x4 xd = advance(head_desc(X + (long long)m0 * K, 3 * M - m0, K * 2), s0 * 64);
+  const i32x4 wd = advance(head_desc(W + (long long)n0 * K, N - n0, K * 4), s0 * 128);
+  int xo[3], wo[2];  // this wave's 3 of the 24 X transfers (plane, 16 rows) and 2 of the 16 W ones (8 rows)
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int blk = 3 * wave + i, row = 16 * (blk & 7) + (lane >> 2);
+    xo[i] = ((blk >> 3) * M + row) * K * 2 + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * (2 * wave + i) + (lane >> 3);
+    wo[i] = row * K * 4 + (((lane & 7) ^ swz_k(row)) << 4);
+  }
+  auto issue = [&](int s, int slot) {
+    unsigned char* dst = ring + slot * kStage;
+    const i32x4 x = advance(xd, s * 64), w = advance(wd, s * 128);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) lds_transfer(x, lds_addr(dst + (3 * wave + i) * 1024), xo[i]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) lds_transfer(w, lds_addr(dst + kXBytes + (2 * wave + i) * 1024), wo[i]);
+  };
+  const int r = lane & 31, h = lane >> 5;
+  int fx[2], fw[2][2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    fx[c] = (64 * wr + r) * 64 + (((2 * c + h) ^ ((r >> 2) & 3)) << 4);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) fw[c][e] = kXBytes + (32 * wc + r) * 128 + (((4 * c + 2 * h + e) ^ swz_k(r)) << 4);
+  }
+  // The largest product's sums and the five small ones' apart: the small ones' roundings are then
+  // 2^-8 of the large ones', which come once per 16 of the contraction.
+  f32x16 acc[2], low[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[b][e] = low[b][e] = 0.f;
+  typedef f32x4 Raw[2];
+  auto read_w = [&](Raw& q, int slot, int c, int e) { q[e] = *reinterpret_cast<const f32x4*>(ring + slot * kStage + fw[c][e]); };
+  auto read_x = [&](u32x4 (&q)[2][3], int slot, int c, int k) {  // k: 0..5 = plane * 2 + tile
+    const int p = k >> 1, b = k & 1;
+    q[b][p] = *reinterpret_cast<const u32x4*>(ring + slot * kStage + p * 8192 + b * 2048 + fx[c]);
+  };
+  auto split_step = [&](u32x4 (&o)[3], Raw& q, int k) {  // 12 steps: pair k / 3, plane k % 3
+    const int pair = k / 3, pl = k % 3, e = pair >> 1, c = 2 * (pair & 1);
+    const float x0 = q[e][c], x1 = q[e][c + 1];
+    uint32_t v = top_pair(x0, x1);
+    asm volatile("" : "+v"(v));
+    o[pl][pair] = v;
+    if (pl < 2) {
+      float r0 = drop_lo(x0, v), r1 = drop_hi(x1, v);
+      asm volatile("" : "+v"(r0), "+v"(r1));
+      q[e][c] = r0;
+      q[e][c + 1] = r1;
+    }
+  };
+  // MFMA i of 12: the six products, smallest first, of the two row tiles.
+  auto mma = [&](const u32x4 (&w)[3], const u32x4 (&x)[2][3], int i) {
+    constexpr int pw[6] = {2, 0, 1, 1, 0, 0}, px[6] = {0, 2, 1, 0, 1, 0};
+    const int p = i >> 1, b = i & 1;
+    f32x16& sum = p == 5 ? acc[b] : low[b];
+    sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, w[pw[p]]),
+                                                  __builtin_bit_cast(bf16x8, x[b][px[p]]), sum, 0, 0, 0);
+  };
+  // Waits for this wave's loads of a step, `ahead` later steps of 5 loads staying in flight, and for
+  // its LDS reads; then for the other waves.
+  auto sync = [&](int ahead) {
+    if (ahead >= 2)
+      wait_vmcnt<10>();
+    else if (ahead == 1)
+      wait_vmcnt<5>();
+    else
+      wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  issue(0, 0);
+  if (ns > 1) issue(1, 1);
+  if (ns > 2) issue(2, 2);
+  u32x4 XA[2][3], XB[2][3], WA[3], WB[3];
+  Raw R0, R1;
+  sync(min(ns - 1, 2));
+#pragma unroll
+  for (int e = 0; e < 2; ++e) { read_w(R0, 0, 0, e); read_w(R1, 0, 1, e); }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) read_x(XA, 0, 0, k);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) split_step(WA, R0, k);
+  int slot = 0;
+  for (int s = 0; s < ns; ++s) {
+    // Chunk 0 (16 of the step's 32), beside the split of chunk 1's weights.
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+      mma(WA, XA, i);
+      if (i < 6) read_x(XB, slot, 1, i);
+      split_step(WB, R1, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int next = slot == 2 ? 0 : slot + 1;
+    // Step s + 1 has landed in every wave's share, and every read of step s is complete: its slot
+    // takes step s + 3.  (After the last step the reads below get an old slot's values: unused.)
+    if (s + 1 < ns) {
+      sync(min(ns - 2 - s, 1));
+      if (s + 3 < ns) issue(s + 3, slot);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) read_w(R0, next, 0, e);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+      mma(WB, XB, i);
+      if (i < 6) read_x(XA, next, 0, i);
+      if (i >= 3)
+#pragma unroll
+        for (int k = 12 * (i - 3) / 9; k < 12 * (i - 2) / 9; ++k) split_step(WA, R0, k);
+      if (i >= 8 && i < 10) read_w(R1, next, 1, i - 8);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot = next;
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const int m = m0 + 64 * wr + 32 * b + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n = n0 + 32 * wc + 8 * g + 4 * h;
+      if (n >= N) continue;
+      f32x4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = acc[b][4 * g + e] + low[b][4 * g + e];
+      if (kMode != kPartial && bias != nullptr) v += load4(bias + n);
+      if (kMode == kGeluPlanes) {
+        store_planes(static_cast<__bf16*>(Yv) + (long long)m * N + n, (long long)M * N,
+                     f32x4{gelu(v[0]), gelu(v[1]), gelu(v[2]), gelu(v[3])});
+      } else {
+        const long long at = ((long long)z * M + m) * N + n;
+        if (kMode == kFinal && residual != nullptr) v += load4(residual + at);
+        store4(static_cast<float*>(Yv) + at, v);
+      }
+    }
+  }
+}
+// y = sum of the S partial sums, + bias, then GELU into planes, or + residual.  Bound: memory.
+template <int kMode>
+__global__ __launch_bounds__(256) void reduce_kernel(const float* __restrict__ part, int S, long long MN,
+                                                     int N, const float* __restrict__ bias,
+                                                     const float* __restrict__ residual,
+                                                     void* __restrict__ y) {
+  const long long i = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= MN) return;
+  f32x4 v = load4(part + i);
+  for (int z = 1; z < S; ++z) v += load4(part + z * MN + i);
+  if (bias != nullptr) v += load4(bias + i % N);
+  if (kMode == kGeluPlanes) {
+    store_planes(static_cast<__bf16*>(y) + i, MN, f32x4{gelu(v[0]), gelu(v[1]), gelu(v[2]), gelu(v[3])});
+  } else {
+    if (residual != nullptr) v += load4(residual + i);
+    store4(static_cast<float*>(y) + i, v);
   }
 }
 
@@ -338,17 +600,45 @@ static int launched() {
   return e == hipSuccess ? TFGFA_OK : -(int)e;
 }
 
-template <int kV, typename Y>
+template <int kV, int kOut>
 static void launch_norm(const float* x, const __bf16* delta, float* sum, const float* scale,
-                        const float* shift, Y* y, long long rows, int d, float eps,
+                        const float* shift, void* y, long long rows, int d, float eps,
                         hipStream_t stream) {
   const dim3 grid((unsigned)rows), block(64);
   if (delta != nullptr)
-    hipLaunchKernelGGL((layernorm_kernel<kV, true, Y>), grid, block, 0, stream, x, delta, sum,
+    hipLaunchKernelGGL((layernorm_kernel<kV, true, kOut>), grid, block, 0, stream, x, delta, sum,
                        scale, shift, y, d, eps);
   else
-    hipLaunchKernelGGL((layernorm_kernel<kV, false, Y>), grid, block, 0, stream, x, delta, sum,
+    hipLaunchKernelGGL((layernorm_kernel<kV, false, kOut>), grid, block, 0, stream, x, delta, sum,
                        scale, shift, y, d, eps);
+}
+
+template <int kV>
+static void launch_norm_out(const float* x, const __bf16* delta, float* sum, const float* scale,
+                            const float* shift, void* y, int out, long long rows, int d, float eps,
+                            hipStream_t stream) {
+  if (out == kOutF32)
+    launch_norm<kV, kOutF32>(x, delta, sum, scale, shift, y, rows, d, eps, stream);
+  else if (out == kOutBf16)
+    launch_norm<kV, kOutBf16>(x, delta, sum, scale, shift, y, rows, d, eps, stream);
+  else
+    launch_norm<kV, kOutPlanes>(x, delta, sum, scale, shift, y, rows, d, eps, stream);
+}
+
+// Splits of the contraction: the fewest rounds of workgroups (one per CU) times steps, counting a
+// split's partial sums as the steps that writing and adding them take.
+static int choose_k_splits(long long tiles, int steps, int cu_count) {
+  int best = 1;
+  long long best_cost = 0;
+  for (int s = 1; s <= TFGPT2_MAX_K_SPLITS && (s == 1 || steps / s >= 8); ++s) {
+    const long long rounds = (tiles * s + cu_count - 1) / cu_count;
+    const long long cost = rounds * ((steps + s - 1) / s + 4) + (s > 1 ? 6 + 2 * s : 0);
+    if (s == 1 || cost < best_cost) {
+      best = s;
+      best_cost = cost;
+    }
+  }
+  return best;
 }
 
 struct RowsArgs {
@@ -410,11 +700,11 @@ static void launch_rows_types(const RowsArgs& a, int parts, bool x_bf16, bool y_
 }  // namespace tfgpt2
 
 extern "C" int tfgpt2_layernorm(const float* x, const void* delta, float* sum, const float* scale,
-                                const float* shift, void* y, int y_bf16, int64_t rows, int d,
+                                const float* shift, void* y, int y_kind, int64_t rows, int d,
                                 float eps, void* hip_stream) {
   using namespace tfgpt2;
   if (rows < 0 || d < 4 || d > TFGPT2_MAX_NORM_DIM || (d & 3)) return TFGFA_ERR_BAD_SHAPE;
-  if (y_bf16 != 0 && y_bf16 != 1) return TFGFA_ERR_DTYPE;
+  if (y_kind < TFGPT2_F32 || y_kind > TFGPT2_PLANES) return TFGFA_ERR_DTYPE;
   if (rows == 0) return TFGFA_OK;
   if (rows > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
   if (!x || !scale || !shift || !y || (delta != nullptr && sum == nullptr)) return TFGFA_ERR_NULL_POINTER;
@@ -423,17 +713,10 @@ extern "C" int tfgpt2_layernorm(const float* x, const void* delta, float* sum, c
     return TFGFA_ERR_ALIGNMENT;
   const __bf16* dl = static_cast<const __bf16*>(delta);
   const hipStream_t stream = (hipStream_t)hip_stream;
-  if (d <= 1024) {
-    if (y_bf16)
-      launch_norm<4>(x, dl, sum, scale, shift, static_cast<__bf16*>(y), rows, d, eps, stream);
-    else
-      launch_norm<4>(x, dl, sum, scale, shift, static_cast<float*>(y), rows, d, eps, stream);
-  } else {
-    if (y_bf16)
-      launch_norm<8>(x, dl, sum, scale, shift, static_cast<__bf16*>(y), rows, d, eps, stream);
-    else
-      launch_norm<8>(x, dl, sum, scale, shift, static_cast<float*>(y), rows, d, eps, stream);
-  }
+  if (d <= 1024)
+    launch_norm_out<4>(x, dl, sum, scale, shift, y, y_kind, rows, d, eps, stream);
+  else
+    launch_norm_out<8>(x, dl, sum, scale, shift, y, y_kind, rows, d, eps, stream);
   return launched();
 }
 
@@ -519,5 +802,55 @@ extern "C" int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_sca
     launch_rows_types<1>(a, parts, x_bf16 != 0, y_bf16 != 0, ln, gelu != 0, stream);
   else
     launch_rows_types<2>(a, parts, x_bf16 != 0, y_bf16 != 0, ln, gelu != 0, stream);
+  return launched();
+}
+
+extern "C" int tfgpt2_linear_planes_splits(int M, int N, int K, int cu_count) {
+  using namespace tfgpt2;
+  if (M < 1 || N < 4 || (N & 3) || K < 32 || K % 32 || cu_count < 1) return 0;
+  if (3LL * M * K * 2 > INT32_MAX || (long long)N * K * 4 > INT32_MAX) return 0;
+  const long long tiles = (long long)((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile);
+  if (tiles * TFGPT2_MAX_K_SPLITS > INT32_MAX / 2) return 0;
+  return choose_k_splits(tiles, K / 32, cu_count);
+}
+
+extern "C" int tfgpt2_linear_planes(const void* x, const float* w, const float* bias, int gelu_planes,
+                                    const float* residual, void* y, float* part, int splits, int M,
+                                    int N, int K, void* hip_stream) {
+  using namespace tfgpt2;
+  if (gelu_planes != 0 && gelu_planes != 1) return TFGFA_ERR_DTYPE;
+  if (M == 0 && N > 0 && K > 0) return TFGFA_OK;
+  if (tfgpt2_linear_planes_splits(M, N, K, 1) == 0) return TFGFA_ERR_BAD_SHAPE;
+  if (splits < 1 || splits > TFGPT2_MAX_K_SPLITS || splits > K / 32 || (gelu_planes && residual))
+    return TFGFA_ERR_BAD_SHAPE;
+  if (!x || !w || !y || (splits > 1 && part == nullptr)) return TFGFA_ERR_NULL_POINTER;
+  if (misaligned(x) || misaligned(w) || misaligned(bias) || misaligned(residual) || misaligned(y) ||
+      misaligned(part))
+    return TFGFA_ERR_ALIGNMENT;
+  const int tm = (M + kTile - 1) / kTile, tn = (N + kTile - 1) / kTile;
+  const int steps = (K / 32 + splits - 1) / splits;
+  const int S = (K / 32 + steps - 1) / steps;  // no split without a step
+  const dim3 grid((unsigned)((tm * tn * S + 7) / 8 * 8));
+  const hipStream_t stream = (hipStream_t)hip_stream;
+  const __bf16* xp = static_cast<const __bf16*>(x);
+  if (S == 1) {
+    if (gelu_planes)
+      hipLaunchKernelGGL(linear_planes_kernel<kGeluPlanes>, grid, dim3(512), 0, stream, xp, w, M, N,
+                         K, tm, tn, 1, steps, bias, residual, y);
+    else
+      hipLaunchKernelGGL(linear_planes_kernel<kFinal>, grid, dim3(512), 0, stream, xp, w, M, N, K, tm,
+                         tn, 1, steps, bias, residual, y);
+    return launched();
+  }
+  hipLaunchKernelGGL(linear_planes_kernel<kPartial>, grid, dim3(512), 0, stream, xp, w, M, N, K, tm,
+                     tn, S, steps, bias, residual, static_cast<void*>(part));
+  const long long MN = (long long)M * N;
+  const dim3 rgrid((unsigned)((MN / 4 + 255) / 256));
+  if (gelu_planes)
+    hipLaunchKernelGGL(reduce_kernel<kGeluPlanes>, rgrid, dim3(256), 0, stream, part, S, MN, N, bias,
+                       residual, y);
+  else
+    hipLaunchKernelGGL(reduce_kernel<kFinal>, rgrid, dim3(256), 0, stream, part, S, MN, N, bias,
+                       residual, y);
   return launched();
 }

@@ -134,7 +134,7 @@ void check(int st, const char* what) {
 }
 
 void gpt2_layernorm(std::uintptr_t x, std::uintptr_t delta, std::uintptr_t sum,
-                    std::uintptr_t scale, std::uintptr_t shift, std::uintptr_t y, bool y_bf16,
+                    std::uintptr_t scale, std::uintptr_t shift, std::uintptr_t y, int y_kind,
                     std::int64_t rows, int d, float eps, std::uintptr_t stream) {
   int st;
   {
@@ -142,7 +142,7 @@ void gpt2_layernorm(std::uintptr_t x, std::uintptr_t delta, std::uintptr_t sum,
     st = tfgpt2_layernorm(reinterpret_cast<const float*>(x), reinterpret_cast<const void*>(delta),
                           reinterpret_cast<float*>(sum), reinterpret_cast<const float*>(scale),
                           reinterpret_cast<const float*>(shift), reinterpret_cast<void*>(y),
-                          y_bf16 ? 1 : 0, rows, d, eps, reinterpret_cast<void*>(stream));
+                          y_kind, rows, d, eps, reinterpret_cast<void*>(stream));
   }
   check(st, "tfgpt2_layernorm");
 }
@@ -203,6 +203,21 @@ void gpt2_linear_rows(
                             y_bf16 ? 1 : 0, M, N, K, reinterpret_cast<void*>(stream));
   }
   check(st, "tfgpt2_linear_rows");
+}
+
+void gpt2_linear_planes(std::uintptr_t x, std::uintptr_t w, std::uintptr_t bias, bool gelu_planes,
+                        std::uintptr_t residual, std::uintptr_t y, std::uintptr_t part, int splits,
+                        int M, int N, int K, std::uintptr_t stream) {
+  int st;
+  {
+    py::gil_scoped_release nogil;
+    st = tfgpt2_linear_planes(reinterpret_cast<const void*>(x), reinterpret_cast<const float*>(w),
+                              reinterpret_cast<const float*>(bias), gelu_planes ? 1 : 0,
+                              reinterpret_cast<const float*>(residual), reinterpret_cast<void*>(y),
+                              reinterpret_cast<float*>(part), splits, M, N, K,
+                              reinterpret_cast<void*>(stream));
+  }
+  check(st, "tfgpt2_linear_planes");
 }
 
 py::dict device_info() {
@@ -272,7 +287,7 @@ PYBIND11_MODULE(_C, m) {
   });
   m.def("gpt2_layernorm", &gpt2_layernorm, "LayerNorm, with an optional residual add before it",
         py::arg("x"), py::arg("delta"), py::arg("sum"), py::arg("scale"), py::arg("shift"),
-        py::arg("y"), py::arg("y_bf16"), py::arg("rows"), py::arg("d"), py::arg("eps"),
+        py::arg("y"), py::arg("y_kind"), py::arg("rows"), py::arg("d"), py::arg("eps"),
         py::arg("stream"));
   m.def("gpt2_gelu", &gpt2_gelu, "GELU (tanh form), elementwise", py::arg("x"), py::arg("y"),
         py::arg("n"), py::arg("stream"));
@@ -283,6 +298,19 @@ PYBIND11_MODULE(_C, m) {
         py::arg("x_bf16"), py::arg("ln_scale"), py::arg("ln_shift"), py::arg("eps"),
         py::arg("parts"), py::arg("gelu"), py::arg("residual"), py::arg("y_bf16"), py::arg("M"),
         py::arg("N"), py::arg("K"), py::arg("stream"));
+  m.def("gpt2_linear_planes", &gpt2_linear_planes,
+        "A float32 linear layer on the bf16 matrix units, from three-way splits", py::arg("x"),
+        py::arg("w"), py::arg("bias"), py::arg("gelu_planes"), py::arg("residual"), py::arg("y"),
+        py::arg("part"), py::arg("splits"), py::arg("M"), py::arg("N"), py::arg("K"),
+        py::arg("stream"));
+  m.def("gpt2_linear_planes_splits", [](int M, int N, int K) {
+    int cu = 0;
+    check(tfgfa_device_info(&cu, nullptr, nullptr, 0), "tfgfa_device_info");
+    return tfgpt2_linear_planes_splits(M, N, K, cu);
+  });
+  m.attr("GPT2_F32") = TFGPT2_F32;
+  m.attr("GPT2_BF16") = TFGPT2_BF16;
+  m.attr("GPT2_PLANES") = TFGPT2_PLANES;
   m.attr("GPT2_MAX_NORM_DIM") = TFGPT2_MAX_NORM_DIM;
   m.attr("GPT2_MAX_ROWS") = TFGPT2_MAX_ROWS;
   m.def("device_info", &device_info, "CU count, shader clock (MHz) and arch of the current device");

@@ -47,15 +47,43 @@ def _ptr(t) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-def layernorm(x, scale, shift, eps: float, dtype=torch.float32, delta=None):
-    """LayerNorm over the last dimension, in ``dtype`` (float32 or bfloat16).  With ``delta`` (bf16,
-    like x): the norm of x + delta, returned as (x + delta, norm)."""
+def _planes(rows: int, width: int, dev):
+    return torch.empty((3, rows, width), dtype=torch.bfloat16, device=dev)
+
+
+def layernorm(x, scale, shift, eps: float, dtype=torch.float32, delta=None, planes: bool = False):
+    """LayerNorm over the last dimension, in ``dtype`` (float32 or bfloat16), or as the three bf16
+    planes (3, rows, width) that :func:`linear_planes` takes.  With ``delta`` (bf16, like x): the norm
+    of x + delta, returned as (x + delta, norm)."""
     d = x.shape[-1]
-    y = torch.empty(x.shape, dtype=dtype, device=x.device)
+    rows = x.numel() // d
+    y = _planes(rows, d, x.device) if planes else torch.empty(x.shape, dtype=dtype, device=x.device)
     s = None if delta is None else torch.empty_like(x)
+    kind = _C.GPT2_PLANES if planes else _C.GPT2_BF16 if dtype == torch.bfloat16 else _C.GPT2_F32
     _launch_on(x.get_device(), _C.gpt2_layernorm, x.data_ptr(), _ptr(delta), _ptr(s), scale.data_ptr(),
-               shift.data_ptr(), y.data_ptr(), dtype == torch.bfloat16, x.numel() // d, d, eps)
+               shift.data_ptr(), y.data_ptr(), kind, rows, d, eps)
     return y if delta is None else (s, y)
+
+
+def planes_splits(rows: int, w) -> int:
+    """Splits of the contraction :func:`linear_planes` would use, 0 where it does not take the sizes."""
+    return _C.gpt2_linear_planes_splits(rows, *w.shape)
+
+
+def linear_planes(x, w, bias, splits: int, gelu: bool = False, residual=None):
+    """x w^T + bias for ``x`` as (3, rows, K) planes and float32 ``w`` (N, K): + ``residual`` (float32, any
+    shape of rows x N, the result's too), or with ``gelu`` its GELU as planes (3, rows, N)."""
+    rows, (N, K), dev = x.shape[1], w.shape, x.device
+    part = None
+    if gelu:
+        y = _planes(rows, N, dev)
+    else:
+        y = torch.empty((rows, N) if residual is None else residual.shape, dtype=torch.float32, device=dev)
+    if splits > 1:
+        part = torch.empty((splits, rows, N), dtype=torch.float32, device=dev)
+    _launch_on(x.get_device(), _C.gpt2_linear_planes, x.data_ptr(), w.data_ptr(), _ptr(bias), gelu,
+               _ptr(residual), y.data_ptr(), _ptr(part), splits, rows, N, K)
+    return y
 
 
 def gelu(x):

@@ -401,14 +401,37 @@ class TransformerBlock(nn.Module):
         return (x.dim() == 3 and g.takes(x, norm1.scale, norm1.shift, norm2.scale, norm2.shift)
                 and norm1._native(x) and norm2._native(x))
 
+    def _plain_mlp(self) -> bool:
+        ff = self.ff
+        return (_plain(ff, FeedForward) and _plain(ff.layers, nn.Sequential) and len(ff.layers) == 3
+                and _plain(ff.layers[0], nn.Linear) and _plain(ff.layers[1], GELU) and _plain(ff.layers[2], nn.Linear))
+
+    def _mlp_splits(self, x):
+        """The contraction splits of the MLP's two linears on the split-float32 kernel, or None where
+        they are not plain float32 linears of sizes it takes, or small: from 2^30 multiplications a
+        linear the whole block's kernels take less time (us, library / split: GPT-2 small 256 rows
+        82 / 85, 613 rows 114 / 105; medium 128 rows 84 / 88, 256 rows 97 / 94; XL 64 rows 104 / 109, 128
+        rows 123 / 117, 1024 rows 481 / 363)."""
+        g = _gpt2()
+        if not self._plain_mlp():
+            return None
+        up, down = self.ff.layers[0], self.ff.layers[2]
+        hidden, d = up.weight.shape
+        if d != x.shape[2] or down.weight.shape != (d, hidden) or not g.takes(
+                x, up.weight, up.bias, down.weight, down.bias):
+            return None
+        rows = x.shape[0] * x.shape[1]
+        if rows * hidden * d < 1 << 30:
+            return None
+        splits = g.planes_splits(rows, up.weight), g.planes_splits(rows, down.weight)
+        return splits if splits[0] and splits[1] else None
+
     def _rows_fused(self, x, cache) -> bool:
         """Whether a decode step may run its projections on the few-row kernel: as for _fused, with
         plain linears, float32 weights, a bf16 cache that holds tokens and few enough rows."""
         g, att, ff = _gpt2(), self.att, self.ff
         if not (cache is not None and cache.length > 0 and x.shape[1] == 1 and att.impl_type in ("hip", "cuda")
-                and att._plain_linears() and _plain(ff, FeedForward) and _plain(ff.layers, nn.Sequential)
-                and len(ff.layers) == 3 and _plain(ff.layers[0], nn.Linear) and _plain(ff.layers[1], GELU)
-                and _plain(ff.layers[2], nn.Linear) and cache.k[0].dtype == torch.bfloat16):
+                and att._plain_linears() and self._plain_mlp() and cache.k[0].dtype == torch.bfloat16):
             return False
         rows, d = x.shape[0], x.shape[2]
         qkv, up, down = (att.W_query, att.W_key, att.W_value), ff.layers[0], ff.layers[2]
@@ -438,7 +461,9 @@ class TransformerBlock(nn.Module):
 
     def _forward_fused(self, x, kv_cache, layer):
         """The block with each norm one kernel: norm1 writes the bf16 that autocast would round its
-        result to (once, not for each projection), the residual add runs inside norm2's kernel."""
+        result to (once, not for each projection), the residual add runs inside norm2's kernel.  The
+        MLP runs on the split-float32 kernel where it takes it: norm2 and the GELU write the three
+        bf16 planes it reads, and the second residual add is part of its last sum."""
         if self._rows_fused(x, kv_cache):
             return self._forward_rows(x, kv_cache, layer)
         g = _gpt2()
@@ -448,6 +473,12 @@ class TransformerBlock(nn.Module):
         with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
             y = self.att(h, kv_cache, layer)
         if g.takes(y, dtypes=(torch.bfloat16,)) and y.shape == x.shape:
+            splits = self._mlp_splits(x)
+            if splits is not None:
+                x, h = g.layernorm(x, norm2.scale, norm2.shift, norm2.eps, delta=y, planes=True)
+                up, down = self.ff.layers[0], self.ff.layers[2]
+                h = g.linear_planes(h, up.weight, up.bias, splits[0], gelu=True)
+                return g.linear_planes(h, down.weight, down.bias, splits[1], residual=x)
             x, h = g.layernorm(x, norm2.scale, norm2.shift, norm2.eps, delta=y)
         else:
             x = y + x
