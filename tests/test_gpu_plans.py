@@ -24,24 +24,28 @@ NARROW = [  # head dims up to 64
     (1, 1, 1025, 1025, True),    # 2 row waves x 4 key groups, one row past a block
     (1, 2, 33, 1100, False),     # the same, unmasked, a ragged last tile
     (1, 1, 1300, 1090, True),    # the same, rows past the last key
-    (1, 130, 1, 1, True),        # 2 x 2: one key, the second group without a tile
+    (1, 256, 65, 1, True),       # 2 x 2: one key, the second group without a tile
     (1, 130, 100, 100, True),
-    (1, 131, 65, 65, True),
+    (1, 200, 96, 96, True),
     (2, 65, 127, 127, True),
-    (1, 44, 641, 641, True),
-    (1, 130, 5, 1001, False),    # 4 x 2, unmasked
+    (1, 256, 5, 1100, False),    # 4 x 2, unmasked
     (1, 150, 127, 1056, False),
     (1, 20, 2049, 2049, True),   # 4 x 2, causal
+    (1, 130, 1, 1, True),        # 32-row blocks, 4 key waves: one row, one key
+    (1, 131, 65, 65, True),
     (1, 60, 640, 640, True),     # whole blocks
+    (1, 44, 641, 641, True),
 ]
 WIDE = [  # head dims past 64
     (1, 3, 130, 130, True),      # 32-row blocks, 4 key waves
-    (1, 70, 65, 65, True),       # 2 x 2
-    (1, 70, 1, 1, True),
-    (1, 25, 600, 97, True),
-    (1, 96, 33, 289, False),
-    (1, 35, 700, 700, True),     # 4 x 2
+    (1, 70, 65, 65, True),
     (1, 200, 3, 705, False),
+    (1, 180, 34, 34, True),      # 2 x 2
+    (1, 140, 33, 65, True),
+    (1, 192, 65, 33, True),
+    (1, 25, 600, 97, True),
+    (1, 35, 700, 700, True),     # 4 x 2
+    (1, 200, 100, 705, False),
     (1, 20, 2049, 2049, True),
     (1, 130, 200, 130, False),   # whole blocks
 ]
