@@ -29,7 +29,7 @@ extern "C" {
 #define TFGPT2_MAX_K_SPLITS 8
 
 /* What a result is written as.  PLANES: (3, rows, width) bf16, three arrays whose values add up to
- * the float32 result exactly (NaN where it is infinite or NaN). */
+ * the float32 result exactly (where it is infinite or NaN: itself, then NaN). */
 #define TFGPT2_F32    0
 #define TFGPT2_BF16   1
 #define TFGPT2_PLANES 2
@@ -84,7 +84,7 @@ int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_scale, const f
  *   y = GELU(x w^T + bias) as PLANES       (3, M, N) bf16          gelu_planes = 1 (no residual)
  *   x  (3, M, K) bf16 PLANES    w  (N, K) float32    bias  (N) or NULL    residual  (M, N) or NULL
  * Every product is that of the float32 values to 2^-26 of itself, sums are float32: as close to the
- * exact result as a float32 GEMM.  Where x or w is infinite, or rounds to it as bf16, the result is NaN.
+ * exact result as a float32 GEMM.  Infinities, NaN and overflow give what they give there.
  * splits: 1..TFGPT2_MAX_K_SPLITS partial sums of the contraction, tfgpt2_linear_planes_splits' choice
  * for a device of cu_count CUs (0: sizes not taken: N a multiple of 4, K of 32, planes and weights
  * below 2 GiB).  part: splits * M * N floats (NULL for one split); the partial sums are

@@ -160,7 +160,9 @@ def test_linear_rows_matches_float64(M, N, K):
 def _to_planes(x):
     out = []
     for _ in range(3):
-        out.append(x.to(torch.bfloat16))
+        t = x.to(torch.bfloat16)
+        cut = (x.view(torch.int32) & -65536).view(torch.float32).to(torch.bfloat16)
+        out.append(torch.where(x.isfinite() & ~t.isfinite(), cut, t))  # no finite value becomes infinite
         x = x - out[-1].float()
     return torch.stack(out)
 
@@ -202,6 +204,53 @@ def test_linear_planes_matches_float64(M, N, K):
         assert _rel(got, y64 + b.double()) <= min(F32, max(1.25 * lib, 2e-7))
         got = gpt2.linear_planes(xp, w, None, splits, gelu=True)
         assert got.shape == (3, M, N) and _rel(_planes64(got), _gelu64(y64)) <= F32
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 3])
+def test_linear_planes_passes_infinities_as_float32_does(splits):
+    """Infinities, NaN, values that round to infinity as bf16 and products that overflow, in x and in
+    the weights, one row or output each: infinite and NaN results where float32's linear has them
+    (no sum here overflows depending on its order), the finite ones to F32 of the sum of their terms'
+    magnitudes."""
+    from custom_flash_attn import gpt2
+
+    top = torch.finfo(torch.float32).max
+    g = torch.Generator(device=DEV).manual_seed(11)
+    M, N, K = 133, 136, 160
+    x, w, b = _randn(g, M, K), _randn(g, N, K) * 0.05, _randn(g, N)
+    w[:, 3] = torch.where(torch.arange(N, device=DEV) % 2 == 0, 0.5, -0.25)  # exact in bf16: lower parts zero
+    w[5, 3] = 0.0
+    x[2, 3], x[3, 3], x[4, 3], x[132, 3] = math.inf, -math.inf, math.nan, math.inf
+    x[6, 3], x[7, 3] = top, -top * (1 - 2.0 ** -10)
+    x[8, 150], x[8, 151] = math.inf, -math.inf   # the last step, alone and against each other
+    x[9, :] = 1e30
+    w[7, :] = 1e30                               # products past the float range
+    w[20, 77], w[21, 78], w[22, 79] = math.inf, math.nan, top
+    x[:, 79] = torch.sign(x[:, 79]) * 0.25
+    x64, w64, b64 = x.double().cpu(), w.double().cpu(), b.double().cpu()
+    ref = torch.nn.functional.linear(x64, w64, b64)
+    terms = torch.nn.functional.linear(x64.abs(), w64.abs(), b64.abs())
+    got = gpt2.linear_planes(_to_planes(x), w, b, splits).cpu()
+    ref32 = ref.float()                          # float32's range: 1e60 is infinite
+    assert torch.equal(got.isnan(), ref32.isnan())
+    assert torch.equal(got[ref32.isinf()], ref32[ref32.isinf()])
+    fin = ref32.isfinite()
+    assert 0 < fin.sum() < fin.numel() and ((got.double() - ref).abs() <= F32 * terms)[fin].all()
+
+
+@pytest.mark.gpu
+def test_planes_hold_the_top_of_the_float_range():
+    """A norm's result that is finite but rounds to infinity as bf16 comes back from its planes exactly."""
+    from custom_flash_attn import gpt2
+
+    K = 64
+    x = torch.where(torch.arange(K, device=DEV) % 2 == 0, 1.0, -1.0).repeat(3, 1)   # its own norm
+    shift = torch.zeros(K, device=DEV)
+    scale = torch.full((K,), torch.finfo(torch.float32).max, device=DEV) * (1 - torch.arange(K, device=DEV) * 2.0 ** -13)
+    y = gpt2.layernorm(x, scale, shift, 1e-9)
+    assert y.isfinite().all() and not y.to(torch.bfloat16).isfinite().all()
+    assert torch.equal(_planes64(gpt2.layernorm(x, scale, shift, 1e-9, planes=True)), y.double())
 
 
 @pytest.mark.gpu

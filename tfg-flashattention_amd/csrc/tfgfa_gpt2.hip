@@ -65,7 +65,9 @@ __device__ __forceinline__ float gelu(float x) {
 
 // A float32 value as three bf16 ones that add up to it exactly: itself rounded to bf16 (8 significant
 // bits), the remainder (at most 2^-9 of it, 16 bits) rounded, and the rest (at most 2^-18, 8 bits).  An
-// infinity, a NaN and what rounds to infinity (the top 2^-9 of the float range) give NaN.
+// infinity or a NaN stays the first, the others are NaN then.  A finite value that rounds to infinity
+// (the top 2^-9 of the float range) has no such split: store_planes truncates it instead (a remainder
+// of 16 bits is left all the same), a weight's gives NaN, and plain_sums what the NaN stands for.
 // top_pair: two values rounded, packed; drop_lo, drop_hi: what the first and the second leave.
 __device__ __forceinline__ uint32_t top_pair(float a, float b) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -81,7 +83,15 @@ __device__ __forceinline__ void store_planes(__bf16* y, long long plane, f32x4 v
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    const u32x2 top = {top_pair(v[0], v[1]), top_pair(v[2], v[3])};
+    u32x2 top = {top_pair(v[0], v[1]), top_pair(v[2], v[3])};
+    if (p == 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t bits = __float_as_uint(v[e]), high = (e & 1) ? 0xffff0000u : 0x0000ffffu;
+        if ((bits & 0x7fff8000u) == 0x7f7f8000u)  // finite, half a unit or more above bf16's largest
+          top[e >> 1] = (top[e >> 1] & ~high) | ((e & 1) ? bits & 0xffff0000u : bits >> 16);
+      }
+    }
     *reinterpret_cast<u32x2*>(y + p * plane) = top;
     v = f32x4{drop_lo(v[0], top[0]), drop_hi(v[1], top[0]), drop_lo(v[2], top[1]), drop_hi(v[3], top[1])};
   }
@@ -246,6 +256,31 @@ __device__ __forceinline__ i32x4 advance(i32x4 desc, int bytes) {
   return d;
 }
 
+// Four outputs n.. of row m over the contraction's k0..k1 with the products in float32.  Infinities in
+// x or w, weights at the top of the float range and overflow meet NaN in the split products where a
+// float32 GEMM need not (inf - inf, inf * 0), so a NaN sum is computed again; ordinary values never are.
+// Ends early where all four are NaN in float32 too (a NaN in x, or in every weight row).
+__device__ __forceinline__ f32x4 plain_sums(const __bf16* X, const float* W, int M, int K, int m, int n,
+                                            int k0, int k1) {
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int k = k0; k < k1; k += 4) {
+    f32x4 x = load4(X + (long long)m * K + k);
+    const f32x4 x1 = load4(X + ((long long)M + m) * K + k), x2 = load4(X + (2LL * M + m) * K + k);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (__builtin_isfinite(x[e])) x[e] += x1[e] + x2[e];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+      const f32x4 w = load4(W + (long long)(n + o) * K + k);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[o] = fmaf(x[e], w[e], s[o]);
+    }
+    if (__builtin_isnan(s[0]) && __builtin_isnan(s[1]) && __builtin_isnan(s[2]) && __builtin_isnan(s[3])) break;
+  }
+  return s;
+}
+
 constexpr int kTile = 128;  // rows and outputs per workgroup
 constexpr int kXBytes = 24 * 1024, kStage = 40 * 1024, kStages = 3;
 // What is written: a split's sums; GELU(sums + bias) as planes; sums + bias + residual.
@@ -398,6 +433,8 @@ __global__ __launch_bounds__(512, 2) void linear_planes_kernel(
       f32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = acc[b][4 * g + e] + low[b][4 * g + e];
+      if (__builtin_isnan((v[0] + v[1]) + (v[2] + v[3])))  // (also of opposite infinities: the same again)
+        v = plain_sums(X, W, M, K, m, n, s0 * 32, (s0 + ns) * 32);
       if (kMode != kPartial && bias != nullptr) v += load4(bias + n);
       if (kMode == kGeluPlanes) {
         store_planes(static_cast<__bf16*>(Yv) + (long long)m * N + n, (long long)M * N,
