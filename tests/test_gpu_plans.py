@@ -95,3 +95,27 @@ def test_key_groups_merge_extreme_rows(B, H, N):
     assert (o[:, 1:].float() - o_ref).abs().max().item() <= 3 * U[torch.bfloat16] * v[:, 1:].abs().max().item()
     assert ((lse[:, 1:] - lse_ref).abs() <= 1e-4 + 1e-5 * lse_ref.abs()).all()
     assert torch.isfinite(lse).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_first_scores_of_minus_infinity(D, dtype):
+    """Keys of infinite magnitude and opposite sign score -inf and drop out of a row, also where they
+    are all a wave's or a key group's first half or tile holds.  A row of nothing else is NaN."""
+    for B, H, Nq, Nk, causal in (NARROW if D == 64 else WIDE):
+        if Nk < 600:
+            continue
+        for width, period in ((32, 64), (64, 256), (256, Nk)):  # first halves, first tiles, the first four tiles
+            print(f"D={D} {dtype} H={H} Nq={Nq} Nk={Nk} causal={causal} {width} of {period}", flush=True)
+            g = torch.Generator(device=DEV).manual_seed(Nq + Nk + period)
+            q, k, v = (torch.randn((B, H, n, D), device=DEV, generator=g).to(dtype) for n in (Nq, Nk, Nk))
+            q[..., 0] = -1
+            k[:, :, torch.arange(Nk, device=DEV) % period < width, 0] = math.inf
+            o, lse = custom_flash_attn.attention(q, k, v, causal=causal, return_lse=True)
+            assert torch.equal(custom_flash_attn.attention(q, k, v, causal=causal).isnan(), o.isnan())
+            o_ref, lse_ref = _reference(q, k, v, causal)
+            seen = lse_ref > -math.inf
+            assert torch.equal(seen, ~o.isnan().any(-1)) and torch.equal(seen, ~o.isnan().all(-1))
+            assert (o.float() - o_ref)[seen].abs().max().item() <= 3 * U[dtype] * v.abs().max().item()
+            assert (lse - lse_ref)[seen].abs().max().item() <= 1e-4
+            assert (lse[~seen] == -math.inf).all()

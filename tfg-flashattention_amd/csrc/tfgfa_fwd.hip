@@ -118,6 +118,10 @@ constexpr int kOutOfRange = 0x7FFFFFF0;
 // *as rounded* for the P.V MFMA, so the rounding of a dominant probability cancels between O's
 // numerator and denominator; the LSE uses l_run, the fp32 sum of the unrounded ones.
 
+// Offset of a row that has seen no score above -inf: finite, so that scores of -inf (q.k past the
+// float range, infinite keys) give probabilities of 0 wherever a wave's or a group's first ones
+// stand, and a merge weighs such a state by 0; a row with no other score is 0 / 0.
+constexpr float kLowestOffset = -0x1.fffffep127f;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -435,8 +439,8 @@ __device__ __forceinline__ float lane_max(const WaveState<Sh>& w) {
 // Moves the exp2 offset of every row to its exact running max, rescaling O and the sums, when
 // some lane's score exceeds its row's offset by more than the margin (wave-uniform branch, taken
 // at a wave's first half and then rarely).  Every computed half has an unmasked key in every
-// row (it starts at or below the wave's first row), so the pair max is finite and the first
-// half always moves m_run off -inf.
+// row (it starts at or below the wave's first row), so the first half with a score above -inf moves
+// m_run off kLowestOffset.
 template <class Sh>
 __device__ __forceinline__ void move_offset(WaveState<Sh>& w, float mx, float scale_log2,
                                             float inv_scale_log2) {
@@ -520,7 +524,7 @@ __device__ __forceinline__ typename Elem<typename Sh::T>::v8 k_operand(const Wav
 //                    the sums of P_u and its conversion to the element type
 // The offset check reads the lane's running sum l_p with this half's probabilities, as rounded
 // to the element type, added.  bf16: a rounded P above 2^64 makes that sum exceed the bound (an
-// overflow gives +inf, a -inf offset on a wave's first half gives +inf or NaN), so a sum above
+// overflow gives +inf, and so does the first offset, kLowestOffset, with any score above -inf), so a sum above
 // the bound, or not a number, takes the rare branch: move the offset to the rows' exact running
 // max, rescale O and the sums, recompute P_u.  A sum above the bound without any single P above
 // it moves the offset early, which is harmless (after a move every P is at most 1, so l_p stays
@@ -805,7 +809,8 @@ struct Strides {
 // rule (offset m_w, rounded-probability sum lp_w, fp32 sum l_w, unnormalised O_w):
 //   M = max_w m_w,  a_w = 2^(m_w - M),  O = sum_w a_w O_w / sum_w a_w lp_w,
 //   LSE = (M + log2 sum_w a_w l_w) ln 2.
-// A wave with no half contributes m_w = -inf (a_w = 0).
+// A wave with no half, or with scores of -inf only, has m_w = kLowestOffset and sums of 0: a_w = 0
+// beside any other.
 // A wave's partial: its unnormalised O rows (fp32, row-major, 64 * kDH columns, 16-B chunk c of
 // row r at physical chunk c ^ (r % (16 kDH))) and its row statistics.
 template <class Sh>
@@ -1039,7 +1044,7 @@ __global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
   for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
-  w.m_run = -INFINITY;
+  w.m_run = kLowestOffset;
   w.thr = -INFINITY;
   w.l_run = 0.f;
   w.l_p = 0.f;
@@ -1320,7 +1325,7 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
-  w.m_run = -INFINITY;
+  w.m_run = kLowestOffset;
   w.thr = -INFINITY;
   w.l_run = 0.f;
   w.l_p = 0.f;
