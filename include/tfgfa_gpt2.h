@@ -84,7 +84,9 @@ int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_scale, const f
  *   y = GELU(x w^T + bias) as PLANES       (3, M, N) bf16          gelu_planes = 1 (no residual)
  *   x  (3, M, K) bf16 PLANES    w  (N, K) float32    bias  (N) or NULL    residual  (M, N) or NULL
  * Every product is that of the float32 values to 2^-26 of itself, sums are float32: as close to the
- * exact result as a float32 GEMM.  Infinities, NaN and overflow give what they give there.
+ * exact result as a float32 GEMM.  A sum that is not finite is computed again from float32 products, so
+ * infinities, NaN and overflow give what they give there.  An operand below 2^-103 in magnitude is
+ * taken to an absolute 2^-125: its lower pieces leave bf16's normal range.
  * splits: 1..TFGPT2_MAX_K_SPLITS partial sums of the contraction, tfgpt2_linear_planes_splits' choice
  * for a device of cu_count CUs (0: sizes not taken: N a multiple of 4, K of 32, planes and weights
  * below 2 GiB).  part: splits * M * N floats (NULL for one split); the partial sums are

@@ -240,6 +240,26 @@ def test_linear_planes_passes_infinities_as_float32_does(splits):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("splits", [1, 3])
+def test_linear_planes_results_at_the_top_of_the_range(splits):
+    """Results within 2^-8 of the largest float, of operands whose first bf16 pieces round up past it:
+    finite, and to F32 of the float64 result, as float32 products give them; past the range infinite."""
+    from custom_flash_attn import gpt2
+
+    M, N, K = 5, 8, 96
+    x, w = torch.zeros(M, K, device=DEV), torch.zeros(N, K, device=DEV)
+    x[0, 0], x[1, 0], x[2, 40], x[3, 0], x[4, 95] = 1.9999, -1.9999, 2 - 2.0 ** -20, 2.0, 1.5
+    w[1::2, :] = 2.0 ** 127
+    w[2, :] = 2.0 ** 127 - 2.0 ** 106
+    ref = (x.double() @ w.double().t().contiguous()).float()
+    got = gpt2.linear_planes(_to_planes(x), w, None, splits)
+    assert ref[0].isfinite().all() and ref[3, 1].isinf() and ref[:3].abs().max() > 3.4e38
+    assert torch.equal(got.isfinite(), ref.isfinite()) and not got.isnan().any()
+    fin = ref.isfinite()
+    assert _rel(got[fin].double() * 2.0 ** -64, ref[fin].double() * 2.0 ** -64) <= F32
+
+
+@pytest.mark.gpu
 def test_planes_hold_the_top_of_the_float_range():
     """A norm's result that is finite but rounds to infinity as bf16 comes back from its planes exactly."""
     from custom_flash_attn import gpt2

@@ -258,7 +258,9 @@ __device__ __forceinline__ i32x4 advance(i32x4 desc, int bytes) {
 
 // Four outputs n.. of row m over the contraction's k0..k1 with the products in float32.  Infinities in
 // x or w, weights at the top of the float range and overflow meet NaN in the split products where a
-// float32 GEMM need not (inf - inf, inf * 0), so a NaN sum is computed again; ordinary values never are.
+// float32 GEMM need not (inf - inf, inf * 0), and a product of first pieces that were rounded up is
+// infinite where the float32 one is within 2^-8 of the range's top, so a sum that is not finite is
+// computed again; ordinary values never are.
 // Ends early where all four are NaN in float32 too (a NaN in x, or in every weight row).
 __device__ __forceinline__ f32x4 plain_sums(const __bf16* X, const float* W, int M, int K, int m, int n,
                                             int k0, int k1) {
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(512, 2) void linear_planes_kernel(
       f32x4 v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = acc[b][4 * g + e] + low[b][4 * g + e];
-      if (__builtin_isnan((v[0] + v[1]) + (v[2] + v[3])))  // (also of opposite infinities: the same again)
+      if (!__builtin_isfinite((v[0] + v[1]) + (v[2] + v[3])))  // (also of four large ones: the same again)
         v = plain_sums(X, W, M, K, m, n, s0 * 32, (s0 + ns) * 32);
       if (kMode != kPartial && bias != nullptr) v += load4(bias + n);
       if (kMode == kGeluPlanes) {
