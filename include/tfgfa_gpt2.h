@@ -8,7 +8,8 @@
  *
  * Conventions as in tfgfa.h: device pointers, the caller owns every buffer, launches are
  * asynchronous on `hip_stream`, arguments are checked before any HIP call; 0 on success, > 0
- * an invalid argument (TFGFA_ERR_*), < 0 a negated hipError_t.  Tensors are contiguous and 16-byte
+ * an invalid argument (TFGFA_ERR_*; TFGFA_ERR_TOO_LARGE past one launch's threads), < 0 a negated
+ * hipError_t.  Tensors are contiguous and 16-byte
  * aligned.  Row counts of 0 launch nothing.
  */
 #ifndef TFGFA_GPT2_H
@@ -25,6 +26,11 @@ extern "C" {
 #define TFGPT2_MAX_NORM_DIM 2048
 #define TFGPT2_MAX_ROWS     8
 #define TFGPT2_MAX_CASTS    10
+/* One launch takes fewer than 2^32 threads: the most rows of a norm (a wave each), values of a GELU or of
+ * one call's casts (four a thread), outputs of a few-row projection with a norm (64 threads an output). */
+#define TFGPT2_MAX_NORM_ROWS 67108863LL
+#define TFGPT2_MAX_VALUES    17179868160LL
+#define TFGPT2_MAX_OUTPUTS   67108860
 /* Most splits of the contraction of tfgpt2_linear_planes. */
 #define TFGPT2_MAX_K_SPLITS 8
 

@@ -83,6 +83,40 @@ def test_kernel_arguments_are_checked_before_any_hip_call():
         _C.gpt2_linear_rows(P, False, 0, 0, 0.0, [(P + 4, 0, P)], False, 0, False, 1, 4, 64, 0)
 
 
+def test_sizes_past_one_launch_are_refused_before_any_hip_call():
+    """HIP launches fewer than 2^32 threads: past that the entry points say so, and the modules keep
+    their torch operators (sizes of meta tensors only)."""
+    from custom_flash_attn import gpt2
+
+    P, big = 0x10000, "launch limits"
+    assert gpt2.MAX_NORM_ROWS * 64 < 2 ** 32 <= (gpt2.MAX_NORM_ROWS + 1) * 64
+    with pytest.raises(RuntimeError, match=big):
+        _C.gpt2_layernorm(P, 0, 0, P, P, P, 0, gpt2.MAX_NORM_ROWS + 1, 4, 1e-5, 0)
+    with pytest.raises(RuntimeError, match=big):
+        _C.gpt2_gelu(P, P, gpt2.MAX_VALUES + 1, 0)
+    with pytest.raises(RuntimeError, match=big):
+        _C.gpt2_cast_bf16([(P, P, gpt2.MAX_VALUES), (P, P, 4)], 0)
+    for K, norm in ((64, P), (64, 0), (8192, 0)):
+        N = 4 * (2 ** 32 // (256 if norm else 512 if K <= 4096 else 1024))
+        with pytest.raises(RuntimeError, match=big):
+            _C.gpt2_linear_rows(P, False, norm, norm, 0.0, [(P, 0, P)], False, 0, False, 1, N, K, 0)
+    norm = mi.LayerNorm({"emb_dim": 4}).to("meta")
+    assert norm._native(torch.empty(gpt2.MAX_NORM_ROWS, 4, device="meta"))
+    assert not norm._native(torch.empty(gpt2.MAX_NORM_ROWS + 1, 4, device="meta"))
+    assert gpt2.rows_fit(1, _C.GPT2_MAX_OUTPUTS, False) and not gpt2.rows_fit(1, _C.GPT2_MAX_OUTPUTS + 4, False)
+
+
+@pytest.mark.gpu
+def test_values_past_one_launch_stay_with_torch(monkeypatch):
+    from custom_flash_attn import gpt2
+
+    x = torch.ones(8, device=DEV)
+    assert gpt2.takes(x)
+    monkeypatch.setattr(gpt2, "MAX_VALUES", 7)
+    assert not gpt2.takes(x)
+    torch.testing.assert_close(mi.GELU()(x), torch.nn.functional.gelu(x, approximate="tanh"))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,d", [(1, 4), (3, 252), (4, 256), (5, 260), (7, 768), (2, 1024), (3, 1028),
                                     (9, 1600), (1, 2048)])

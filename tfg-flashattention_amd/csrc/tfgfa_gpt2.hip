@@ -634,6 +634,9 @@ __global__ __launch_bounds__(64 * kW) void linear_rows_kernel(
 
 static bool misaligned(const void* p) { return ((uintptr_t)p & 15u) != 0; }
 
+// A launch of `blocks` workgroups of `threads` threads is past HIP's limit: 2^32 - 1 threads.
+static bool too_many(long long blocks, int threads) { return blocks > (long long)UINT32_MAX / threads; }
+
 static int launched() {
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? TFGFA_OK : -(int)e;
@@ -680,6 +683,12 @@ static int choose_k_splits(long long tiles, int steps, int cu_count) {
   return best;
 }
 
+// Either launch of a linear on planes is past HIP's limit.
+static bool planes_too_large(long long tiles, int M, int N, int S) {
+  return too_many((tiles * S + 7) / 8 * 8, 512) ||
+         (S > 1 && too_many(((long long)M * N / 4 + 255) / 256, 256));
+}
+
 struct RowsArgs {
   const void* x;
   const float* ln_scale;
@@ -709,6 +718,7 @@ static void launch_rows_norm(const RowsArgs& a, int parts, hipStream_t stream) {
 
 // Without: the fewest waves and strips that take the width in one batch, up to 8192; wider ones
 // loop.
+static int plain_waves(int K) { return K <= 4096 ? 8 : 16; }
 template <int kG, typename X>
 static void launch_rows_plain(const RowsArgs& a, int parts, hipStream_t stream) {
   if (a.K <= 1024)
@@ -745,7 +755,7 @@ extern "C" int tfgpt2_layernorm(const float* x, const void* delta, float* sum, c
   if (rows < 0 || d < 4 || d > TFGPT2_MAX_NORM_DIM || (d & 3)) return TFGFA_ERR_BAD_SHAPE;
   if (y_kind < TFGPT2_F32 || y_kind > TFGPT2_PLANES) return TFGFA_ERR_DTYPE;
   if (rows == 0) return TFGFA_OK;
-  if (rows > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
+  if (too_many(rows, 64)) return TFGFA_ERR_TOO_LARGE;
   if (!x || !scale || !shift || !y || (delta != nullptr && sum == nullptr)) return TFGFA_ERR_NULL_POINTER;
   if (misaligned(x) || misaligned(delta) || misaligned(sum) || misaligned(scale) ||
       misaligned(shift) || misaligned(y))
@@ -764,7 +774,7 @@ extern "C" int tfgpt2_gelu(const float* x, float* y, int64_t n, void* hip_stream
   if (n < 0) return TFGFA_ERR_BAD_SHAPE;
   if (n == 0) return TFGFA_OK;
   const long long blocks = (n + 4LL * kGeluThreads - 1) / (4LL * kGeluThreads);
-  if (blocks > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
+  if (too_many(blocks, kGeluThreads)) return TFGFA_ERR_TOO_LARGE;
   if (!x || !y) return TFGFA_ERR_NULL_POINTER;
   if (misaligned(x) || misaligned(y)) return TFGFA_ERR_ALIGNMENT;
   hipLaunchKernelGGL(gelu_kernel, dim3((unsigned)blocks), dim3(kGeluThreads), 0,
@@ -790,7 +800,7 @@ extern "C" int tfgpt2_cast_bf16(int count, const float* const* src, void* const*
   }
   a.count = count;
   const long long blocks = (units + kCastThreads - 1) / kCastThreads;
-  if (blocks > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
+  if (too_many(blocks, kCastThreads)) return TFGFA_ERR_TOO_LARGE;
   if (blocks == 0) return TFGFA_OK;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(kCastThreads), 0,
                      (hipStream_t)hip_stream, a);
@@ -815,7 +825,7 @@ extern "C" int tfgpt2_linear_rows(const void* x, int x_bf16, const float* ln_sca
   if ((y_bf16 && (!ln || gelu)) || (gelu && !ln)) return TFGFA_ERR_DTYPE;
   if (M == 0) return TFGFA_OK;
   const long long tiles = ((long long)N + kTileRows - 1) / kTileRows;
-  if (tiles * parts > INT32_MAX) return TFGFA_ERR_TOO_LARGE;
+  if (too_many(tiles * parts, 64 * (ln ? kNormWaves : plain_waves(K)))) return TFGFA_ERR_TOO_LARGE;
   if (!x || !w || !bias || !y) return TFGFA_ERR_NULL_POINTER;
   RowsArgs a = {};
   for (int p = 0; p < parts; ++p) {
@@ -848,9 +858,10 @@ extern "C" int tfgpt2_linear_planes_splits(int M, int N, int K, int cu_count) {
   using namespace tfgpt2;
   if (M < 1 || N < 4 || (N & 3) || K < 32 || K % 32 || cu_count < 1) return 0;
   if (3LL * M * K * 2 > INT32_MAX || (long long)N * K * 4 > INT32_MAX) return 0;
-  const long long tiles = (long long)((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile);
-  if (tiles * TFGPT2_MAX_K_SPLITS > INT32_MAX / 2) return 0;
-  return choose_k_splits(tiles, K / 32, cu_count);
+  const long long tiles = (((long long)M + kTile - 1) / kTile) * (((long long)N + kTile - 1) / kTile);
+  const int S = choose_k_splits(tiles, K / 32, cu_count);
+  if (planes_too_large(tiles, M, N, S)) return planes_too_large(tiles, M, N, 1) ? 0 : 1;
+  return S;
 }
 
 extern "C" int tfgpt2_linear_planes(const void* x, const float* w, const float* bias, int gelu_planes,
@@ -866,9 +877,10 @@ extern "C" int tfgpt2_linear_planes(const void* x, const float* w, const float* 
   if (misaligned(x) || misaligned(w) || misaligned(bias) || misaligned(residual) || misaligned(y) ||
       misaligned(part))
     return TFGFA_ERR_ALIGNMENT;
-  const int tm = (M + kTile - 1) / kTile, tn = (N + kTile - 1) / kTile;
+  const int tm = ((long long)M + kTile - 1) / kTile, tn = ((long long)N + kTile - 1) / kTile;
   const int steps = (K / 32 + splits - 1) / splits;
   const int S = (K / 32 + steps - 1) / steps;  // no split without a step
+  if (planes_too_large((long long)tm * tn, M, N, S)) return TFGFA_ERR_TOO_LARGE;
   const dim3 grid((unsigned)((tm * tn * S + 7) / 8 * 8));
   const hipStream_t stream = (hipStream_t)hip_stream;
   const __bf16* xp = static_cast<const __bf16*>(x);

@@ -313,6 +313,9 @@ PYBIND11_MODULE(_C, m) {
   m.attr("GPT2_PLANES") = TFGPT2_PLANES;
   m.attr("GPT2_MAX_NORM_DIM") = TFGPT2_MAX_NORM_DIM;
   m.attr("GPT2_MAX_ROWS") = TFGPT2_MAX_ROWS;
+  m.attr("GPT2_MAX_NORM_ROWS") = TFGPT2_MAX_NORM_ROWS;
+  m.attr("GPT2_MAX_VALUES") = TFGPT2_MAX_VALUES;
+  m.attr("GPT2_MAX_OUTPUTS") = TFGPT2_MAX_OUTPUTS;
   m.def("device_info", &device_info, "CU count, shader clock (MHz) and arch of the current device");
   m.def("strerror", [](int st) { return std::string(tfgfa_strerror(st)); });
   m.def("abi_version", []() { return tfgfa_abi_version(); });

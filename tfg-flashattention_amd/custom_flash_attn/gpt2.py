@@ -12,6 +12,8 @@ from . import _C, _launch_on
 
 MAX_NORM_DIM = _C.GPT2_MAX_NORM_DIM
 MAX_ROWS = _C.GPT2_MAX_ROWS
+MAX_NORM_ROWS = _C.GPT2_MAX_NORM_ROWS
+MAX_VALUES = _C.GPT2_MAX_VALUES
 _NORM_LDS_FLOATS = 15360  # rows * (width + 4) of a projection with a norm before it
 _TYPES = (torch.Tensor, torch.nn.Parameter)
 
@@ -27,10 +29,10 @@ def eager() -> bool:
 
 
 def takes(x: torch.Tensor, *params, dtypes=(torch.float32,)) -> bool:
-    """``x`` (of one of ``dtypes``) and the float32 ``params`` (None allowed) are plain, contiguous,
-    16-byte aligned tensors on one GPU and need no gradient."""
+    """``x`` (of one of ``dtypes``, of at most one launch's values) and the float32 ``params`` (None
+    allowed) are plain, contiguous, 16-byte aligned tensors on one GPU and need no gradient."""
     if not (type(x) in _TYPES and x.is_cuda and x.dtype in dtypes and x.is_contiguous()
-            and x.data_ptr() % 16 == 0):
+            and x.data_ptr() % 16 == 0 and x.numel() <= MAX_VALUES):
         return False
     dev, grad = x.device, torch.is_grad_enabled()
     if grad and x.requires_grad:
@@ -100,8 +102,8 @@ def cast_bf16(pairs) -> None:
 
 
 def rows_fit(rows: int, width: int, norm: bool) -> bool:
-    """Whether :func:`linear_rows` takes ``rows`` rows of ``width`` values."""
-    return (1 <= rows <= MAX_ROWS and width % 4 == 0 and width >= 4
+    """Whether :func:`linear_rows` takes ``rows`` rows of ``width`` values, and gives as many."""
+    return (1 <= rows <= MAX_ROWS and width % 4 == 0 and 4 <= width <= _C.GPT2_MAX_OUTPUTS
             and (not norm or (width <= MAX_NORM_DIM and rows * (width + 4) <= _NORM_LDS_FLOATS)))
 
 

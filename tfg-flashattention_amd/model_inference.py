@@ -170,6 +170,7 @@ class MultiHeadAttention(nn.Module):
         wq, wk, wv, wo = self.W_query, self.W_key, self.W_value, self.out_proj
         rows, cols = wq.weight.shape
         return (x.dim() == 3 and x.shape[2] == cols and rows % 8 == 0 and cols % 8 == 0
+                and x.numel() + 4 * rows * (cols + 1) <= g.MAX_VALUES
                 and wk.weight.shape == wv.weight.shape == (rows, cols) and wo.weight.shape == (rows, rows)
                 and (wq.bias is None) == (wk.bias is None) == (wv.bias is None)
                 and g.takes(x, *(t for m in (wq, wk, wv, wo) for t in (m.weight, m.bias)),
@@ -333,9 +334,9 @@ class LayerNorm(nn.Module):
         self.shift = nn.Parameter(torch.zeros(config["emb_dim"]))
 
     def _native(self, x) -> bool:
-        d = x.shape[-1] if x.dim() else 0
-        return (d % 4 == 0 and 4 <= d <= _gpt2().MAX_NORM_DIM and self.scale.shape == (d,)
-                and self.shift.shape == (d,))
+        g, d = _gpt2(), x.shape[-1] if x.dim() else 0
+        return (d % 4 == 0 and 4 <= d <= g.MAX_NORM_DIM and x.numel() <= d * g.MAX_NORM_ROWS
+                and self.scale.shape == (d,) and self.shift.shape == (d,))
 
     def forward(self, x):
         g = _gpt2() if x.is_cuda else None
