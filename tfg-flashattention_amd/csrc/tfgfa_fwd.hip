@@ -118,9 +118,11 @@ constexpr int kOutOfRange = 0x7FFFFFF0;
 // *as rounded* for the P.V MFMA, so the rounding of a dominant probability cancels between O's
 // numerator and denominator; the LSE uses l_run, the fp32 sum of the unrounded ones.
 
-// Offset of a row that has seen no score above -inf: finite, so that scores of -inf (q.k past the
-// float range, infinite keys) give probabilities of 0 wherever a wave's or a group's first ones
-// stand, and a merge weighs such a state by 0; a row with no other score is 0 / 0.
+// An offset moves off its first value, -inf, to no less than this: finite, so that scores of -inf (q.k
+// past the float range, infinite keys) give probabilities of 0 wherever a wave's or a group's
+// first ones stand, and a merge weighs such a state by 0; a row with no other score is 0 / 0.  (Starting
+// at this value instead costs 0.3-0.6%: from -inf the compiler knows that the first half moves
+// the offset, and leaves its first probabilities out.)
 constexpr float kLowestOffset = -0x1.fffffep127f;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -439,13 +441,12 @@ __device__ __forceinline__ float lane_max(const WaveState<Sh>& w) {
 // Moves the exp2 offset of every row to its exact running max, rescaling O and the sums, when
 // some lane's score exceeds its row's offset by more than the margin (wave-uniform branch, taken
 // at a wave's first half and then rarely).  Every computed half has an unmasked key in every
-// row (it starts at or below the wave's first row), so the first half with a score above -inf moves
-// m_run off kLowestOffset.
+// row (it starts at or below the wave's first row); the first half always moves m_run off -inf.
 template <class Sh>
 __device__ __forceinline__ void move_offset(WaveState<Sh>& w, float mx, float scale_log2,
                                             float inv_scale_log2) {
-  if (__builtin_amdgcn_ballot_w64(mx > w.thr) != 0) {
-    const float m_new = fmaxf(w.m_run, pair_max(mx) * scale_log2);
+  if (__builtin_amdgcn_ballot_w64(mx >= w.thr) != 0) {  // thr starts at -inf, where mx may be
+    const float m_new = fmaxf(fmaxf(w.m_run, kLowestOffset), pair_max(mx) * scale_log2);
     const float alpha = __builtin_amdgcn_exp2f(w.m_run - m_new);
     w.m_run = m_new;
     w.thr = (m_new + Elem<typename Sh::T>::kMargin) * inv_scale_log2;
@@ -524,7 +525,7 @@ __device__ __forceinline__ typename Elem<typename Sh::T>::v8 k_operand(const Wav
 //                    the sums of P_u and its conversion to the element type
 // The offset check reads the lane's running sum l_p with this half's probabilities, as rounded
 // to the element type, added.  bf16: a rounded P above 2^64 makes that sum exceed the bound (an
-// overflow gives +inf, and so does the first offset, kLowestOffset, with any score above -inf), so a sum above
+// overflow gives +inf, a -inf offset on a wave's first half gives +inf or NaN), so a sum above
 // the bound, or not a number, takes the rare branch: move the offset to the rows' exact running
 // max, rescale O and the sums, recompute P_u.  A sum above the bound without any single P above
 // it moves the offset early, which is harmless (after a move every P is at most 1, so l_p stays
@@ -598,7 +599,7 @@ __device__ __forceinline__ void fused_step(WaveState<Sh>& w, const Lds& lds, flo
       // the sum does, is +inf or is a NaN (the device pass assumes no NaN in float compares).
       if (__builtin_amdgcn_ballot_w64(__float_as_uint(hs) > __float_as_uint(kSumBound)) != 0) {
         const float mx = lane_max(w);
-        const float m_new = fmaxf(w.m_run, pair_max(mx) * scale_log2);
+        const float m_new = fmaxf(fmaxf(w.m_run, kLowestOffset), pair_max(mx) * scale_log2);
         const float alpha = __builtin_amdgcn_exp2f(w.m_run - m_new);
         w.m_run = m_new;
         w.thr = (m_new + Elem<T>::kMargin) * inv_scale_log2;
@@ -809,8 +810,8 @@ struct Strides {
 // rule (offset m_w, rounded-probability sum lp_w, fp32 sum l_w, unnormalised O_w):
 //   M = max_w m_w,  a_w = 2^(m_w - M),  O = sum_w a_w O_w / sum_w a_w lp_w,
 //   LSE = (M + log2 sum_w a_w l_w) ln 2.
-// A wave with no half, or with scores of -inf only, has m_w = kLowestOffset and sums of 0: a_w = 0
-// beside any other.
+// A wave with no half contributes m_w = -inf, one with scores of -inf only kLowestOffset and sums of 0:
+// a_w = 0 beside any other.
 // A wave's partial: its unnormalised O rows (fp32, row-major, 64 * kDH columns, 16-B chunk c of
 // row r at physical chunk c ^ (r % (16 kDH))) and its row statistics.
 template <class Sh>
@@ -1044,7 +1045,7 @@ __global__ __launch_bounds__(64 * Sh::kWaves, Sh::kSimdWaves) void fwd_kernel(
   for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
-  w.m_run = kLowestOffset;
+  w.m_run = -INFINITY;
   w.thr = -INFINITY;
   w.l_run = 0.f;
   w.l_p = 0.f;
@@ -1325,7 +1326,7 @@ __global__ __launch_bounds__(SplitLayout<Sh>::kWaves * 64, 1) void fwd_split_ker
   for (int i = 0; i < Sh::kOT; ++i)
 #pragma unroll
     for (int t = 0; t < 16; ++t) w.o[i][t] = 0.f;
-  w.m_run = kLowestOffset;
+  w.m_run = -INFINITY;
   w.thr = -INFINITY;
   w.l_run = 0.f;
   w.l_p = 0.f;
@@ -1591,8 +1592,11 @@ static void launch_plan(const LaunchArgs& a, Plan plan, hipStream_t stream) {
       launch_instance<Shape<kD, T, kMaskD, kLse, 2, 2>, kDense>(a, stream);
       break;
     case Plan::kGroups4:
-      if constexpr (kD <= kDHalf) launch_instance<Shape<kD, T, kMaskD, kLse, 2, 4>, kDense>(a, stream);
-      break;
+      if constexpr (kD <= kDHalf) {
+        launch_instance<Shape<kD, T, kMaskD, kLse, 2, 4>, kDense>(a, stream);
+        break;
+      }
+      [[fallthrough]];  // never chosen past 64 head dims, where it is not compiled
     case Plan::kWhole:
       launch_instance<Shape<kD, T, kMaskD, kLse>, kDense>(a, stream);
       break;
