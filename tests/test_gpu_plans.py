@@ -1,6 +1,6 @@
 """The forward's key-split workgroups and head-dim instances at the sizes where they can go wrong:
 ends of 32-key halves, 64-key tiles and query blocks, groups without a tile, head dims at the edges
-of the compiled ones (GPU box only).  Each shape's comment names the kernel it reaches on 256 CUs.
+of the compiled ones (GPU box only).
 
 Reference: float32 attention from the same 16-bit values.  With u the unit roundoff of the type
 (2^-8 bf16, 2^-11 fp16), the probabilities, their sum and the output are each rounded once:
@@ -19,36 +19,64 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 U = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 
-#        B, H, Nq, Nk, causal
-NARROW = [  # head dims up to 64
-    (1, 1, 1025, 1025, True),    # 2 row waves x 4 key groups, one row past a block
-    (1, 2, 33, 1100, False),     # the same, unmasked, a ragged last tile
-    (1, 1, 1300, 1090, True),    # the same, rows past the last key
-    (1, 256, 65, 1, True),       # 2 x 2: one key, the second group without a tile
-    (1, 130, 100, 100, True),
-    (1, 200, 96, 96, True),
-    (2, 65, 127, 127, True),
-    (1, 256, 5, 1100, False),    # 4 x 2, unmasked
-    (1, 150, 127, 1056, False),
-    (1, 20, 2049, 2049, True),   # 4 x 2, causal
-    (1, 130, 1, 1, True),        # 32-row blocks, 4 key waves: one row, one key
-    (1, 131, 65, 65, True),
-    (1, 60, 640, 640, True),     # whole blocks
-    (1, 44, 641, 641, True),
-]
-WIDE = [  # head dims past 64
-    (1, 3, 130, 130, True),      # 32-row blocks, 4 key waves
-    (1, 70, 65, 65, True),
-    (1, 200, 3, 705, False),
-    (1, 180, 34, 34, True),      # 2 x 2
-    (1, 140, 33, 65, True),
-    (1, 192, 65, 33, True),
-    (1, 25, 600, 97, True),
-    (1, 35, 700, 700, True),     # 4 x 2
-    (1, 200, 100, 705, False),
-    (1, 20, 2049, 2049, True),
-    (1, 130, 200, 130, False),   # whole blocks
-]
+# The kernel each (B, H, Nq, Nk, causal) reaches on 256 CUs (checked in test_plan_cpu.py).
+NARROW_PLANS = {  # head dims up to 64
+    "kGroups4": [                  # 2 row waves x 4 key groups
+        (1, 1, 1025, 1025, True),  # one row past a block
+        (1, 2, 33, 1100, False),   # unmasked, a ragged last tile
+        (1, 1, 1300, 1090, True),  # rows past the last key
+        (1, 256, 5, 1100, False),
+    ],
+    "kPairs": [                    # 2 x 2: a causal call's first block has one tile, its second group none
+        (1, 100, 200, 200, True),
+        (1, 60, 321, 500, True),
+        (1, 21, 1153, 1153, True),
+    ],
+    "kGroups2": [                  # 4 x 2
+        (1, 150, 127, 1056, False),
+        (1, 20, 2049, 2049, True),
+    ],
+    "kHalves": [                   # 32-row blocks, 4 key waves
+        (1, 130, 1, 1, True),      # one row, one key
+        (1, 131, 65, 65, True),
+        (1, 40, 97, 130, False),
+        (1, 25, 700, 700, True),   # more than one round
+    ],
+    "kWhole": [
+        (1, 256, 65, 1, True),
+        (1, 130, 100, 100, True),
+        (1, 200, 96, 96, True),
+        (2, 65, 127, 127, True),
+        (1, 60, 640, 640, True),
+        (1, 44, 641, 641, True),
+    ],
+}
+WIDE_PLANS = {  # head dims past 64
+    "kHalves": [
+        (1, 3, 130, 130, True),
+        (1, 70, 65, 65, True),
+        (1, 200, 3, 705, False),
+    ],
+    "kPairs": [
+        (1, 20, 703, 703, True),
+        (1, 180, 34, 300, False),
+        (1, 150, 64, 993, False),
+    ],
+    "kGroups2": [
+        (1, 35, 700, 700, True),
+        (1, 200, 100, 705, False),
+        (1, 20, 2049, 2049, True),
+    ],
+    "kWhole": [
+        (1, 180, 34, 34, True),
+        (1, 140, 33, 65, True),
+        (1, 192, 65, 33, True),
+        (1, 25, 600, 97, True),
+        (1, 130, 200, 130, False),
+    ],
+}
+NARROW = [s for shapes in NARROW_PLANS.values() for s in shapes]
+WIDE = [s for shapes in WIDE_PLANS.values() for s in shapes]
 
 
 def _reference(q, k, v, causal):

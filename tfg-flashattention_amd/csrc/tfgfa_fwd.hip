@@ -18,7 +18,7 @@
 //   Where that leaves CUs idle (small batches), the same kernel runs with kS key groups of kR row
 //   waves: group g takes tiles g, g + kS, .. through a K/V ring of its own, and the groups' softmax
 //   states merge through LDS at the end; the grids too small even for that run fwd_split_kernel.
-//   choose_plan holds the lines between them and the times they rest on.
+//   tfgfa_plan.h holds the lines between them and the times they rest on.
 //
 // Per-wave software pipeline (32-key halves u = 0, 1, ...)
 //   half-step u:  O += V_{u-1} P_{u-1}   interleaved with   P_u = exp2(S_u - m)
@@ -81,12 +81,12 @@
 #include <stdint.h>
 #include <string.h>
 
-#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
 #include "tfgfa.h"
 #include "tfgfa_device.h"
+#include "tfgfa_plan.h"
 
 namespace tfgfa {
 
@@ -1485,72 +1485,6 @@ static int validate(const void* q, const void* k, const void* v, const void* o, 
   return TFGFA_OK;
 }
 
-// Which kernel runs a problem.  A grid that leaves CUs idle, or fills them once, takes as long as
-// its longest wave's chain of half-steps (N/32 of them, ~0.4 us each whatever runs beside them);
-// splitting the keys over several waves shortens the chain, at the price of a merge and, where
-// fewer than 4 waves share a K/V tile, of more traffic from the L2.
-//   kWhole    fwd_kernel, 4 row waves, one group: the most work per byte, three workgroups a CU
-//   kGroups2  4 row waves x 2 key groups (128 rows, 8 waves)
-//   kPairs    2 row waves x 2 key groups (64 rows, 4 waves)
-//   kGroups4  2 row waves x 4 key groups (64 rows, 8 waves), head dims up to 64
-//   kHalves   fwd_split_kernel: one 32-row block, 4 waves
-// The lines below are where the measured times cross on 256 CUs (bf16, us, graph replays; N x N
-// causal unless marked; "blocks" are 128-row query blocks, h the longest chain):
-//   D = 64                       blocks   h   kWhole kHalves kGroups2 kPairs kGroups4
-//     B1 H12 N512                   48   16     9.1    6.0      8.6     7.0     6.7
-//     B1 H16 N1024                 128   32    14.5    9.3     12.5    10.0     9.4
-//     B1 H8 N2048                  128   64    25.3   15.7     20.4    16.1    14.1
-//     B1 H12 N2048                 192   64    25.9   19.2     20.9    17.1    16.2
-//     B2 H16 N777                  224   25    12.0   10.9     10.8     8.8    11.6
-//     B1 H16 N2048                 256   64    25.9   23.8     21.4    18.0    18.5
-//     B8 H12 N136 (480 row blocks) 192    5            5.2              6.0
-//     B8 H16 N200 (896 row blocks) 256    7     6.4    7.3      6.8     6.0     9.3
-//     B2 H16 1000 x 1333 unmasked  256   42    19.2   27.8     17.2    18.2    22.2
-//     B4 H16 500 x 300 unmasked    256   10     7.7   11.9      8.2     8.2    12.2
-//     B3 H12 N1024                 288   32    16.1   17.3     13.7    13.1    17.9
-//     B4 H20 N512                  320   16    10.3   12.9     11.8    11.5    15.0
-//     B2 H25 N1024                 400   32    16.9   23.1     18.2    20.0    25.9
-//     B1 H25 N2048                 400   64    29.0   42.8     25.6    30.1    36.3
-//     B1 H16 N4096                 512  128    52.7   70.2     45.9    48.5    55.4
-//     B1 H16 N8192                1024  256   148.0  251.6    158.2   161.6   185.6
-//   D = 128 (80 where marked); row blocks of 32: kHalves takes one workgroup a CU
-//     B4 H20 N57 (160 row blocks)   80    2            5.7              7.8
-//     B1 H25 320 x 162 unm. (250)   75    6            6.4              7.8
-//     B1 H16 N625 (320)             80   20           11.5             12.8
-//     B1 H16 N300                   48   10     9.6    7.8     10.8     8.8
-//     B1 H12 N1024                  96   32    21.2   16.3     20.0    16.7
-//     B2 H16 300 x 700 unmasked     96   22    15.8   22.8     16.2    13.6
-//     B1 H25 N600                  125   19    15.4   17.0     14.6    14.1
-//     B8 H12 N233 (384 of 64 rows) 192    8    10.6   13.7              15.1
-//     B1 H12 N2048                 192   64    36.2   45.2     31.9    27.0
-//     B1 H25 N1024                 200   32    22.5   36.1     21.7    23.5
-//     B2 H16 1000 x 1333 unm., 80  256   42    23.7   59.1     22.8    33.6
-//     B4 H16 N500                  256   16    14.7   24.0     15.0    17.8
-//     B1 H12 N3000, 80             288   94    45.4   72.4     38.2    46.7
-//     B2 H25 N1024                 400   32    26.9   68.8     29.9    45.4
-//     B1 H16 N4096                 512  128    85.9  186.2     76.3   105.6
-// The choice depends on the sizes only, never on strides or outputs, so every instance of one
-// problem takes the same arithmetic.
-enum class Plan { kWhole, kHalves, kGroups2, kPairs, kGroups4 };
-static Plan choose_plan(long long heads, int cu_count, int Nq, int Nk, int D, int causal) {
-  const int h = ((causal ? std::min(Nq, Nk) : Nk) + 31) / 32;
-  const long long cu = cu_count;
-  const long long blocks = heads * ((Nq + kBlockRows - 1) / kBlockRows);
-  const long long row_blocks = heads * ((Nq + kWaveRows - 1) / kWaveRows);  // kHalves' grid
-  if (causal && blocks > cu && blocks <= 2 * cu && h >= 64) return Plan::kGroups2;
-  if (D <= kDHalf) {
-    if (row_blocks <= 2 * cu && h <= 32) return Plan::kHalves;  // one round, two workgroups a CU
-    if (2 * blocks <= cu) return Plan::kGroups4;
-    if (!causal) return blocks <= cu && h >= 32 ? Plan::kGroups2 : Plan::kWhole;
-    if (blocks <= cu) return h >= 64 && 4 * blocks <= 3 * cu ? Plan::kGroups4 : Plan::kPairs;
-    return 4 * blocks <= 5 * cu && h >= 22 ? Plan::kPairs : Plan::kWhole;
-  }
-  if (row_blocks <= cu || (causal && 2 * row_blocks <= 3 * cu && h >= 16)) return Plan::kHalves;
-  // kPairs, one workgroup a CU: in one round, or with chains that outweigh the second.
-  if (4 * blocks <= 3 * cu && (heads * ((Nq + 63) / 64) <= cu || h >= 22)) return Plan::kPairs;
-  return blocks <= cu && h >= 22 ? Plan::kGroups2 : Plan::kWhole;
-}
-
 struct LaunchArgs {
   const void *q, *k, *v;
   void* o;
@@ -1671,7 +1605,7 @@ static int launch(const void* q, const void* k, const void* v, void* o, float* l
   int cu_count = 0;
   const int ist = tfgfa_device_info(&cu_count, nullptr, nullptr, 0);
   if (ist != TFGFA_OK) return ist;
-  const Plan plan = choose_plan(a.BH, cu_count, Nq, Nk, D, causal);
+  const Plan plan = choose_plan(a.BH, cu_count, Nq, Nk, D, causal != 0);
   const hipStream_t stream = (hipStream_t)hip_stream;
   if (dtype == TFGFA_DTYPE_BF16)
     launch_dims<__bf16>(a, dense, plan, stream);

@@ -18,6 +18,7 @@
 
 #include "tfgfa.h"
 #include "tfgfa_gpt2.h"
+#include "tfgfa_plan.h"
 
 namespace py = pybind11;
 
@@ -308,6 +309,13 @@ PYBIND11_MODULE(_C, m) {
     check(tfgfa_device_info(&cu, nullptr, nullptr, 0), "tfgfa_device_info");
     return tfgpt2_linear_planes_splits(M, N, K, cu);
   });
+  m.def("fwd_plan",
+        [](long long heads, int cu_count, int Nq, int Nk, int D, bool causal) {
+          static const char* const names[] = {"kWhole", "kHalves", "kGroups2", "kPairs", "kGroups4"};
+          return names[(int)tfgfa::choose_plan(heads, cu_count, Nq, Nk, D, causal)];
+        },
+        "The kernel that runs a forward of these sizes", py::arg("heads"), py::arg("cu_count"),
+        py::arg("Nq"), py::arg("Nk"), py::arg("D"), py::arg("causal"));
   m.attr("GPT2_F32") = TFGPT2_F32;
   m.attr("GPT2_BF16") = TFGPT2_BF16;
   m.attr("GPT2_PLANES") = TFGPT2_PLANES;
