@@ -461,3 +461,22 @@ def test_last_logits_are_the_models_last_position(tokens):
         assert torch.equal(mi._last_logits(model, idx), want)
         hook.remove()
     assert seen == [tokens]
+
+
+def test_compiled_modules_are_called():
+    """A module that was compiled in place runs its compiled form: its parameters are not taken."""
+    def module(cls, *a, **kw):
+        m = cls(*a, **kw)
+        calls = []
+        m._compiled_call_impl = lambda *x, **k: (calls.append(1), m._call_impl(*x, **k))[1]  # as Module.compile sets it
+        return m, calls
+
+    cfg = dict(mi.GPT_CONFIG_124M)
+    cfg.update({"emb_dim": 64, "n_layers": 1, "n_heads": 2, "vocab_size": 50, "context_length": 64,
+                "drop_rate": 0.0, "impl_type": "manual"})
+    model, calls = module(mi.GPTModel, cfg)
+    with torch.no_grad():
+        mi._last_logits(model.eval(), torch.randint(0, 50, (1, 40)))
+    assert calls and not mi._plain(model, mi.GPTModel)
+    linear, _ = module(torch.nn.Linear, 4, 4)
+    assert not mi._plain(linear, torch.nn.Linear) and mi._plain(torch.nn.Linear(4, 4), torch.nn.Linear)

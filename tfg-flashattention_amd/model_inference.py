@@ -56,10 +56,11 @@ def _gpt2():
 
 
 def _plain(module, cls) -> bool:
-    """``module`` is a ``cls`` as this file or torch defines it, with no hook that a call of it
-    would run: a caller may then take its parameters and leave the call out."""
+    """``module`` is a ``cls`` as this file or torch defines it, with no hook and no compiled form
+    (``module.compile()``) that a call of it would run: a caller may then take its parameters and
+    leave the call out."""
     return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
-            and "forward" not in module.__dict__)
+            and "forward" not in module.__dict__ and module._compiled_call_impl is None)
 
 
 def _no_global_hooks() -> bool:
