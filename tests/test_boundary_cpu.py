@@ -4,6 +4,8 @@ Python shim's checks.  No kernel is launched: every call here returns before any
 import ctypes
 import os
 import re
+import subprocess
+import sys
 import types
 
 import pytest
@@ -615,3 +617,17 @@ def test_decode_workspace_not_cached_under_graph_capture(monkeypatch):
     assert c is d and c.numel() >= 256
     assert c is not a and c is not b  # eager calls never get a captured call's buffer
     assert list(cfa._WORKSPACES) == [(dev, 1234)]
+
+
+@pytest.mark.parametrize("missing", ["_cuda_getDevice _cuda_getCurrentRawStream", "_len_torch_dispatch_stack",
+                                     "_functorch"])
+def test_import_without_torchs_private_names(missing):
+    """A torch without one of the private names that the launch path uses: the package imports, and what
+    cannot be asked has the GPT-2 modules run their torch operators."""
+    code = (f"import torch\nfrom torch import _dynamo\nfor n in {missing!r}.split(): delattr(torch._C, n)\n"
+            "import custom_flash_attn\nfrom custom_flash_attn import gpt2\n"
+            f"assert gpt2._ANSWERS is {missing.startswith('_cuda')}\n"
+            "assert gpt2._ANSWERS or gpt2.eager() is False\n"
+            "assert callable(custom_flash_attn._current_device) and callable(custom_flash_attn._current_stream)\n")
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "tfg-flashattention_amd"))
+    subprocess.run([sys.executable, "-c", code], check=True, env=env, timeout=120)

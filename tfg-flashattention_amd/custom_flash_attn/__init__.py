@@ -38,9 +38,11 @@ MAX_HEAD_DIM = 128  # attention() / flash_attn_forward(): any head dim up to 128
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
 
-# The current device and a device's current stream as plain integers.
-_current_device = torch._C._cuda_getDevice
-_current_stream = torch._C._cuda_getCurrentRawStream
+# The current device and a device's current stream as plain integers: torch's own short ways, or, in a
+# torch without them, its public functions.
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+_current_stream = getattr(torch._C, "_cuda_getCurrentRawStream",
+                          lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _launch_on(index: int, launch, *args) -> None:

@@ -18,11 +18,23 @@ _NORM_LDS_FLOATS = 15360  # rows * (width + 4) of a projection with a norm befor
 _TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
+def _has(obj, path: str) -> bool:
+    for name in path.split("."):
+        obj = getattr(obj, name, None)
+    return obj is not None
+
+
+# What eager() asks torch; a torch without one of them has the modules run its operators.
+_ANSWERS = _has(forward_ad, "_current_level") and all(_has(torch, n) for n in (
+    "compiler.is_compiling", "_C._get_tracing_state", "_C._len_torch_dispatch_stack",
+    "_C._len_torch_function_stack", "_C._functorch.peek_interpreter_stack"))
+
+
 def eager() -> bool:
     """No tracing, compilation, function transform, forward-mode level or torch mode is active, so
     a kernel launched on raw pointers is what the torch operators would have been."""
     C = torch._C
-    return not (torch.compiler.is_compiling() or C._get_tracing_state() is not None
+    return not (not _ANSWERS or torch.compiler.is_compiling() or C._get_tracing_state() is not None
                 or C._len_torch_dispatch_stack() or C._len_torch_function_stack()
                 or C._functorch.peek_interpreter_stack() is not None
                 or forward_ad._current_level >= 0)
