@@ -56,8 +56,9 @@ extern "C" {
 
 /* 8: tfgfa_decode_splits, tfgfa_decode_scratch_bytes and tfgfa_stream_read added;
  * tfgfa_decode_noalloc splits only as far as its scratch holds instead of returning
- * TFGFA_ERR_SCRATCH. */
-#define TFGFA_ABI_VERSION 8
+ * TFGFA_ERR_SCRATCH.
+ * 9: the six tfgpt2_* entry points added (tfgfa_gpt2.h). */
+#define TFGFA_ABI_VERSION 9
 
 /* Status codes (> 0: invalid argument). */
 #define TFGFA_OK                 0

@@ -70,6 +70,14 @@ def test_library_exports_every_declared_symbol(lib):
         assert hasattr(lib, n), f"{n} declared in include/tfgfa.h but not exported"
 
 
+def test_library_exports_the_gpt2_entry_points_of_abi_9(lib):
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "tfgfa_gpt2.h")).read(), flags=re.S)
+    names = sorted(set(re.findall(r"\b(tfgpt2_\w+)\s*\(", text)))
+    assert names == ["tfgpt2_cast_bf16", "tfgpt2_gelu", "tfgpt2_layernorm", "tfgpt2_linear_planes",
+                     "tfgpt2_linear_planes_splits", "tfgpt2_linear_rows"]
+    assert all(hasattr(lib, n) for n in names) and lib.tfgfa_abi_version() >= 9
+
+
 def _split_bytes(bh, D, S):
     """Workspace bytes of a split of S (include/tfgfa.h, tfgfa_decode_splits): arrival words
     (B*H*128 rounded up to 256), then B*H*S partials of D + 1 floats; none for S = 1."""
