@@ -42,13 +42,14 @@ def _cu_count():
 
 def _heads(grid, B, nq):
     """Heads per batch row that send a (B, H, nq) problem to one kernel: "split" (the split-key
-    kernel, whose grid is chosen while B * H * ceil(nq / 128) is at most the CU count) or
-    "regular" (fwd_kernel, one workgroup per 128-row query block)."""
+    kernel: few query blocks, and no chain here is longer than the 32 halves it is chosen for) or
+    "regular" (fwd_kernel with one group, one workgroup per 128-row query block: every grid of more
+    than two blocks per CU).  tests/test_gpu_plans.py has the kernels between them."""
     nqb = (nq + 127) // 128
     if grid == "split":
         assert B * 3 * nqb <= _cu_count()
         return 3
-    return _cu_count() // (B * nqb) + 1
+    return 2 * _cu_count() // (B * nqb) + 1
 
 
 def _sample(x, B, H):

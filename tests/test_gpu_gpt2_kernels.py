@@ -40,16 +40,19 @@ def _gelu64(x):
 
 
 def test_kernel_arguments_are_checked_before_any_hip_call():
-    P = 0x10000
+    P, F = 0x10000, _C.GPT2_F32
+    for kind in (-1, _C.GPT2_PLANES + 1):
+        with pytest.raises(RuntimeError, match="dtype"):
+            _C.gpt2_layernorm(P, 0, 0, P, P, P, kind, 1, 64, 1e-5, 0)
     with pytest.raises(RuntimeError, match="negative batch|shape|size"):
-        _C.gpt2_layernorm(P, 0, 0, P, P, P, False, 1, 6, 1e-5, 0)          # width not a multiple of 4
+        _C.gpt2_layernorm(P, 0, 0, P, P, P, F, 1, 6, 1e-5, 0)          # width not a multiple of 4
     with pytest.raises(RuntimeError):
-        _C.gpt2_layernorm(P, 0, 0, P, P, P, False, 1, 2052, 1e-5, 0)       # too wide
+        _C.gpt2_layernorm(P, 0, 0, P, P, P, F, 1, 2052, 1e-5, 0)       # too wide
     with pytest.raises(RuntimeError, match="null"):
-        _C.gpt2_layernorm(P, P, 0, P, P, P, False, 1, 64, 1e-5, 0)         # delta without sum
+        _C.gpt2_layernorm(P, P, 0, P, P, P, F, 1, 64, 1e-5, 0)         # delta without sum
     with pytest.raises(RuntimeError, match="misaligned"):
-        _C.gpt2_layernorm(P + 4, 0, 0, P, P, P, False, 1, 64, 1e-5, 0)
-    _C.gpt2_layernorm(0, 0, 0, 0, 0, 0, False, 0, 64, 1e-5, 0)             # no rows: nothing to do
+        _C.gpt2_layernorm(P + 4, 0, 0, P, P, P, F, 1, 64, 1e-5, 0)
+    _C.gpt2_layernorm(0, 0, 0, 0, 0, 0, F, 0, 64, 1e-5, 0)             # no rows: nothing to do
     with pytest.raises(RuntimeError, match="misaligned"):
         _C.gpt2_gelu(P + 8, P, 4, 0)
     _C.gpt2_gelu(0, 0, 0, 0)
@@ -122,7 +125,7 @@ def test_values_past_one_launch_stay_with_torch(monkeypatch):
                                     (9, 1600), (1, 2048)])
 def test_layernorm_matches_float64(rows, d):
     """Widths at the edges of a lane's four values, of a wave's 256 and of the two register sizes;
-    rows that fill and do not fill a workgroup; an offset mean, so the variance must be centred."""
+    one and several rows (a workgroup each); an offset mean, so the variance must be centred."""
     from custom_flash_attn import gpt2
 
     g = torch.Generator(device=DEV).manual_seed(rows * 10007 + d)

@@ -80,7 +80,8 @@ WIDE = [s for shapes in WIDE_PLANS.values() for s in shapes]
 
 
 def _reference(q, k, v, causal):
-    q, k, v = q.float(), k.float(), v.float()
+    if q.dtype != torch.float64:
+        q, k, v = q.float(), k.float(), v.float()
     s = torch.matmul(q, k.transpose(-1, -2).contiguous()) / math.sqrt(q.shape[-1])
     if causal:
         s.masked_fill_(torch.ones(s.shape[-2:], dtype=torch.bool, device=DEV).triu(1), -math.inf)
@@ -112,17 +113,51 @@ def test_every_plan_and_head_dim(D, dtype):
 @pytest.mark.parametrize("B,H,N", [(1, 4, 1500), (2, 16, 777), (1, 25, 2048)])
 def test_key_groups_merge_extreme_rows(B, H, N):
     """Rows whose keys differ by hundreds between groups (one group's weight is 0), rows of equal
-    scores, and values at the type's largest: every merge weight stays finite."""
+    scores, and in the first head values near the largest that O is finite for (max|V| < 2^62): the
+    float32 partials and their merge keep the relative accuracy of ordinary ones."""
     g = torch.Generator(device=DEV).manual_seed(N)
     q, k, v = (torch.randn((B, H, N, 64), device=DEV, generator=g).to(torch.bfloat16) for _ in range(3))
     q[:, :, ::3] = 0
     k[:, :, 64:96] *= 40
-    v[:, 0] = 3.0e38
+    v[:, 0] *= 2.0 ** 55
     o, lse = custom_flash_attn.forward_lse(q, k, v)
-    o_ref, lse_ref = _reference(q[:, 1:], k[:, 1:], v[:, 1:], True)
-    assert (o[:, 1:].float() - o_ref).abs().max().item() <= 3 * U[torch.bfloat16] * v[:, 1:].abs().max().item()
-    assert ((lse[:, 1:] - lse_ref).abs() <= 1e-4 + 1e-5 * lse_ref.abs()).all()
-    assert torch.isfinite(lse).all()
+    o_ref, lse_ref = _reference(q, k, v, True)
+    for part in (slice(0, 1), slice(1, None)):
+        err = (o[:, part].float() - o_ref[:, part]).abs().max().item()
+        assert err <= 3 * U[torch.bfloat16] * v[:, part].abs().max().item()
+    assert ((lse - lse_ref).abs() <= 1e-4 + 1e-5 * lse_ref.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("kind", ["rising", "falling", "zigzag halves", "zigzag tiles"])
+def test_offset_moves_inside_key_groups(kind, dtype):
+    """Scores that climb past the offset's margin in every half, fall, or alternate by +-40 between a
+    group's halves or between the groups, at shapes of each key-group kernel.  Against float64.  Scores of
+    magnitude up to `span` are rounded to 2^-24 of it by each of the D / 16 accumulating MFMAs of the dot
+    product and four times after it (times the scale, less the offset, plus log2 of the sum, times ln 2),
+    so the LSE, and each probability relatively, is off by up to (D / 16 + 4) span 2^-24."""
+    for D, plans in ((64, NARROW_PLANS), (128, WIDE_PLANS)):
+        for plan, group in plans.items():
+            for B, H, Nq, Nk, causal in (group if "Groups" in plan or plan == "kPairs" else ()):
+                print(f"{kind} D={D} {dtype} {plan} H={H} Nq={Nq} Nk={Nk} causal={causal}", flush=True)
+                g = torch.Generator(device=DEV).manual_seed(Nq + Nk + D)
+                q, k, v = (torch.randn((B, H, n, D), device=DEV, generator=g) for n in (Nq, Nk, Nk))
+                j = torch.arange(Nk, device=DEV)
+                rise = 0.75 * (j if kind == "rising" else Nk - j)
+                sign = 1.0 - 2.0 * ((j // (32 if kind == "zigzag halves" else 64)) % 2)
+                q, k = 0.1 * q, 0.1 * k
+                q[..., 0] = 8.0
+                k[..., 0] += (rise if kind in ("rising", "falling") else 40.0 * sign) * math.sqrt(D) / 8
+                q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+                o, lse = custom_flash_attn.attention(q, k, v, causal=causal, return_lse=True)
+                assert torch.equal(custom_flash_attn.attention(q, k, v, causal=causal), o)
+                pick = sorted({0, H // 2, H - 1})
+                o_ref, lse_ref = _reference(*(t[:, pick].double() for t in (q, k, v)), causal)
+                span = lse_ref.abs().max().item() + 40
+                rounding = (D / 16 + 4) * span * 2.0 ** -24
+                err = (o[:, pick].double() - o_ref).abs().max().item()
+                assert err <= (3 * U[dtype] + 2 * rounding) * v[:, pick].abs().max().item()
+                assert (lse[:, pick] - lse_ref).abs().max().item() <= 1e-4 + rounding
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
