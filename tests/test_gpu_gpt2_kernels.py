@@ -113,11 +113,13 @@ def test_sizes_past_one_launch_are_refused_before_any_hip_call():
 def test_values_past_one_launch_stay_with_torch(monkeypatch):
     from custom_flash_attn import gpt2
 
-    x = torch.ones(8, device=DEV)
-    assert gpt2.takes(x)
+    x, calls = torch.ones(8, device=DEV), []
+    monkeypatch.setattr(gpt2, "gelu", lambda x: (calls.append(1), x)[1])
+    mi.GELU()(x)
+    assert calls
     monkeypatch.setattr(gpt2, "MAX_VALUES", 7)
-    assert not gpt2.takes(x)
     torch.testing.assert_close(mi.GELU()(x), torch.nn.functional.gelu(x, approximate="tanh"))
+    assert len(calls) == 1
 
 
 @pytest.mark.gpu

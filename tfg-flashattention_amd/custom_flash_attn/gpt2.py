@@ -34,17 +34,22 @@ def eager() -> bool:
     """No tracing, compilation, function transform, forward-mode level or torch mode is active, so
     a kernel launched on raw pointers is what the torch operators would have been."""
     C = torch._C
-    return not (not _ANSWERS or torch.compiler.is_compiling() or C._get_tracing_state() is not None
+    return not (torch.compiler.is_compiling() or C._get_tracing_state() is not None
                 or C._len_torch_dispatch_stack() or C._len_torch_function_stack()
                 or C._functorch.peek_interpreter_stack() is not None
                 or forward_ad._current_level >= 0)
 
 
+if not _ANSWERS:
+    def eager() -> bool:
+        return False
+
+
 def takes(x: torch.Tensor, *params, dtypes=(torch.float32,)) -> bool:
-    """``x`` (of one of ``dtypes``, of at most one launch's values) and the float32 ``params`` (None
-    allowed) are plain, contiguous, 16-byte aligned tensors on one GPU and need no gradient."""
+    """``x`` (of one of ``dtypes``) and the float32 ``params`` (None allowed) are plain, contiguous,
+    16-byte aligned tensors on one GPU and need no gradient."""
     if not (type(x) in _TYPES and x.is_cuda and x.dtype in dtypes and x.is_contiguous()
-            and x.data_ptr() % 16 == 0 and x.numel() <= MAX_VALUES):
+            and x.data_ptr() % 16 == 0):
         return False
     dev, grad = x.device, torch.is_grad_enabled()
     if grad and x.requires_grad:

@@ -59,8 +59,10 @@ def _plain(module, cls) -> bool:
     """``module`` is a ``cls`` as this file or torch defines it, with no hook and no compiled form
     (``module.compile()``) that a call of it would run: a caller may then take its parameters and
     leave the call out."""
-    return (type(module) is cls and not module._forward_hooks and not module._forward_pre_hooks
-            and "forward" not in module.__dict__ and module._compiled_call_impl is None)
+    if type(module) is not cls:
+        return False
+    d = module.__dict__  # holds what an instance adds; as attributes they are a lookup in each class first
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "_compiled_call_impl" in d)
 
 
 def _no_global_hooks() -> bool:
@@ -156,8 +158,8 @@ class MultiHeadAttention(nn.Module):
         )
 
     def _plain_linears(self) -> bool:
-        return (_plain(self, MultiHeadAttention)
-                and all(_plain(m, nn.Linear) for m in (self.W_query, self.W_key, self.W_value, self.out_proj)))
+        return (_plain(self, MultiHeadAttention) and _plain(self.W_query, nn.Linear) and _plain(self.W_key, nn.Linear)
+                and _plain(self.W_value, nn.Linear) and _plain(self.out_proj, nn.Linear))
 
     def _cast_together(self, x) -> bool:
         """Whether autocast's bf16 copies of x and of the four linears may be made in one launch:
@@ -354,7 +356,7 @@ class GELU(nn.Module):
 
     def forward(self, x):
         g = _gpt2() if x.is_cuda else None
-        if g is not None and g.eager() and g.takes(x):
+        if g is not None and g.eager() and g.takes(x) and x.numel() <= g.MAX_VALUES:
             return g.gelu(x)
         return 0.5 * x * (1 + torch.tanh(math.sqrt(2.0 / math.pi) * (x + 0.044715 * torch.pow(x, 3))))
 
