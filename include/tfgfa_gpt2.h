@@ -22,7 +22,8 @@ extern "C" {
 #endif
 
 /* Largest row width of the norm (a row lives in one wave's registers), the most rows of the
- * few-row projections and the most arrays of one cast. */
+ * few-row projections (8 normed rows of 1600 take 50 of the 60 KiB of LDS they may; more rows were
+ * not measured) and the most arrays of one cast. */
 #define TFGPT2_MAX_NORM_DIM 2048
 #define TFGPT2_MAX_ROWS     8
 #define TFGPT2_MAX_CASTS    10

@@ -128,8 +128,8 @@ __device__ __forceinline__ void normalise_row(f32x4 (&v)[kV], int d, int lane, f
 // stays in registers, and a reduction is 6 cross-lane steps with no barrier.  scale and shift are
 // loaded with the row, not after the reductions.  kV * 256 elements per row.
 //   613 rows of 1600: 4.9 us to bf16, 5.1 us with the residual (four rows per workgroup,
-//   scale and shift loaded where used: 7.2 and 9.3); the operators they stand for: about 32 us a
-//   norm, and 86 us for the mixed bf16 + float32 add before the second.
+//   scale and shift loaded where used: 7.2 and 9.3), 6.7 with the residual into planes; the operators
+//   they stand for: about 32 us a norm, and 86 us for the mixed bf16 + float32 add before the second.
 enum { kOutF32 = 0, kOutBf16 = 1, kOutPlanes = 2 };
 
 template <int kV, bool kDelta, int kOut>
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kCastThreads) void cast_kernel(Casts a) {
 // ---------------------------------------------------------------------------------------
 // The MLP's float32 linears: y = x w^T + bias for many rows.
 //
-// Bound: the matrix units.  The float32 MFMA peaks at 157 TFLOP/s (a library GEMM reaches 114-139 of
+// Bound: the matrix units.  The float32 MFMA peaks at 157 TFLOP/s (a library GEMM reaches 110-139 of
 // it), the bf16 one at 16 times that.  A float32 value is the exact sum of three bf16 values, so a
 // product of two is nine bf16 products; the six larger ones are computed (smallest first, float32
 // accumulation), the other three are below 2^-26 of the product, less than float32 rounds it by.

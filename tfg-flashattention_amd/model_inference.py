@@ -285,8 +285,9 @@ class KVCache:
 
 class GraphedDecoder:
     """One decode step of ``model`` (batch ``batch``, cache of ``max_len`` rows) captured in a
-    HIP graph and replayed per token, so a step costs one graph launch instead of the ~20
-    kernel launches (and their Python) per layer of an eager step.
+    HIP graph and replayed per token, so a step costs one graph launch instead of the kernel
+    launches (and their Python) of each layer of an eager step: five up to 8 sequences (the few-row
+    projections), about 20 past them.
 
     The step reads its token from ``self.tok`` and leaves the last position's logits in
     ``self.logits``.  Everything it depends on lives in device memory: the positions and the
