@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the causal attention forward on one MI355X.
 
-Workload (BASELINE.json metric and configs[2]): causal attention forward, bf16, d=64, at
+Workload: causal attention forward, bf16, d=64, at
 the GPT-2-XL shape B=8, H=25, N=1024; Q, K ~ N(0, 3^2), V ~ N(0, 1); scale 1/8.  One step =
 one launch of the drop-in forward over one batch: custom_flash_attn.forward(q, k, v), the
 call the reference's GPT-2 attention makes (src/py/model_inference.py:85-90,
@@ -15,7 +15,7 @@ Prints one JSON line.  ``value`` is TFLOP/s with the FlashAttention causal conve
 (4*B*H*N^2*d/2 FLOPs per forward), from the K timed steps bracketed by synchronisations.
 ``roofline`` compares it with the dense bf16 MFMA peak; ``cpu_baseline`` times the
 reference's PyTorch CPU attention path (the "manual" branch of src/py/model_inference.py:68-75)
-on this host's cores.  ``configs`` times every BASELINE.json attention config (1-4, plus the
+on this host's cores.  ``configs`` times every named attention workload (config1-4, plus the
 drop-in O-only call at config 3) by per-launch events: the median of at least 200 launches
 after a warm-up of at least 0.1 s, whatever --steps and --warmup say.  ``triton_wrapper_surface``
 times the general entry point the same way on fp16 and head dim 128 (the surface of the
@@ -50,7 +50,7 @@ MIN_PER_CALL = 200  # per-launch timings behind every median
 
 
 class BenchConfig:
-    """One of BASELINE.json's attention configs 1-4 as the GPU legs run it: shape, input
+    """One of the attention workloads config1-4 as the GPU legs run it: shape, input
     distribution (Q, K ~ N(0, sigma_qk^2), V ~ N(0, sigma_v^2), bf16) and the seed of its
     inputs.  The same table as the test oracle's (a CPU test checks they agree); kept here so
     that the timed legs import nothing from the oracle."""
@@ -131,7 +131,7 @@ def _graphed(step, dev, per_graph=10):
 
 def cpu_threads():
     """Threads for the CPU baseline: every core of this process's affinity mask, capped at the
-    host's CPU share per GPU when the environment states one (OMP_NUM_THREADS; the GPU boxes
+    host's CPU share per GPU when the environment states one (OMP_NUM_THREADS: hosts that share their GPUs
     set it to 16 and allot that many cores per GPU, whatever the affinity mask lists)."""
     aff = len(os.sched_getaffinity(0))
     share = os.environ.get("OMP_NUM_THREADS", "")
@@ -204,7 +204,7 @@ def cpu_baseline(gpu_o_sample, q_sample, k_sample, v_sample, heads_in_sample):
 
 
 def cpu_baseline_configs():
-    """The same CPU path on BASELINE.json configs 1-4 at full shape, on the oracle's seeded
+    """The same CPU path on the workloads config1-4 at full shape, on the oracle's seeded
     inputs (oracle.make_inputs); config 4's (B,H,N,N) fp32 scores (4.3 GB) are formed one
     head at a time.  One warm-up, median of 3 runs each."""
     import torch
@@ -642,7 +642,7 @@ CONFIG_SETS = {"config1": 4, "config2": 6, "config3": 4, "config4": 5}
 
 
 def time_configs(dev):
-    """Every BASELINE.json attention config (1-4) through the C ABI on this build's kernel, O + LSE
+    """Every attention workload (config1-4) through the C ABI on this build's kernel, O + LSE
     (the headline's outputs), plus config 3 through the drop-in O-only call: seeded inputs of
     each config's distribution, input sets rotated so that the working set of one launch is
     not left in the Infinity Cache by the previous one (config 1, 1.6 MB per set, stays
@@ -881,7 +881,7 @@ def main():
     ap.add_argument("--no-surface", action="store_true",
                     help="skip the fp16 / head dim 128 legs (the Triton wrapper's surface)")
     ap.add_argument("--no-configs", action="store_true",
-                    help="skip the per-config legs (BASELINE.json configs 1-4, per-launch medians)")
+                    help="skip the per-config legs (config1-4, per-launch medians)")
     ap.add_argument("--cpu-heads", type=int, default=200,
                     help="heads of the workload timed by the CPU baseline")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",

@@ -1,7 +1,7 @@
 """CPU oracle for the causal attention forward - TEST INFRASTRUCTURE ONLY.
 
 Only ``tests/``, ``__graft_entry__.smoke()`` and ``bench.py``'s ``cpu_baseline`` leg
-may import this package, and only as the checker.  The product path
+may import this package, and only as the oracle.  The product path
 (``custom_flash_attn`` -> ``libtfgfa.so``) never imports or calls it.
 
 Contents (each restates the reference; file:line cited at each function):
@@ -12,7 +12,7 @@ Contents (each restates the reference; file:line cited at each function):
     same math over the first L cached keys (fp64 numpy);
   * ``manual_attention_torch`` - the reference's PyTorch CPU "manual" branch, fp32
     (the CPU baseline timed by bench.py);
-  * ``CONFIGS`` / ``make_inputs`` - the seeded inputs of BASELINE.json's configs.
+  * ``CONFIGS`` / ``make_inputs`` - the seeded inputs of the named workloads.
 
 Pinning (tests/test_oracle.py): against torch's scaled_dot_product_attention in
 fp64 (the library routine the reference's own tests use,

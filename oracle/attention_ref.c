@@ -2,7 +2,7 @@
  * attention_ref.c - CPU oracle for the causal attention forward.
  *
  * TEST INFRASTRUCTURE ONLY.  Only tests/, __graft_entry__.smoke() and bench.py's
- * cpu_baseline leg may load this library, and only as the checker: the product path
+ * cpu_baseline leg may load this library, and only as the oracle: the product path
  * (custom_flash_attn / libtfgfa.so) never calls it.
  *
  * A plain restatement, in fp64, of the reference's "manual" attention branch

@@ -1,7 +1,7 @@
 """CPU oracle for the causal attention forward - TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may use this
-module, as the checker; the product path never does.
+module, as the oracle; the product path never does.
 """
 from __future__ import annotations
 
@@ -181,7 +181,7 @@ def manual_attention_torch(q, k, v):
 
 
 # --------------------------------------------------------------------------------------
-# BASELINE.json configs 1-4 (config 5, the GPT-2-medium forward, lives in the tests).
+# The attention workloads 1-4 (the fifth, the GPT-2-medium forward, lives in the tests).
 
 
 @dataclass(frozen=True)

@@ -12,7 +12,7 @@ test/py/test_cuda_implementation.py:14-19, :78-80), so these are built here:
     (the library routine the reference's tests compare with, :49-52) and against the
     C oracle, so a fixture never records an unchecked number.
   * inputs_sha256.json - SHA-256 of the bf16 bytes of the seeded Q, K, V of
-    BASELINE.json configs 1-4 (oracle.make_inputs), pinning the input generator.
+    the workloads config1-4 (oracle.make_inputs), pinning the input generator.
 
 Run from the repository root:  python tests/golden/make_golden.py
 """

@@ -1,5 +1,5 @@
 """Cached GPT-2 decoding (prefill kernel + decode kernel with a KV cache) against the
-reference's full-recompute path (GPU box only, except the argument checks).
+reference's full-recompute path (needs a GPU, except the argument checks).
 
 The reference's generate() re-runs the whole prefix per token (src/py/model_inference.py:
 199-228); the logits it samples from are those of the last position of a full forward.  Here

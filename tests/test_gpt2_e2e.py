@@ -1,5 +1,5 @@
-"""end-to-end GPT-2-medium forward with every layer's attention on
-the HIP kernel, logits compared with the CPU fp32 "manual" path (GPU box only).
+"""End-to-end GPT-2-medium forward with every layer's attention on
+the HIP kernel, logits compared with the CPU fp32 "manual" path (needs a GPU).
 
 Model: 24 layers, d_model 1024, 16 heads of 64, MLP 4096, GELU, pre-LN, vocab 50257,
 context 1024, qkv_bias True (src/py/model_inference.py:393-415).  Weights are seeded

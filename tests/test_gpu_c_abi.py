@@ -1,4 +1,4 @@
-"""The C ABI called directly through ctypes, as a non-Python FFI would bind it (GPU box only).
+"""The C ABI called directly through ctypes, as a non-Python FFI would bind it (needs a GPU).
 
 Each compute entry point of include/tfgfa.h is called with the argument lists a reference-side
 ctypes binding would use (argtypes from the header's prototypes), on raw device pointers from

@@ -1,4 +1,4 @@
-"""Decode step over a KV cache (tfgfa_decode_bf16) against the CPU oracle (GPU box only).
+"""Decode step over a KV cache (tfgfa_decode_bf16) against the CPU oracle (needs a GPU).
 
 The oracle is ``decode_np``: the last row of the causal forward over the first L cached
 tokens (what the reference's generate() recomputes per token, src/py/model_inference.py:

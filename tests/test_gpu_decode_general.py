@@ -1,8 +1,8 @@
 """Decode step widened to fp16 and head dims up to 128 (tfgfa_decode) against the CPU oracle
-(GPU box only).
+(needs a GPU).
 
 ``decode_np`` (fp64, the last row of the causal forward over the first L cached tokens,
-pinned in tests/test_oracle.py) is the checker, on inputs already rounded to the element type.
+pinned in tests/test_oracle.py) is the reference, on inputs already rounded to the element type.
 Tolerances as for the forward: max|dO| <= 2e-2, mean|dO| <= 2e-3, max|dLSE| <= 1e-3, with
 Q, K ~ N(0, 3^2) and V ~ N(0, 1).
 

@@ -1,6 +1,6 @@
 """The general forward (tfgfa_fwd): fp16 and bf16, head dims up to 128, N_q != N_k, strided
 operands - the surface of the reference's Triton wrapper _flash_attn_forward
-(src/py/triton_implementation.py:184-241).  GPU box only.
+(src/py/triton_implementation.py:184-241).  needs a GPU.
 
 Against the CPU oracle (attention_c / attention_np, pinned in tests/test_oracle.py, including
 N_q != N_k and other head dims) on the same dtype-rounded inputs: max|dO| <= 2e-2,

@@ -1,5 +1,5 @@
 """The GPT-2 block kernels (include/tfgfa_gpt2.h) against float64 references of the same
-functions, and the modules that use them against their torch operators (GPU box only, except the
+functions, and the modules that use them against their torch operators (needs a GPU, except the
 argument checks).
 
 Tolerances.  Values are float32 with float32 sums: a result carries a few roundings of 2^-24

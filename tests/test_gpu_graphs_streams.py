@@ -1,4 +1,4 @@
-"""HIP graph capture and concurrent streams (GPU box only).
+"""HIP graph capture and concurrent streams (needs a GPU).
 
 The entry points allocate nothing and clear no memory with memsets, so a caller may capture
 them in a HIP graph.  Each graph below is replayed several times with eager work and

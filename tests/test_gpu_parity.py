@@ -1,8 +1,8 @@
-"""Parity of the HIP kernel with the CPU oracle (GPU box only).
+"""Parity of the HIP kernel with the CPU oracle (needs a GPU).
 
-Tolerances (BASELINE.json north_star): against the fp64/fp32 oracle on the same
+Tolerances: against the fp64/fp32 oracle on the same
 bf16-rounded inputs, max|dO| <= 2e-2 and mean|dO| <= 2e-3; LSE (natural log) max
-abs error <= 1e-3.  Shapes: BASELINE.json configs 1-4 (config 1 and 2 in full,
+abs error <= 1e-3.  Shapes: the workloads config1-4 (config 1 and 2 in full,
 config 3 and 4 on sampled query rows of every head), the reference's boundary
 lengths (test/py/test_cuda_implementation.py:93) and more edge cases.
 
@@ -87,7 +87,7 @@ def test_golden_fixtures(fname):
     _check(o, lse, z["o"], z["lse"], fname)
 
 
-# ------------------------------------------------------------------ BASELINE configs
+# ------------------------------------------------------------------ the named workloads
 
 
 def _config_inputs(name):

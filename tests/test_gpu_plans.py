@@ -1,6 +1,6 @@
 """The forward's key-split workgroups and head-dim instances at the sizes where they can go wrong:
 ends of 32-key halves, 64-key tiles and query blocks, groups without a tile, head dims at the edges
-of the compiled ones (GPU box only).
+of the compiled ones (needs a GPU).
 
 Reference: float32 attention from the same 16-bit values.  With u the unit roundoff of the type
 (2^-8 bf16, 2^-11 fp16), the probabilities, their sum and the output are each rounded once:

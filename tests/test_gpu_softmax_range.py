@@ -1,4 +1,4 @@
-"""The forward's softmax over extreme score patterns (GPU box only).
+"""The forward's softmax over extreme score patterns (needs a GPU).
 
 The kernel keeps a per-row exp2 offset that moves only when a lane's running sum of its
 probabilities, as rounded for the MFMA, would pass a bound (bf16: 2^64; fp16: the largest finite

@@ -1,11 +1,11 @@
-"""Strided operands through tfgfa_fwd_bf16_strided (GPU box only).
+"""Strided operands through tfgfa_fwd_bf16_strided (needs a GPU).
 
 The kernel's arithmetic does not depend on where rows live, so every strided call is
 checked bit-for-bit against the contiguous entry point on the same values, and once
 against the CPU oracle (tolerances as in test_gpu_parity.py: max|dO| <= 2e-2,
 mean|dO| <= 2e-3, max|dLSE| <= 1e-3).  Output buffers are filled with a sentinel first:
 elements that are not part of O (padding between rows, heads or batches) must keep it.
-Inputs follow the BASELINE configs' distributions (Q, K ~ N(0, 2^2..3^2), V ~ N(0, 1)),
+Inputs follow the workloads' distributions (Q, K ~ N(0, 2^2..3^2), V ~ N(0, 1)),
 the distributions the tolerances are stated for: O's error scales with |V|.
 """
 import sys

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/) before it is trusted as the checker of the HIP kernel.
+"""Pins the CPU oracle (oracle/) before it is trusted as the oracle of the HIP kernel.
 
 Each check is chosen so that a plausible mistake in the oracle fails at least one of
 them (see test_planted_mistakes_are_caught): the diagonal dropped from the causal mask,

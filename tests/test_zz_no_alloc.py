@@ -1,6 +1,6 @@
 """tfgfa_decode_noalloc - the decode step with its split partials in the library's static
 scratch instead of a caller's workspace - against tfgfa_decode with a full workspace, through
-the C ABI (GPU box only).
+the C ABI (needs a GPU).
 
 Two calls in a row on the same GPU, the second smaller than the first, so the second runs on a
 scratch still holding the first call's partials.  Named to be collected last: it passes alone in
