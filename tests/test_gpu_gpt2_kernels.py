@@ -103,10 +103,18 @@ def test_sizes_past_one_launch_are_refused_before_any_hip_call():
         N = 4 * (2 ** 32 // (256 if norm else 512 if K <= 4096 else 1024))
         with pytest.raises(RuntimeError, match=big):
             _C.gpt2_linear_rows(P, False, norm, norm, 0.0, [(P, 0, P)], False, 0, False, 1, N, K, 0)
-    norm = mi.LayerNorm({"emb_dim": 4}).to("meta")
-    assert norm._native(torch.empty(gpt2.MAX_NORM_ROWS, 4, device="meta"))
-    assert not norm._native(torch.empty(gpt2.MAX_NORM_ROWS + 1, 4, device="meta"))
+    norm = mi.LayerNorm({"emb_dim": 32}).to("meta")
+    assert norm._native(torch.empty(gpt2.MAX_NORM_ROWS, 32, device="meta"))
+    assert not norm._native(torch.empty(gpt2.MAX_NORM_ROWS + 1, 32, device="meta"))
     assert gpt2.rows_fit(1, _C.GPT2_MAX_OUTPUTS, False) and not gpt2.rows_fit(1, _C.GPT2_MAX_OUTPUTS + 4, False)
+
+
+@pytest.mark.parametrize("d", [4, 28, 32])
+def test_many_narrow_rows_stay_with_torch(d):
+    """Up to 28 values a row the torch operators take less time than a wave per row from some 37000 rows."""
+    norm = mi.LayerNorm({"emb_dim": d}).to("meta")
+    assert norm._native(torch.empty(32768, d, device="meta"))
+    assert norm._native(torch.empty(300000, d, device="meta")) is (d >= 32)
 
 
 @pytest.mark.gpu

@@ -338,8 +338,12 @@ class LayerNorm(nn.Module):
         self.shift = nn.Parameter(torch.zeros(config["emb_dim"]))
 
     def _native(self, x) -> bool:
+        """Whether the kernel takes x's rows: one wave each, so many rows far narrower than its 256 values
+        cost it more than the torch operators' passes over them (us, kernel / operators: 300000 x 4 111 /
+        36, x 16 111 / 87, x 32 112 / 164; 30000 x 4 14.5 / 18.9)."""
         g, d = _gpt2(), x.shape[-1] if x.dim() else 0
-        return (d % 4 == 0 and 4 <= d <= g.MAX_NORM_DIM and x.numel() <= d * g.MAX_NORM_ROWS
+        return (d % 4 == 0 and 4 <= d <= g.MAX_NORM_DIM
+                and x.numel() <= d * (g.MAX_NORM_ROWS if d >= 32 else 32768)
                 and self.scale.shape == (d,) and self.shift.shape == (d,))
 
     def forward(self, x):
@@ -416,7 +420,9 @@ class TransformerBlock(nn.Module):
         they are not plain float32 linears of sizes it takes, or small: from 2^30 multiplications a
         linear the whole block's kernels take less time (us, library / split: GPT-2 small 256 rows
         82 / 85, 613 rows 114 / 105; medium 128 rows 84 / 88, 256 rows 97 / 94; XL 64 rows 104 / 109, 128
-        rows 123 / 117, 1024 rows 481 / 363)."""
+        rows 123 / 117, 1024 rows 481 / 363), or little more where a last tile of 128 rows is nearly empty
+        (XL 130 rows 118 / 130, 257 rows 165 / 168; large 165 rows 98 / 101), with fewer calls for the host
+        (XL 130 rows, eager: 229 / 185)."""
         g = _gpt2()
         if not self._plain_mlp():
             return None
@@ -433,7 +439,9 @@ class TransformerBlock(nn.Module):
 
     def _rows_fused(self, x, cache) -> bool:
         """Whether a decode step may run its projections on the few-row kernel: as for _fused, with
-        plain linears, float32 weights, a bf16 cache that holds tokens and few enough rows."""
+        plain linears, float32 weights, a bf16 cache that holds tokens and few enough rows.  (us per layer,
+        few-row kernels / the general path with 8 rows: replayed, GPT-2 small 33 / 47, medium 35 / 53,
+        large 85 / 61, XL 98 / 75; launched eagerly 92 / 240.)"""
         g, att, ff = _gpt2(), self.att, self.ff
         if not (cache is not None and cache.length > 0 and x.shape[1] == 1 and att.impl_type in ("hip", "cuda")
                 and att._plain_linears() and self._plain_mlp() and cache.k[0].dtype == torch.bfloat16):
