@@ -43,6 +43,8 @@
  *     N_k * max|V| < 2^112   (fp16; always true, fp16 values are below 2^16).
  * Past that bound a bf16 row may come out inf or NaN where the exact-offset reference
  * stays finite.  LSE is not affected.
+ * A score of -inf (q.k past the float range, infinite keys) has probability 0 wherever it stands in
+ * the row; a row of nothing else has O NaN and LSE -inf.
  */
 #ifndef TFGFA_H
 #define TFGFA_H
